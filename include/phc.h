@@ -470,9 +470,8 @@ phc_status phc_lb_train(phc_lb *h, int steps, int batch_per_face, float lr, uint
 /* No counterpart in the reference.  phc_lb_train for callers that cannot
  * allocate device memory (code under graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): the same steps and the same values, with
- * the per-call buffers (minibatch indices, per-block partial gradients and
- * losses, loss history) in one static device array per GPU instead of
- * buffers allocated per call.  Limits: batch_per_face <= 8192 and
+ * the per-call buffers (per-block partial gradients and losses, loss history)
+ * in one static device array per GPU instead of buffers allocated per call.  Limits: batch_per_face <= 8192 and
  * steps <= 16384 per call (PHC_ERR_INVALID beyond).  Calls that overlap on
  * one GPU share that array and race. */
 phc_status phc_lb_train_noalloc(phc_lb *h, int steps, int batch_per_face, float lr, uint64_t seed,

@@ -302,21 +302,33 @@ __global__ void __launch_bounds__(LB_CB) lb_onpolicy_kernel(LbOnPolicyArgs A)
 }
 
 // ------------------------------------------------------------ training
-constexpr int LB_TB = 64;  // samples (threads) per training block
+constexpr int LB_TB = 64;         // samples per training block: one per lane
+constexpr int LB_TW = 8;          // wavefronts per training block
+constexpr int LB_TT = LB_TB * LB_TW;
+constexpr int LB_TS = LB_TB + 4;  // row stride of the per-unit LDS rows (16-byte aligned, rows 4 banks apart)
 
 struct LbBatch {
     const float *samples[LB_FACES];
-    const int *idx[LB_FACES];  // positions in samples (nullptr: 0..count-1)
-    int count[LB_FACES];
+    int count[LB_FACES];       // samples of the batch per face
+    int population[LB_FACES];  // stored samples a random batch draws from
     int block_start[LB_FACES + 1];
+    int random;       // 1: sample n of face f is a random stored one (lb_batch_index), 0: stored sample n
+    uint64_t iseed;   // seed of the random draw (face f: iseed + f)
     float inv_total;  // 1 / total samples in the batch
     float noise;      // std of the Gaussian noise added to the field inputs (0: none)
     uint64_t nseed;
     // non-null: each block writes its gradient sum to partial[block][p] and
-    // its loss to ploss[block] (summed in a fixed order by lb_reduce_kernel,
+    // its loss to ploss[block] (summed in a fixed order by lb_update_kernel,
     // so training repeats bit for bit); null: float atomics into grad, loss
     float *partial, *ploss;
 };
+
+// Position in face f's store of sample n of a random batch, uniform in [0, population).
+__device__ inline int lb_batch_index(const LbBatch &B, int f, int n)
+{
+    const uint64_t key = B.iseed + (uint64_t)f + 0x632be59bd9b4e019ull * (uint64_t)(n + 1);
+    return (int)(lb_hash(key) % (uint32_t)B.population[f]);
+}
 
 // Standard normal from four hashed uniforms (Irwin-Hall, rescaled to unit variance).
 __device__ inline float lb_gauss(uint64_t key)
@@ -329,145 +341,279 @@ __device__ inline float lb_gauss(uint64_t key)
 
 // Forward, loss and backward of one batch: every block takes LB_TB samples of
 // one face; the weights are used rounded to bf16 (the stored inference
-// precision), arithmetic in FP32.  Per-sample activations and deltas go to
-// LDS; each thread then sums the gradient of a strided subset of the face's
-// parameters over the block's samples and adds it to grad (FP32 atomics).
-__global__ void __launch_bounds__(LB_TB) lb_train_kernel(const float *__restrict__ theta, float *grad, float *loss,
+// precision), arithmetic in FP32.
+//
+// A batch of 4096 samples per face is only 384 blocks, so a step is bound by
+// one block's serial chain, not by the chip: 8 wavefronts share a block's 64
+// samples (lane = sample, a wavefront owns 4 of the 32 hidden units), and the
+// gradient takes 2 parameters per thread.  LDS rows are per unit with the
+// samples along the row, so a unit's 4 neighbouring samples, like a weight
+// row's 4 neighbouring entries, are one 16-byte read.  Every sum keeps one
+// fixed order (inputs, hidden units, samples ascending).
+// Batch 4096 per face, MI355X: 14.8 us, and 5.9 us for the update kernel; one
+// wavefront per block with a thread per sample took 63.5 us, beside 40.3 us for
+// the sums over blocks, 6 x 4.6 us to draw the batch and 4.8 us for Adam.
+__global__ void __launch_bounds__(LB_TT) lb_train_kernel(const float *__restrict__ theta, float *grad, float *loss,
                                                          LbBatch B)
 {
-    __shared__ float w[LB_NP];
-    __shared__ float sx[LB_TB][LB_NIN + 1];
-    __shared__ float sh1[LB_TB][LB_H + 1], sh2[LB_TB][LB_H + 1], sd1[LB_TB][LB_H + 1], sd2[LB_TB][LB_H + 1];
-    __shared__ float sdy[LB_TB];
-    __shared__ int sdep[LB_TB];
-    __shared__ float sloss[LB_TB];
+    constexpr int IN4 = (LB_NIN + 3) / 4 * 4;  // inputs padded to whole 16-byte reads
+    constexpr int UW = LB_H / LB_TW;           // hidden units per wavefront
+    static_assert(LB_H == 32 && LB_NIN == 19 && LB_W == 4 && LB_TT == 512, "thread ranges of the gradient below");
+    __shared__ __align__(16) float w1[LB_H][IN4], w2[LB_H][LB_H];
+    __shared__ float b1[LB_W][LB_H], b2[LB_H], w3[LB_H], b3;
+    __shared__ __align__(16) float sx[IN4][LB_TS], sh1[LB_H][LB_TS], sh2[LB_H][LB_TS], sd1[LB_H][LB_TS],
+        sd2[LB_H][LB_TS];
+    __shared__ __align__(16) float sdy[LB_TB], sloss[LB_TB];
+    __shared__ __align__(16) int sdep[LB_TB];
     int f = 0;
     while (f + 1 < LB_FACES && (int)blockIdx.x >= B.block_start[f + 1]) ++f;
     const int chunk = blockIdx.x - B.block_start[f];
-    const int tid = threadIdx.x;
-    for (int p = tid; p < LB_NP; p += LB_TB) w[p] = bf2f(f2bf(theta[f * LB_NP + p]));
-    __syncthreads();
-    const int pos = chunk * LB_TB + tid;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), u0 = wv * UW;
+    const int pos = chunk * LB_TB + lane;
     const bool valid = pos < B.count[f];
-    float t = 0.f;
-    int d = 0;
-    if (valid) {
-        const int si = B.idx[f] ? B.idx[f][pos] : pos;
-        const float *s = B.samples[f] + (int64_t)si * LB_NSTRIDE;
-        for (int m = 0; m < LB_NIN; ++m) sx[tid][m] = s[m];
-        t = s[LB_NIN];
-        d = min(max((int)s[LB_NIN + 1], 0), LB_W - 1);
-        if (B.noise > 0.f) {
-            // denoising: perturb the field inputs that exist at this depth
-            // (offsets inside the region), keep the clean target, so the
-            // network learns not to amplify errors in its own inputs
-            const uint64_t key = (B.nseed * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)f << 40) ^ (uint64_t)si;
-            for (int m = 0; m < 18; ++m)
-                if (m % 9 >= 4 - d) sx[tid][m] += B.noise * lb_gauss(key * 32ull + (uint64_t)m);
-        }
-    } else {
-        for (int m = 0; m < LB_NIN; ++m) sx[tid][m] = 0.f;
-    }
-    // forward; activations stay in this thread's LDS rows
-    for (int i = 0; i < LB_H; ++i) {
-        float a = w[LB_OFF_B1 + d * LB_H + i];
+    // every load of the block is issued before the first is used: the sample's
+    // target and depth, a share of its inputs per wavefront, the weights
+    constexpr int MW = (IN4 + LB_TW - 1) / LB_TW, PW = (LB_NP + LB_TT - 1) / LB_TT;
+    const int si = !valid ? 0 : B.random ? lb_batch_index(B, f, pos) : pos;
+    const float *s = B.samples[f] + (int64_t)si * LB_NSTRIDE;
+    float x0[MW], t = 0.f, depth = 0.f, wt[PW];
 #pragma unroll
-        for (int m = 0; m < LB_NIN; ++m) a = fmaf(w[LB_OFF_W1 + i * LB_NIN + m], sx[tid][m], a);
-        sh1[tid][i] = fmaxf(a, 0.f);
+    for (int q = 0; q < MW; ++q) x0[q] = (valid && wv + q * LB_TW < LB_NIN) ? s[wv + q * LB_TW] : 0.f;
+    if (valid) {
+        t = s[LB_NIN];
+        depth = s[LB_NIN + 1];
     }
-    float y = w[LB_OFF_B3];
-    for (int i = 0; i < LB_H; ++i) {
-        float a = w[LB_OFF_B2 + i];
-#pragma unroll 8
-        for (int j = 0; j < LB_H; ++j) a = fmaf(w[LB_OFF_W2 + i * LB_H + j], sh1[tid][j], a);
-        const float h2 = fmaxf(a, 0.f);
-        sh2[tid][i] = h2;
-        y = fmaf(w[LB_OFF_W3 + i], h2, y);
+    const float *th = theta + f * LB_NP;
+#pragma unroll
+    for (int q = 0; q < PW; ++q) wt[q] = th[min(tid + q * LB_TT, LB_NP - 1)];
+    const int d = min(max((int)depth, 0), LB_W - 1);
+#pragma unroll
+    for (int q = 0; q < MW; ++q) {
+        const int m = wv + q * LB_TW;
+        float x = x0[q];
+        // denoising: perturb the field inputs that exist at this depth
+        // (offsets inside the region), keep the clean target, so the
+        // network learns not to amplify errors in its own inputs
+        if (valid && B.noise > 0.f && m < 18 && m % 9 >= 4 - d) {
+            const uint64_t key = (B.nseed * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)f << 40) ^ (uint64_t)si;
+            x += B.noise * lb_gauss(key * 32ull + (uint64_t)m);
+        }
+        if (m < IN4) sx[m][lane] = x;
     }
-    // backward
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+        const int p = tid + q * LB_TT;
+        const float v = bf2f(f2bf(wt[q]));
+        if (p < LB_OFF_B1) w1[p / LB_NIN][p % LB_NIN] = v;
+        else if (p < LB_OFF_W2) b1[(p - LB_OFF_B1) / LB_H][(p - LB_OFF_B1) % LB_H] = v;
+        else if (p < LB_OFF_B2) w2[(p - LB_OFF_W2) / LB_H][(p - LB_OFF_W2) % LB_H] = v;
+        else if (p < LB_OFF_W3) b2[p - LB_OFF_B2] = v;
+        else if (p < LB_OFF_B3) w3[p - LB_OFF_W3] = v;
+        else if (p < LB_NP) b3 = v;
+    }
+    if (tid < LB_H) w1[tid][LB_NIN] = 0.f;
+    __syncthreads();
+    // layer 1
+    {
+        float x[LB_NIN];
+#pragma unroll
+        for (int m = 0; m < LB_NIN; ++m) x[m] = sx[m][lane];
+#pragma unroll
+        for (int q = 0; q < UW; ++q) {
+            const int i = u0 + q;
+            float a = b1[d][i];
+#pragma unroll
+            for (int m = 0; m < LB_NIN; m += 4) {
+                const float4 wq = *(const float4 *)&w1[i][m];
+                a = fmaf(wq.x, x[m], a);
+                if (m + 1 < LB_NIN) a = fmaf(wq.y, x[m + 1], a);
+                if (m + 2 < LB_NIN) a = fmaf(wq.z, x[m + 2], a);
+                if (m + 3 < LB_NIN) a = fmaf(wq.w, x[m + 3], a);
+            }
+            sh1[i][lane] = fmaxf(a, 0.f);
+        }
+    }
+    __syncthreads();
+    // layer 2
+    {
+        float x[LB_H];
+#pragma unroll
+        for (int j = 0; j < LB_H; ++j) x[j] = sh1[j][lane];
+#pragma unroll
+        for (int q = 0; q < UW; ++q) {
+            const int i = u0 + q;
+            float a = b2[i];
+#pragma unroll
+            for (int j = 0; j < LB_H; j += 4) {
+                const float4 wq = *(const float4 *)&w2[i][j];
+                a = fmaf(wq.x, x[j], a);
+                a = fmaf(wq.y, x[j + 1], a);
+                a = fmaf(wq.z, x[j + 2], a);
+                a = fmaf(wq.w, x[j + 3], a);
+            }
+            sh2[i][lane] = fmaxf(a, 0.f);
+        }
+    }
+    __syncthreads();
+    // output and its error, formed by every wavefront for its own use
+    float y = b3;
+#pragma unroll
+    for (int i = 0; i < LB_H; ++i) y = fmaf(w3[i], sh2[i][lane], y);
     const float e = valid ? y - t : 0.f;
     const float dy = 2.f * B.inv_total * e;
-    sloss[tid] = e * e;
-    sdy[tid] = dy;
-    sdep[tid] = d;
-    for (int i = 0; i < LB_H; ++i) sd2[tid][i] = sh2[tid][i] > 0.f ? dy * w[LB_OFF_W3 + i] : 0.f;
-    for (int j = 0; j < LB_H; ++j) {  // W2^T d2, masked by relu'
-        float a = 0.f;
-#pragma unroll 8
-        for (int i = 0; i < LB_H; ++i) a = fmaf(w[LB_OFF_W2 + i * LB_H + j], sd2[tid][i], a);
-        sd1[tid][j] = sh1[tid][j] > 0.f ? a : 0.f;
+    if (wv == 0) {
+        sloss[lane] = e * e;
+        sdy[lane] = dy;
+        sdep[lane] = d;
+    }
+#pragma unroll
+    for (int q = 0; q < UW; ++q) sd2[u0 + q][lane] = sh2[u0 + q][lane] > 0.f ? dy * w3[u0 + q] : 0.f;
+    __syncthreads();
+    // W2^T d2, masked by relu'
+    {
+        float a[UW];
+#pragma unroll
+        for (int q = 0; q < UW; ++q) a[q] = 0.f;
+#pragma unroll
+        for (int i = 0; i < LB_H; ++i) {
+            const float di = sd2[i][lane];
+            const float4 wa = *(const float4 *)&w2[i][u0];
+            a[0] = fmaf(wa.x, di, a[0]);
+            a[1] = fmaf(wa.y, di, a[1]);
+            a[2] = fmaf(wa.z, di, a[2]);
+            a[3] = fmaf(wa.w, di, a[3]);
+        }
+#pragma unroll
+        for (int q = 0; q < UW; ++q) sd1[u0 + q][lane] = sh1[u0 + q][lane] > 0.f ? a[q] : 0.f;
     }
     __syncthreads();
-    if (tid == 0) {
-        float sum = 0.f;
-        for (int k = 0; k < LB_TB; ++k) sum += sloss[k];
-        if (B.ploss) B.ploss[blockIdx.x] = sum * B.inv_total;
-        else atomicAdd(loss, sum * B.inv_total);
-    }
-    float *gf = grad + f * LB_NP;
-    for (int p = tid; p < LB_NP; p += LB_TB) {
-        float g = 0.f;
-        if (p < LB_OFF_B1) {
-            const int i = p / LB_NIN, m = p % LB_NIN;
-            for (int k = 0; k < LB_TB; ++k) g = fmaf(sd1[k][i], sx[k][m], g);
-        } else if (p < LB_OFF_W2) {
-            const int dd = (p - LB_OFF_B1) / LB_H, i = (p - LB_OFF_B1) % LB_H;
-            for (int k = 0; k < LB_TB; ++k) g += (sdep[k] == dd) ? sd1[k][i] : 0.f;
-        } else if (p < LB_OFF_B2) {
-            const int i = (p - LB_OFF_W2) / LB_H, j = (p - LB_OFF_W2) % LB_H;
-            for (int k = 0; k < LB_TB; ++k) g = fmaf(sd2[k][i], sh1[k][j], g);
-        } else if (p < LB_OFF_W3) {
-            const int i = p - LB_OFF_B2;
-            for (int k = 0; k < LB_TB; ++k) g += sd2[k][i];
-        } else if (p < LB_OFF_B3) {
-            const int i = p - LB_OFF_W3;
-            for (int k = 0; k < LB_TB; ++k) g = fmaf(sdy[k], sh2[k][i], g);
-        } else {
-            for (int k = 0; k < LB_TB; ++k) g += sdy[k];
-        }
-        if (B.partial) B.partial[(int64_t)blockIdx.x * LB_NP + p] = g;
+
+    float *gf = B.partial ? B.partial + (int64_t)blockIdx.x * LB_NP : grad + f * LB_NP;
+    auto put = [&](int p, float g) {
+        if (B.partial) gf[p] = g;
         else atomicAdd(gf + p, g);
+    };
+    // products delta[i] x input[j] and delta[i + 16] x input[j] summed over
+    // the samples (consecutive threads take consecutive rows: no bank conflict)
+    auto outer = [&](const float(*dl)[LB_TS], int i, const float *in, float g[2]) {
+        g[0] = g[1] = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < LB_TB; k += 4) {
+            const float4 d0 = *(const float4 *)&dl[i][k], d1 = *(const float4 *)&dl[i + LB_H / 2][k];
+            const float4 x = *(const float4 *)&in[k];
+            g[0] = fmaf(d0.w, x.w, fmaf(d0.z, x.z, fmaf(d0.y, x.y, fmaf(d0.x, x.x, g[0]))));
+            g[1] = fmaf(d1.w, x.w, fmaf(d1.z, x.z, fmaf(d1.y, x.y, fmaf(d1.x, x.x, g[1]))));
+        }
+    };
+    {
+        float g[2];
+        const int i = tid >> 5, j = tid & 31;
+        outer(sd2, i, sh1[j], g);
+        put(LB_OFF_W2 + i * LB_H + j, g[0]);
+        put(LB_OFF_W2 + (i + LB_H / 2) * LB_H + j, g[1]);
+    }
+    if (tid < LB_H / 2 * LB_NIN) {  // 304 threads: W1
+        float g[2];
+        const int i = tid / LB_NIN, m = tid % LB_NIN;
+        outer(sd1, i, sx[m], g);
+        put(LB_OFF_W1 + i * LB_NIN + m, g[0]);
+        put(LB_OFF_W1 + (i + LB_H / 2) * LB_NIN + m, g[1]);
+    } else if (tid < 320) {
+        if (tid < 306) {  // the loss and b3
+            const float *v = tid == 304 ? sloss : sdy;
+            float a = 0.f;
+#pragma unroll 4
+            for (int k = 0; k < LB_TB; k += 4) {
+                const float4 q = *(const float4 *)&v[k];
+                a = (((a + q.x) + q.y) + q.z) + q.w;
+            }
+            if (tid == 305) put(LB_OFF_B3, a);
+            else if (B.ploss) B.ploss[blockIdx.x] = a * B.inv_total;
+            else atomicAdd(loss, a * B.inv_total);
+        }
+    } else if (tid < 448) {  // b1: depth q of unit i
+        const int i = tid & 31, q = (tid - 320) >> 5;
+        float a = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < LB_TB; k += 4) {
+            const float4 v = *(const float4 *)&sd1[i][k];
+            const int4 dk = *(const int4 *)&sdep[k];
+            a += dk.x == q ? v.x : 0.f;
+            a += dk.y == q ? v.y : 0.f;
+            a += dk.z == q ? v.z : 0.f;
+            a += dk.w == q ? v.w : 0.f;
+        }
+        put(LB_OFF_B1 + q * LB_H + i, a);
+    } else if (tid < 480) {  // b2
+        const int i = tid - 448;
+        float a = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < LB_TB; k += 4) {
+            const float4 v = *(const float4 *)&sd2[i][k];
+            a = (((a + v.x) + v.y) + v.z) + v.w;
+        }
+        put(LB_OFF_B2 + i, a);
+    } else {  // w3
+        const int i = tid - 480;
+        float a = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < LB_TB; k += 4) {
+            const float4 v = *(const float4 *)&sh2[i][k], q = *(const float4 *)&sdy[k];
+            a = fmaf(q.w, v.w, fmaf(q.z, v.z, fmaf(q.y, v.y, fmaf(q.x, v.x, a))));
+        }
+        put(LB_OFF_W3 + i, a);
     }
 }
 
-// Gradient of each face = its blocks' partial sums added in block order;
-// loss = the blocks' partial losses added in block order.
-__global__ void lb_reduce_kernel(LbBatch B, float *grad, float *loss)
+// One training step's update: the gradient of a parameter = its face's blocks'
+// partial sums added in block order, then Adam; the last block adds the
+// blocks' partial losses in block order (staged through LDS: a serial chain
+// of loads from memory took most of 40 us for 384 blocks).
+constexpr int LB_UT = 64;  // threads per block: 172 blocks, so the partial sums' loads spread over the chip
+__global__ void __launch_bounds__(LB_UT) lb_update_kernel(LbBatch B, float *theta, float *m, float *v, float *loss,
+                                                          float lr, float b1, float b2, float c1, float c2, float eps)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < LB_FACES * LB_NP) {
-        const int f = t / LB_NP, p = t - f * LB_NP;
-        float g = 0.f;
-        for (int b = B.block_start[f]; b < B.block_start[f + 1]; ++b) g += B.partial[(int64_t)b * LB_NP + p];
-        grad[t] = g;
-    }
-    if (t == 0) {
+    const int tid = threadIdx.x;
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ __align__(16) float part[4 * LB_UT];
+        const int n = B.block_start[LB_FACES];
         float acc = 0.f;
-        for (int b = 0; b < B.block_start[LB_FACES]; ++b) acc += B.ploss[b];
-        *loss = acc;
+        for (int k0 = 0; k0 < n; k0 += 4 * LB_UT) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int k = k0 + q * LB_UT + tid;
+                part[q * LB_UT + tid] = k < n ? B.ploss[k] : 0.f;
+            }
+            __syncthreads();
+            const int len = min(4 * LB_UT, n - k0);
+            if (tid == 0)
+                for (int k = 0; k < len; ++k) acc += part[k];
+            __syncthreads();
+        }
+        if (tid == 0) *loss = acc;
+        return;
     }
-}
-
-// Random minibatch positions: idx[f][n] uniform in [0, count_f).
-__global__ void lb_random_idx_kernel(int *idx, int n, int count, uint64_t seed)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) idx[t] = (int)(lb_hash(seed + 0x632be59bd9b4e019ull * (uint64_t)(t + 1)) % (uint32_t)count);
-}
-
-// Adam step on every parameter; clears the gradient.
-__global__ void lb_adam_kernel(float *theta, float *grad, float *m, float *v, int n, float lr, float b1, float b2,
-                               float c1, float c2, float eps)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const float g = grad[t];
+    const int t = blockIdx.x * LB_UT + tid;
+    if (t >= LB_FACES * LB_NP) return;
+    const int f = t / LB_NP, p = t - f * LB_NP;
+    const float *q = B.partial + p;
+    float g = 0.f;
+    int b = B.block_start[f];
+    const int end = B.block_start[f + 1];
+    for (; b + 16 <= end; b += 16) {
+        float x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = q[(int64_t)(b + k) * LB_NP];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) g += x[k];
+    }
+    for (; b < end; ++b) g += q[(int64_t)b * LB_NP];
     const float mt = b1 * m[t] + (1.f - b1) * g;
     const float vt = b2 * v[t] + (1.f - b2) * g * g;
     m[t] = mt;
     v[t] = vt;
     theta[t] -= lr * (mt * c1) / (sqrtf(vt * c2) + eps);
-    grad[t] = 0.f;
 }
 
 __global__ void lb_fill_kernel(float *p, int n, float val)
@@ -925,7 +1071,7 @@ using namespace phc;
 
 struct phc_lb {
     int device = 0;  // the device current at create (the stream's device)
-    DevBuf theta, grad, m, v, loss, wbf, idx;
+    DevBuf theta, grad, m, v, loss, wbf;
     DevBuf data[LB_FACES];
     DevBuf count;  // unsigned long long per face
     int64_t cap = 0;
@@ -935,10 +1081,10 @@ struct phc_lb {
 };
 
 // ---------------------------------------------------- training without allocation
-// phc_lb_train_noalloc keeps phc_lb_train's per-call buffers (minibatch
-// indices, per-block partial gradients and losses, loss history) in one static
-// device array, `scratch`, of fixed size: LB_NA_MAX_BATCH samples per face and
-// LB_NA_MAX_STEPS steps per call, 5.6 MiB.  Each GPU holds its own copy until
+// phc_lb_train_noalloc keeps phc_lb_train's per-call buffers (per-block
+// partial gradients and losses, loss history) in one static device array,
+// `scratch`, of fixed size: LB_NA_MAX_BATCH samples per face and
+// LB_NA_MAX_STEPS steps per call, 5.4 MiB.  Each GPU holds its own copy until
 // the process ends; its address on a device is resolved once, at the first
 // phc_lb_create with that device current, and kept in lb_na_ptr.  Calls on one
 // GPU share the array: calls that overlap on one GPU race.
@@ -949,9 +1095,7 @@ constexpr size_t lb_na_round(size_t n) { return (n + 63) / 64 * 64; }  // 256-by
 constexpr size_t LB_NA_PART = 0;
 constexpr size_t LB_NA_PLOSS = LB_NA_PART + lb_na_round((size_t)LB_NA_MAX_BLOCKS * LB_NP);
 constexpr size_t LB_NA_LOSS = LB_NA_PLOSS + lb_na_round(LB_NA_MAX_BLOCKS);
-constexpr size_t LB_NA_IDX = LB_NA_LOSS + lb_na_round(LB_NA_MAX_STEPS);
-constexpr size_t LB_NA_FLOATS = LB_NA_IDX + lb_na_round((size_t)LB_FACES * LB_NA_MAX_BATCH);
-static_assert(sizeof(int) == sizeof(float), "indices share the float array");
+constexpr size_t LB_NA_FLOATS = LB_NA_LOSS + lb_na_round(LB_NA_MAX_STEPS);
 
 static __device__ __align__(256) float scratch[LB_NA_FLOATS];
 
@@ -1003,7 +1147,7 @@ static phc_status lb_counts(phc_lb *h, int64_t c[LB_FACES])
 static phc_status lb_launch_train(phc_lb *h, const LbBatch &B)
 {
     if (B.block_start[LB_FACES] == 0) return PHC_OK;
-    hipLaunchKernelGGL(lb_train_kernel, dim3(B.block_start[LB_FACES]), dim3(LB_TB), 0, h->stream,
+    hipLaunchKernelGGL(lb_train_kernel, dim3(B.block_start[LB_FACES]), dim3(LB_TT), 0, h->stream,
                        h->theta.as<float>(), h->grad.as<float>(), h->loss.as<float>(), B);
     PHC_HIP(hipGetLastError());
     return PHC_OK;
@@ -1063,7 +1207,7 @@ phc_status phc_lb_destroy(phc_lb *h)
 {
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    for (DevBuf *b : {&h->theta, &h->grad, &h->m, &h->v, &h->loss, &h->wbf, &h->idx, &h->count}) b->release();
+    for (DevBuf *b : {&h->theta, &h->grad, &h->m, &h->v, &h->loss, &h->wbf, &h->count}) b->release();
     for (auto &b : h->data) b.release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -1266,14 +1410,15 @@ phc_status phc_lb_eval(phc_lb *h, float *loss, float *grad)
     for (int f = 0; f < LB_FACES; ++f) tot += c[f];
     if (tot == 0) return fail(PHC_ERR_STATE, "no samples");
     LbBatch B;
+    B.random = 0;
+    B.iseed = 0;
     B.noise = 0.f;
     B.nseed = 0;
     B.partial = B.ploss = nullptr;
     B.block_start[0] = 0;
     for (int f = 0; f < LB_FACES; ++f) {
         B.samples[f] = h->data[f].as<float>();
-        B.idx[f] = nullptr;
-        B.count[f] = (int)c[f];
+        B.count[f] = B.population[f] = (int)c[f];
         B.block_start[f + 1] = B.block_start[f] + (int)((c[f] + LB_TB - 1) / LB_TB);
     }
     B.inv_total = 1.f / (float)tot;
@@ -1299,12 +1444,13 @@ phc_status phc_lb_set_train_noise(phc_lb *h, float std)
     return PHC_OK;
 }
 
-// The training loop of phc_lb_train on given per-call buffers: idx (LB_FACES x
-// batch_per_face ints), lh (steps floats), part (per-block partial gradients,
-// LB_NP floats per block), pl (per-block losses).  Every buffer is written
-// before it is read, so none needs clearing.
+// The training loop of phc_lb_train on given per-call buffers: lh (steps
+// floats), part (per-block partial gradients, LB_NP floats per block), pl
+// (per-block losses).  Every buffer is written before it is read, so none
+// needs clearing.  Two launches per step: the batch is drawn inside the
+// training kernel, the sums over blocks and Adam are one kernel.
 static phc_status lb_train_core(phc_lb *h, const int64_t *c, int steps, int batch_per_face, float lr, uint64_t seed,
-                                int *idx, float *lh, float *part, float *pl, float *loss_history)
+                                float *lh, float *part, float *pl, float *loss_history)
 {
     int nf = 0;
     for (int f = 0; f < LB_FACES; ++f) nf += c[f] > 0;
@@ -1312,32 +1458,27 @@ static phc_status lb_train_core(phc_lb *h, const int64_t *c, int steps, int batc
     B.block_start[0] = 0;
     for (int f = 0; f < LB_FACES; ++f) {
         B.samples[f] = h->data[f].as<float>();
-        B.idx[f] = idx + (size_t)f * batch_per_face;
+        B.population[f] = (int)c[f];
         B.count[f] = c[f] > 0 ? batch_per_face : 0;
         B.block_start[f + 1] = B.block_start[f] + (B.count[f] + LB_TB - 1) / LB_TB;
     }
+    B.random = 1;
     B.inv_total = 1.f / ((float)batch_per_face * nf);
     const int np = LB_FACES * LB_NP;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     B.partial = part;
     B.ploss = pl;
     for (int s = 0; s < steps; ++s) {
-        for (int f = 0; f < LB_FACES; ++f)
-            if (c[f] > 0)
-                hipLaunchKernelGGL(lb_random_idx_kernel, dim3((batch_per_face + 255) / 256), dim3(256), 0, h->stream,
-                                   idx + (size_t)f * batch_per_face, batch_per_face, (int)c[f],
-                                   seed * 1000003ull + (uint64_t)s * LB_FACES + f);
+        B.iseed = seed * 1000003ull + (uint64_t)s * LB_FACES;
         B.noise = h->noise;
         B.nseed = seed * 7919ull + (uint64_t)s;
-        hipLaunchKernelGGL(lb_train_kernel, dim3(B.block_start[LB_FACES]), dim3(LB_TB), 0, h->stream,
+        hipLaunchKernelGGL(lb_train_kernel, dim3(B.block_start[LB_FACES]), dim3(LB_TT), 0, h->stream,
                            h->theta.as<float>(), h->grad.as<float>(), lh + s, B);
-        hipLaunchKernelGGL(lb_reduce_kernel, dim3((np + 255) / 256), dim3(256), 0, h->stream, B,
-                           h->grad.as<float>(), lh + s);
         ++h->adam_t;
         const float c1 = 1.f / (1.f - std::pow(b1, (float)h->adam_t));
         const float c2 = 1.f / (1.f - std::pow(b2, (float)h->adam_t));
-        hipLaunchKernelGGL(lb_adam_kernel, dim3((np + 255) / 256), dim3(256), 0, h->stream, h->theta.as<float>(),
-                           h->grad.as<float>(), h->m.as<float>(), h->v.as<float>(), np, lr, b1, b2, c1, c2, eps);
+        hipLaunchKernelGGL(lb_update_kernel, dim3((np + LB_UT - 1) / LB_UT + 1), dim3(LB_UT), 0, h->stream, B,
+                           h->theta.as<float>(), h->m.as<float>(), h->v.as<float>(), lh + s, lr, b1, b2, c1, c2, eps);
     }
     PHC_HIP(hipGetLastError());
     PHC_TRY(lb_upload_bf16(h));
@@ -1370,13 +1511,12 @@ phc_status phc_lb_train(phc_lb *h, int steps, int batch_per_face, float lr, uint
     PHC_TRY(lb_train_check(h, steps, batch_per_face, lr, c));
     int nblocks = 0;
     for (int f = 0; f < LB_FACES; ++f) nblocks += c[f] > 0 ? (batch_per_face + LB_TB - 1) / LB_TB : 0;
-    PHC_TRY(h->idx.alloc(sizeof(int) * (size_t)batch_per_face * LB_FACES));
     DevBuf lh, part, pl;
     PHC_TRY(lh.alloc(sizeof(float) * std::max(steps, 1)));
     PHC_TRY(part.alloc(sizeof(float) * (size_t)nblocks * LB_NP));
     PHC_TRY(pl.alloc(sizeof(float) * (size_t)nblocks));
-    return lb_train_core(h, c, steps, batch_per_face, lr, seed, h->idx.as<int>(), lh.as<float>(), part.as<float>(),
-                         pl.as<float>(), loss_history);
+    return lb_train_core(h, c, steps, batch_per_face, lr, seed, lh.as<float>(), part.as<float>(), pl.as<float>(),
+                         loss_history);
 }
 
 phc_status phc_lb_train_noalloc(phc_lb *h, int steps, int batch_per_face, float lr, uint64_t seed,
@@ -1391,8 +1531,8 @@ phc_status phc_lb_train_noalloc(phc_lb *h, int steps, int batch_per_face, float 
         return fail(PHC_ERR_INVALID, "%d steps exceed the no-alloc limit %d per call", steps, LB_NA_MAX_STEPS);
     float *base = lb_na_base(h->device);
     if (!base) return fail(PHC_ERR_STATE, "no scratch address for device %d", h->device);
-    return lb_train_core(h, c, steps, batch_per_face, lr, seed, reinterpret_cast<int *>(base + LB_NA_IDX),
-                         base + LB_NA_LOSS, base + LB_NA_PART, base + LB_NA_PLOSS, loss_history);
+    return lb_train_core(h, c, steps, batch_per_face, lr, seed, base + LB_NA_LOSS, base + LB_NA_PART,
+                         base + LB_NA_PLOSS, loss_history);
 }
 
 phc_status phc_lb_infer(phc_lb *h, int face, const float *samples, int64_t n, float *y)

@@ -312,3 +312,47 @@ def test_training_repeats_bit_for_bit(gpu, noise):
     assert np.array_equal(runs[0][0], runs[1][0])
     assert np.array_equal(runs[0][1], runs[1][1])
     assert np.all(np.isfinite(runs[0][0]))
+
+
+def drawn_positions(seed, face, batch, population):
+    """Positions phc_lb_train draws for the first step: a splittable hash of
+    (seed, face, n) modulo the stored count."""
+    with np.errstate(over="ignore"):
+        x = (np.uint64(seed) * np.uint64(1000003) + np.uint64(face)
+             + np.uint64(0x632be59bd9b4e019) * np.arange(1, batch + 1, dtype=np.uint64))
+        x ^= x >> np.uint64(33)
+        x *= np.uint64(0xff51afd7ed558ccd)
+        x ^= x >> np.uint64(33)
+        x *= np.uint64(0xc4ceb9fe1a85ec53)
+        x ^= x >> np.uint64(33)
+    return (x.astype(np.uint32) % np.uint32(population)).astype(int)
+
+
+@pytest.mark.parametrize("batch", [1, 63, 64, 65, 1030])
+def test_one_training_step_matches_oracle(gpu, batch):
+    """Minibatches below, at and past the 64 samples of a block, one face
+    without samples: the first loss within the gradient tests' 1e-4, and Adam's
+    first update -lr g / (|g| + 1e-8) wherever |g| is far enough from 0 for its
+    sign to be certain (FP32 gradients are within 1e-4 of the largest) and for
+    the 1e-8 to change it by less than 1e-3; theta's own rounding adds 6e-5."""
+    banner("one training step, batch %d" % batch)
+    rng = np.random.default_rng(31)
+    data = random_samples(rng, [500, 90, 0, 64, 1, 2000])
+    lb = gpu.LearnedBoundary(seed=12)
+    lb.set_capacity(2048)
+    for f, S in enumerate(data):
+        if len(S):
+            lb.add_samples(f, S)
+    before = lb.params().astype(np.float64)
+    lr = 1e-3
+    hist = lb.train(1, batch_per_face=batch, lr=lr, seed=7)
+    after = lb.params().astype(np.float64)
+    lb.close()
+    drawn = [S[drawn_positions(7, f, batch, len(S))] if len(S) else S for f, S in enumerate(data)]
+    loss, grad = lo.loss_grad(before, drawn)
+    assert abs(hist[0] - loss) <= 1e-4 * loss
+    sure = np.abs(grad) >= max(1e-3 * np.abs(grad).max(), 1e-5)
+    assert sure.sum() > 500
+    want = -lr * np.sign(grad)
+    assert np.max(np.abs((after - before) - want)[sure]) <= 2e-3 * lr
+    assert np.array_equal(after[2], before[2])
