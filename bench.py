@@ -11,7 +11,7 @@ roofline block uses the mean stencil-kernel duration from those events and
 16 algorithmic bytes per point update (read pn, pnm1, vp^2dt^2; write pnp1).
 
 Beside the headline line: "batch" reports the batched multi-shot workload
-(64 uneven shots, 800 steps, one persistent launch per step) and the same shots
+(64 uneven shots, 800 steps, one launch per step) and the same shots
 run one at a time; "sem_p4" the SEM order-4 workload (401^3 nodes, FP32
 separable kernel, and its FP32-vs-FP64 precision over 2000 steps);
 "sem2d" the SEM2D step on the reference's published 2D mesh and on a large 2D
@@ -136,7 +136,7 @@ def cpu_baseline_sem2d(steps=200):
 def bench_batch(phc, nsteps=800, nshots=64, baselines=True, shape=None):
     """Batched multi-shot FD: 64 shots, each axis drawn from U[128, 384], per-shot
     6-layer vp and Ricker f0 in U[5, 15] Hz, 20-point sponge, dt from CFL 0.4,
-    nsteps steps; all shots advanced by one persistent launch per step, the run
+    nsteps steps; all shots advanced by one launch per step, the run
     captured in one hipGraph.  Baselines: the same shots run one after the
     other through the single-grid path (graph-captured each), with its default
     launch shape and with a shape autotuned per shot."""

@@ -349,7 +349,7 @@ int phc_sem_element_from_point(int ex, int ey, int ez, float lx, float ly, float
                                float y, float z);
 
 /* ================================================================= BATCH
- * Many FD shots advanced together: one persistent launch per time step does
+ * Many FD shots advanced together: one launch per time step does
  * the FD step of every shot.  Each shot is the FD problem of the reference's
  * driver (src/fd/FDTDmain.cpp:9-108: FDTDKernel::addRHS + computeOneStepSB per
  * sample, FDTDkernels.hpp:75-128) on its own grid size, source position,
@@ -373,13 +373,16 @@ typedef struct {
     float sponge_alpha;
     float init_value;         /* initial value of both levels */
     int arith;                /* PHC_FD_ARITH_* */
-    int tile_j, block_waves;  /* 0 = default (16 x 16) */
-    int chunk_i;              /* planes per work item, 0 = default (64); -m
-                               * (m = 1..4): each shot's per-XCD schedule
-                               * (as phc_fd_params.chunk_i), XCD x's entries
-                               * in queue x, shot after shot */
-    int blocks_per_cu;        /* 0 = default (1) */
-    int k_remainder;          /* a shot's last, partial k tile: as in phc_fd_params */
+    int tile_j, block_waves;  /* 0 = default (8 x 8) */
+    int chunk_i;              /* planes per work item at most, 0 = chosen from
+                               * the shots' sizes; -m (m = 1..4): each shot's
+                               * per-XCD schedule (as phc_fd_params.chunk_i),
+                               * XCD x's entries to XCD x, shot after shot */
+    int blocks_per_cu;        /* blocks per CU one round of the per-XCD
+                               * schedules counts on, 0 = default (1) */
+    int k_remainder;          /* a shot's last, partial 64-point tile along k: 1
+                               * point by point, 0 (default) and -1 as a tile.
+                               * Same values either way. */
 } phc_batch_params;
 
 phc_status phc_batch_create(const phc_batch_params *p, phc_batch **out);
@@ -401,8 +404,8 @@ phc_status phc_batch_set_timing(phc_batch *h, int enable);
 /* Mean duration in ms of one batched step launch of the last timed run. */
 phc_status phc_batch_last_run_kernel_ms(phc_batch *h, double *ms_per_step);
 phc_status phc_batch_synchronize(phc_batch *h);
-/* Autotuner (no reference counterpart): block shape, chunk length and
- * resident blocks per CU timed on a copy of the shots (state not advanced). */
+/* Autotuner (no reference counterpart): block shape, chunk length and the
+ * schedules' blocks per CU timed on a copy of the shots (state not advanced). */
 phc_status phc_batch_autotune(phc_batch *h, int steps_per_trial, int *tile_j, int *block_waves,
                               int *chunk_i, int *blocks_per_cu);
 

@@ -1,15 +1,14 @@
-// batch.hip -- many FD shots on uneven grids in one persistent launch per
-// time step (phc_batch_* C ABI).
+// batch.hip -- many FD shots on uneven grids, one launch per time step
+// (phc_batch_* C ABI).
 //
 // No reference counterpart: the reference runs one shot per process (its FD
 // driver, src/fd/FDTDmain.cpp:9-108).  Each shot here is exactly that FD
 // problem -- same setup, same step (FDTDkernels.hpp:8-34, 108-128), same
 // sponge -- on its own grid size, source and model.  One launch advances every
-// shot by one step: the (shot, tile, chunk) work items of all shots are dealt
-// to a fixed number of resident blocks, each block marching its items with the
-// same tile body as the single-grid kernel (fd_tile).  The run is captured in
-// one hipGraph; the autotuner picks block shape, chunk length and resident
-// blocks per CU.
+// shot by one step: one block per (shot, tile column, plane range) work item,
+// dealt to the XCDs by a host-built table, each block marching its item with
+// the same tile body as the single-grid kernel (fd_tile).  The run is captured
+// in one hipGraph; the autotuner picks block shape and chunk length.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -33,17 +32,14 @@ struct ShotDesc {
     const float *rhs;
     int64_t src_off;
     int krem;         // first k of the shot's remainder slab (0: none)
+    int tiles_k;      // k tiles of the shot's tile columns
 };
 
-// One unit of work: tile column (kt, jt) of i-chunk ic of one shot; kt < 0:
-// part jt of the shot's k-remainder slab, BATCH_SLAB_PASSES x the block's
-// threads points in slab order.
-// A tile column (k tile kt, j tile jt) of one shot marched over planes
-// [i0, i1); kt < 0: part jt of the shot's remainder slab.
-struct WorkItem {
-    int shot, kt, jt, i0, i1;
-};
-constexpr int BATCH_SLAB_PASSES = 8;
+// One block's work, an int4 (shot, w, i0, i1): w >= 0: tile column w (k tile
+// w % tiles_k, j tile w / tiles_k) of the shot marched over planes [i0, i1);
+// w < 0: part -1 - w of the shot's k-remainder slab, BATCH_SLAB_PASSES x the
+// block's threads points in slab order; i0 >= i1: nothing (padding).
+constexpr int BATCH_SLAB_PASSES = 4;
 
 // The per-grid fields fd_tile reads, for one work item (scalar registers).
 struct FdGrid {
@@ -60,76 +56,81 @@ struct FdGrid {
     int jrem;  // no j-remainder slab in the batch (0)
 };
 
-// Work queues of one step: queue q holds items[start[q] .. start[q]+len[q]),
-// a contiguous run of tiles in spatial order of roughly equal cost.
-constexpr int BATCH_QUEUES = 8;  // one per XCD
-struct BatchQueues {
-    int start[BATCH_QUEUES];
-    int len[BATCH_QUEUES];
+constexpr int BATCH_XCDS = 8;
+
+// Receivers of the level a launch reads as current (the previous step's
+// result), sampled by extra blocks after the others, one receiver per thread.
+struct BatchSample {
+    const int64_t *off;
+    float *out;
+    int n, nrec, stride, step;  // n = shots x nrec (0: no sampling blocks)
 };
 
+// out[t * stride + step] = the level's value at receiver t.  A receiver on the
+// source point reads the value recorded before the fused injection of the
+// next step.
+__device__ __forceinline__ void batch_sample(const BatchSample &r, const ShotDesc *shots, const float *traces,
+                                             int level, int t)
+{
+    if (t >= r.n) return;
+    const int s = t / r.nrec;
+    const ShotDesc &d = shots[s];
+    const int64_t o = r.off[t];
+    r.out[(int64_t)t * r.stride + r.step] =
+        (o == d.src_off) ? traces[(int64_t)s * r.stride + r.step] : d.lev[level][o];
+}
+
 // One time step of every shot.  `c` holds what the shots share (coefficients,
-// sponge table, chunk length, deferred damping flag).  The hardware deals
-// consecutive blocks round-robin over the 8 XCDs, so block b starts on queue
-// b % 8: the blocks of one XCD take the tiles of one contiguous region in
-// order, and neighbouring tiles that run side by side share their halo rows
-// in that XCD's L2.  A block whose queue is empty takes items from the other
-// queues.  counter[q] (zero at the start of the step) is the next unclaimed
-// position of queue q.
+// sponge table, deferred damping flag).  The hardware deals block b to XCD
+// b % 8 and starts an XCD's blocks in order as slots on its CUs free up; the
+// table gives each XCD a contiguous run of items in spatial order and of
+// about equal cost, so neighbouring tiles that run side by side share their
+// halo rows in that XCD's L2.  A block holds one item and several blocks are
+// resident per CU, so one block's first loads (9 planes of ring, about 3 us
+// with the descriptor reads) run beside the others' marches; resident blocks
+// that claimed their items from a queue one after the other left that
+// latency and the claim's open: 12 shots of U[96,224]^3, best shape of each,
+// 200 us per step against 240 (47.7 M points: 3.8 against 3.2 TB/s).
 template <int R, int TY, int NJ, int ARITH, typename IT>
 __global__ void __launch_bounds__(FD_TK *TY)
-fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const WorkItem *__restrict__ items,
-                BatchQueues qs, int cur, int it, int inj, float *traces, int trace_stride, int step,
-                int *counter)
+fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__restrict__ items, int nitems,
+                int cur, int it, int inj, float *traces, int trace_stride, int step, BatchSample rec)
 {
     using SH = FdTileShape<R, TY, NJ>;
     __shared__ float tile[2][SH::LH][SH::LW];
-    __shared__ int claimed[2];  // alternating slots: a slot is rewritten two claims later,
-    int slot = 0;               // after a barrier every thread passes once it has read it
-    const bool leader = threadIdx.x == 0 && threadIdx.y == 0;
-    const int q0 = blockIdx.x % BATCH_QUEUES;
-    for (int d = 0; d < BATCH_QUEUES; ++d) {
-        const int q = (q0 + d) % BATCH_QUEUES;
-        while (true) {
-            if (leader) claimed[slot] = atomicAdd(counter + q, 1);
-            lds_barrier();
-            const int pos = claimed[slot];
-            slot ^= 1;
-            if (pos >= qs.len[q]) break;
-            const WorkItem wi = items[qs.start[q] + pos];
-            const ShotDesc &sd = shots[wi.shot];
-            FdGrid g;
-            g.L = sd.L;
-            g.pn = sd.lev[cur];
-            g.pnm1 = sd.lev[1 - cur];
-            g.vp = sd.vp;
-            g.fy = sd.fy;
-            g.fz = sd.fz;
-            g.src_off = sd.src_off;
-            g.inj = inj;
-            g.rhs_next = inj ? sd.rhs[it + 1] : 0.f;
-            g.trace = traces + (int64_t)wi.shot * trace_stride + step;
-            g.ilo = 0; g.ihi = sd.L.nx;
-            g.jlo = 0; g.jhi = sd.L.ny;
-            g.klo = 0; g.khi = sd.L.nz;
-            g.krem = sd.krem;
-            g.jrem = 0;
-            if (wi.kt < 0) {
-                constexpr int T = FD_TK * TY;
-                for (int m = 0; m < BATCH_SLAB_PASSES; ++m)
-                    fd_rem_points<R, ARITH, IT>(c, g, ((int64_t)wi.jt * BATCH_SLAB_PASSES + m) * T, T);
-                continue;
-            }
-            fd_tile<R, TY, NJ, ARITH, IT>(c, g, wi.kt, wi.jt, wi.i0, wi.i1, tile);
-        }
+    constexpr int T = FD_TK * TY;
+    if ((int)blockIdx.x >= nitems) {
+        batch_sample(rec, shots, traces, cur,
+                     ((int)blockIdx.x - nitems) * T + (int)(threadIdx.y * FD_TK + threadIdx.x));
+        return;
     }
-}
-
-// Zero the per-step work counters (a kernel, so that captured graphs replay it).
-__global__ void fd_batch_zero_kernel(int *counter, int n)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) counter[t] = 0;
+    const int4 wi = items[blockIdx.x];
+    if (wi.z >= wi.w) return;  // padding of a shorter XCD list (whole block)
+    const ShotDesc &sd = shots[wi.x];
+    FdGrid g;
+    g.L = sd.L;
+    g.pn = sd.lev[cur];
+    g.pnm1 = sd.lev[1 - cur];
+    g.vp = sd.vp;
+    g.fy = sd.fy;
+    g.fz = sd.fz;
+    g.src_off = sd.src_off;
+    g.inj = inj;
+    g.rhs_next = inj ? sd.rhs[it + 1] : 0.f;
+    g.trace = traces + (int64_t)wi.x * trace_stride + step;
+    g.ilo = 0; g.ihi = sd.L.nx;
+    g.jlo = 0; g.jhi = sd.L.ny;
+    g.klo = 0; g.khi = sd.L.nz;
+    g.krem = sd.krem;
+    g.jrem = 0;
+    if (wi.y < 0) {
+        const int64_t part = -1 - wi.y;
+        for (int m = 0; m < BATCH_SLAB_PASSES; ++m)
+            fd_rem_points<R, ARITH, IT>(c, g, (part * BATCH_SLAB_PASSES + m) * T, T);
+        return;
+    }
+    const int tk = sd.tiles_k;
+    fd_tile<R, TY, NJ, ARITH, IT>(c, g, wi.y % tk, wi.y / tk, wi.z, wi.w, tile);
 }
 
 // rhs[it] into every shot's current level at its source (FDTDkernels.hpp:121-128)
@@ -142,22 +143,14 @@ __global__ void fd_batch_inject_kernel(const ShotDesc *shots, int nshots, int cu
     p[d.src_off] = add_nc(p[d.src_off], mul_nc(d.vp[d.src_off], d.rhs[it]));
 }
 
-// Receiver sampling of every shot after a step: out[(shot*nrec + r)*stride +
-// step] = new level at the receiver.  A receiver on the source point reads the
-// value recorded before the fused injection of the next step.
-__global__ void fd_batch_sample_kernel(const ShotDesc *shots, int nshots, const int64_t *offs, int nrec,
-                                       int level, float *out, int stride, int step, const float *traces)
+// Receivers of the last step of a run (the others are sampled by the step launches).
+__global__ void fd_batch_sample_kernel(BatchSample rec, const ShotDesc *shots, const float *traces, int level)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nshots * nrec) return;
-    const int s = t / nrec;
-    const ShotDesc &d = shots[s];
-    const int64_t o = offs[t];
-    out[(int64_t)t * stride + step] = (o == d.src_off) ? traces[(int64_t)s * stride + step] : d.lev[level][o];
+    batch_sample(rec, shots, traces, level, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-using BatchFn = void (*)(FdStepArgs, const ShotDesc *, const WorkItem *, BatchQueues, int, int, int, float *,
-                        int, int, int *);
+using BatchFn = void (*)(FdStepArgs, const ShotDesc *, const int4 *, int, int, int, int, float *, int, int,
+                         BatchSample);
 
 template <int R, int TY, int NJ>
 static BatchFn batch_arith(int arith)
@@ -170,6 +163,7 @@ static BatchFn batch_pick(int R, int ty, int nj, int arith)
 {
     if (R != 4) return nullptr;
     if (ty == 16 && nj == 1) return batch_arith<4, 16, 1>(arith);
+    if (ty == 8 && nj == 1) return batch_arith<4, 8, 1>(arith);
     if (ty == 8 && nj == 2) return batch_arith<4, 8, 2>(arith);
     if (ty == 4 && nj == 2) return batch_arith<4, 4, 2>(arith);
     if (ty == 4 && nj == 4) return batch_arith<4, 4, 4>(arith);
@@ -190,15 +184,13 @@ struct phc_batch {
     std::vector<FdLayout> L;
     std::vector<int> src;
     std::vector<ShotDesc> hdesc;
-    DevBuf pool, shots, items, traces, rec, recoff, counters;
+    DevBuf pool, shots, items, traces, rec, recoff;
     int cur = 1;      // level holding the current field (the reference's i2)
     int pending = 0;  // the previous level still owes its sponge product
     hipStream_t stream = nullptr;
     int ty = 16, nj = 1, chunk_i = 64, blocks_per_cu = 1, cus = 256;
-    int krem_mode = 0;  // phc_batch_params.k_remainder (as requested)
-    int krem_eff = 0;   // the mode the work list uses (the autotuner may pick -1 for 0)
-    int nitems = 0;
-    BatchQueues queues;
+    int krem_mode = 0;  // phc_batch_params.k_remainder
+    int nitems = 0;  // entries of the work table, padding included
     int nrec = 0;  // receivers per shot
     int timing = 0;
     double last_ms = 0.0;
@@ -214,36 +206,53 @@ static void batch_drop_graph(phc_batch *h)
     h->g_it0 = h->g_n = h->g_cur = h->g_pending = h->g_nrec = -1;
 }
 
-// Work items of every shot for the current shape, dealt to BATCH_QUEUES
-// queues (one per XCD).  A shot whose last k tile would hold 1..32 points
-// (mode 0; any partial tile with mode 1, none with -1) gets its remainder
-// slab as point-by-point items instead.
+// Planes per work item when the caller gives none.  With x planes of tile
+// columns per resident block, items of c planes waste about (2R+1)/c of the
+// time on ring lead-ins (loads without a stencil) and c/2x on the part-empty
+// last round, so the best c grows with sqrt(x).  The factor 3 fits the best
+// chunk lengths measured (x = 20, 66, 112, 321: 16, 24, 32, 48).
+static int batch_default_chunk(const phc_batch *h, const int *dims)
+{
+    const int TJ = h->ty * h->nj;
+    double planes = 0.0;
+    for (int s = 0; s < h->nshots; ++s)
+        planes += (double)((dims[3 * s + 2] + FD_TK - 1) / FD_TK) * ((dims[3 * s + 1] + TJ - 1) / TJ) * dims[3 * s];
+    const double slots = (double)h->cus * std::max(32 / (h->ty * h->nj), 1);
+    return std::clamp((int)std::lround(3.0 * std::sqrt(planes / slots)), 8, 64);
+}
+
+// Work items of every shot for the current shape, one list per XCD,
+// interleaved into the table (entry 8 l + x = entry l of XCD x's list, shorter
+// lists padded).  With k_remainder 1 a shot's partial last k tile becomes
+// point-by-point items instead (as a tile it was faster on every survey
+// measured: 200 against 228 us per step on 12 shots of U[96,224]^3, 40
+// against 50 on 14 of U[60,100]^3, 642 against 686 on 24 of U[128,256]^3).
 // * chunk_i > 0: items in spatial order (shot, i-chunk, j-tile, k-tile,
 //   then the slab parts), cut into contiguous runs of about equal cost
 //   (planes incl. the 2R lead-in x rows; a slab point costs a few tile
 //   points: it reads its stencil from memory).
 // * chunk_i = -m: each shot's per-XCD schedule (xcd_sched.hpp, split m, one
-//   round = the XCD's resident blocks): queue x takes the entries of XCD x,
-//   shot after shot, so an XCD's blocks march one shot's plane range over a
-//   band of its columns in phase, as the single-grid schedule does; slab
-//   parts go to the queue with the least work so far.
+//   round = blocks_per_cu blocks on each of the XCD's CUs): list x takes the
+//   entries of XCD x, shot after shot; slab parts go to the list with the
+//   least work so far.
 static phc_status batch_build_items(phc_batch *h)
 {
-    std::vector<std::vector<WorkItem>> qitems(BATCH_QUEUES);
-    std::vector<double> qcost(BATCH_QUEUES, 0.0);
-    std::vector<WorkItem> items;
+    std::vector<std::vector<int4>> lists(BATCH_XCDS);
+    std::vector<double> lcost(BATCH_XCDS, 0.0);
+    std::vector<int4> items;
     std::vector<double> cost;
     const int TJ = h->ty * h->nj;
     const int T = FD_TK * h->ty;
     const bool sched = h->chunk_i < 0;
-    const int slots = std::max(h->cus / BATCH_QUEUES, 1) * h->blocks_per_cu;
+    const int slots = std::max(h->cus / BATCH_XCDS, 1) * h->blocks_per_cu;
     std::vector<int4> tab;
     for (int s = 0; s < h->nshots; ++s) {
         const FdLayout &L = h->L[s];
         const int full = L.nz / FD_TK, rem = L.nz - full * FD_TK;
-        const bool slab = h->krem_eff >= 0 && full > 0 && rem > 0 && (h->krem_eff == 1 || rem <= FD_TK / 2);
+        const bool slab = h->krem_mode == 1 && full > 0 && rem > 0;
         h->hdesc[s].krem = slab ? FD_TK * full : 0;
         const int tk = slab ? full : (L.nz + FD_TK - 1) / FD_TK, tj = (L.ny + TJ - 1) / TJ;
+        h->hdesc[s].tiles_k = tk;
         auto tile_cost = [&](int jt, int planes) {
             return (double)(planes + 2 * h->R) * std::min(TJ, L.ny - jt * TJ);
         };
@@ -252,60 +261,56 @@ static phc_status batch_build_items(phc_batch *h)
             for (size_t b = 0; b < tab.size(); ++b) {
                 const int4 e = tab[b];
                 if (e.y >= e.z) continue;
-                const int x = (int)(b % BATCH_QUEUES), kt = e.x % tk, jt = e.x / tk;
-                qitems[x].push_back({s, kt, jt, e.y, e.z});
-                qcost[x] += tile_cost(jt, e.z - e.y);
+                const int x = (int)(b % BATCH_XCDS);
+                lists[x].push_back(make_int4(s, e.x, e.y, e.z));
+                lcost[x] += tile_cost(e.x / tk, e.z - e.y);
             }
         } else {
             const int nc = (L.nx + h->chunk_i - 1) / h->chunk_i;
-            for (int ic = 0; ic < nc; ++ic)
-                for (int jt = 0; jt < tj; ++jt)
-                    for (int kt = 0; kt < tk; ++kt) {
-                        const int i0 = ic * h->chunk_i, i1 = std::min(i0 + h->chunk_i, L.nx);
-                        items.push_back({s, kt, jt, i0, i1});
-                        cost.push_back(tile_cost(jt, i1 - i0));
-                    }
+            for (int ic = 0; ic < nc; ++ic) {
+                const int i0 = (int)((int64_t)L.nx * ic / nc), i1 = (int)((int64_t)L.nx * (ic + 1) / nc);
+                for (int w = 0; w < tk * tj; ++w) {
+                    items.push_back(make_int4(s, w, i0, i1));
+                    cost.push_back(tile_cost(w / tk, i1 - i0));
+                }
+            }
         }
         if (slab) {
             const int64_t pts = (int64_t)rem * L.ny * L.nx, per = (int64_t)BATCH_SLAB_PASSES * T;
             for (int64_t q = 0; q * per < pts; ++q) {
                 const double c = 3.0 * (double)std::min(per, pts - q * per) / FD_TK;
+                const int4 it = make_int4(s, -1 - (int)q, 0, 1);
                 if (sched) {
-                    const int x = (int)(std::min_element(qcost.begin(), qcost.end()) - qcost.begin());
-                    qitems[x].push_back({s, -1, (int)q, 0, 0});
-                    qcost[x] += c;
+                    const int x = (int)(std::min_element(lcost.begin(), lcost.end()) - lcost.begin());
+                    lists[x].push_back(it);
+                    lcost[x] += c;
                 } else {
-                    items.push_back({s, -1, (int)q, 0, 0});
+                    items.push_back(it);
                     cost.push_back(c);
                 }
             }
         }
     }
-    // the descriptors carry each shot's slab start
+    // the descriptors carry each shot's slab start and tile count
     PHC_HIP(hipMemcpy(h->shots.ptr, h->hdesc.data(), sizeof(ShotDesc) * h->nshots, hipMemcpyHostToDevice));
-    if (sched) {
-        for (int k = 0; k < BATCH_QUEUES; ++k) {
-            h->queues.start[k] = (int)items.size();
-            h->queues.len[k] = (int)qitems[k].size();
-            items.insert(items.end(), qitems[k].begin(), qitems[k].end());
-        }
-    } else {
+    if (!sched) {
         const double total = std::accumulate(cost.begin(), cost.end(), 0.0);
-        int q = 0;
         double acc = 0.0;
-        h->queues.start[0] = 0;
         for (size_t i = 0; i < items.size(); ++i) {
+            // the list whose share of the cost holds the item's middle
+            const int x = (int)((acc + 0.5 * cost[i]) / total * BATCH_XCDS);
+            lists[std::min(x, BATCH_XCDS - 1)].push_back(items[i]);
             acc += cost[i];
-            while (q + 1 < BATCH_QUEUES && acc >= total * (q + 1) / BATCH_QUEUES) h->queues.start[++q] = (int)i + 1;
         }
-        while (q + 1 < BATCH_QUEUES) h->queues.start[++q] = (int)items.size();
-        for (int k = 0; k < BATCH_QUEUES; ++k)
-            h->queues.len[k] =
-                (k + 1 < BATCH_QUEUES ? h->queues.start[k + 1] : (int)items.size()) - h->queues.start[k];
     }
-    h->nitems = (int)items.size();
-    PHC_TRY(h->items.alloc(sizeof(WorkItem) * items.size()));
-    PHC_HIP(hipMemcpy(h->items.ptr, items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice));
+    size_t longest = 0;
+    for (const auto &l : lists) longest = std::max(longest, l.size());
+    std::vector<int4> table(BATCH_XCDS * longest, make_int4(0, 0, 0, 0));
+    for (int x = 0; x < BATCH_XCDS; ++x)
+        for (size_t l = 0; l < lists[x].size(); ++l) table[BATCH_XCDS * l + x] = lists[x][l];
+    h->nitems = (int)table.size();
+    PHC_TRY(h->items.alloc(sizeof(int4) * table.size()));
+    PHC_HIP(hipMemcpy(h->items.ptr, table.data(), sizeof(int4) * table.size(), hipMemcpyHostToDevice));
     return PHC_OK;
 }
 
@@ -324,54 +329,49 @@ static void batch_common(const phc_batch *h, FdStepArgs &c, int damp)
 
 // One batched step: every shot from level `cur` (current) and 1-cur
 // (previous, overwritten by the new level).  traces[shot*stride + step] gets
-// each shot's new source value before the fused injection of rhs[it+1].
+// each shot's new source value before the fused injection of rhs[it+1]; `rec`
+// samples the receivers of level `cur`.
 static phc_status batch_launch(phc_batch *h, int cur, int it, int inj, int damp, float *traces, int stride,
-                               int step, int *counter)
+                               int step, const BatchSample &rec)
 {
     BatchFn fn = batch_pick(h->R, h->ty, h->nj, h->arith);
     if (!fn) return fail(PHC_ERR_INVALID, "no batched kernel for %d waves x %d rows", h->ty, h->nj);
     FdStepArgs c;
     batch_common(h, c, damp);
-    // resident blocks, a multiple of the queue count (no more than there are items)
-    const int grid = std::max(BATCH_QUEUES, std::min(h->nitems, h->cus * h->blocks_per_cu) / BATCH_QUEUES * BATCH_QUEUES);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(FD_TK, h->ty), 0, h->stream, c, h->shots.as<ShotDesc>(),
-                       h->items.as<WorkItem>(), h->queues, cur, it, inj, traces, stride, step, counter);
+    const int T = FD_TK * h->ty;
+    hipLaunchKernelGGL(fn, dim3(h->nitems + (rec.n + T - 1) / T), dim3(FD_TK, h->ty), 0, h->stream, c,
+                       h->shots.as<ShotDesc>(), h->items.as<int4>(), h->nitems, cur, it, inj, traces, stride, step,
+                       rec);
     PHC_HIP(hipGetLastError());
     return PHC_OK;
 }
 
 // The whole run on h->stream: injection of rhs[it0] into every current level,
-// then one batched step per sample (plus receiver sampling).  With `ev`,
+// then one batched step per sample; a step's receivers are sampled by the
+// next step's launch, the last step's by a launch of their own.  With `ev`,
 // events bracket every batched launch.
-static phc_status batch_zero_counters(phc_batch *h, int n)
-{
-    hipLaunchKernelGGL(fd_batch_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, h->stream,
-                       h->counters.as<int>(), n);
-    PHC_HIP(hipGetLastError());
-    return PHC_OK;
-}
-
 static phc_status batch_enqueue(phc_batch *h, int it0, int nsteps, hipEvent_t *ev)
 {
-    PHC_TRY(batch_zero_counters(h, nsteps * BATCH_QUEUES));
     hipLaunchKernelGGL(fd_batch_inject_kernel, dim3((h->nshots + 63) / 64), dim3(64), 0, h->stream,
                        h->shots.as<ShotDesc>(), h->nshots, h->cur, it0);
     PHC_HIP(hipGetLastError());
     int cur = h->cur;
+    BatchSample rec{h->recoff.as<int64_t>(), h->rec.as<float>(), 0, h->nrec, nsteps, 0};
     for (int s = 0; s < nsteps; ++s) {
         const int damp = (s == 0) ? h->pending : (h->sw > 0 ? 1 : 0);
+        rec.n = s > 0 ? h->nshots * h->nrec : 0;
+        rec.step = s - 1;
         if (ev) PHC_HIP(hipEventRecord(ev[2 * s], h->stream));
-        PHC_TRY(batch_launch(h, cur, it0 + s, s + 1 < nsteps ? 1 : 0, damp, h->traces.as<float>(), nsteps, s,
-                             h->counters.as<int>() + s * BATCH_QUEUES));
+        PHC_TRY(batch_launch(h, cur, it0 + s, s + 1 < nsteps ? 1 : 0, damp, h->traces.as<float>(), nsteps, s, rec));
         if (ev) PHC_HIP(hipEventRecord(ev[2 * s + 1], h->stream));
-        if (h->nrec > 0) {
-            const int n = h->nshots * h->nrec;
-            hipLaunchKernelGGL(fd_batch_sample_kernel, dim3((n + 255) / 256), dim3(256), 0, h->stream,
-                               h->shots.as<ShotDesc>(), h->nshots, h->recoff.as<int64_t>(), h->nrec, 1 - cur,
-                               h->rec.as<float>(), nsteps, s, h->traces.as<float>());
-            PHC_HIP(hipGetLastError());
-        }
         cur = 1 - cur;
+    }
+    if (h->nrec > 0) {
+        rec.n = h->nshots * h->nrec;
+        rec.step = nsteps - 1;
+        hipLaunchKernelGGL(fd_batch_sample_kernel, dim3((rec.n + 255) / 256), dim3(256), 0, h->stream, rec,
+                           h->shots.as<ShotDesc>(), h->traces.as<float>(), cur);
+        PHC_HIP(hipGetLastError());
     }
     return PHC_OK;
 }
@@ -402,7 +402,11 @@ phc_status phc_batch_create(const phc_batch_params *p, phc_batch **out)
         return fail(PHC_ERR_INVALID, "bad chunk_i (planes per item, or -1..-4) or blocks_per_cu");
     if (p->k_remainder < -1 || p->k_remainder > 1)
         return fail(PHC_ERR_INVALID, "k_remainder must be -1, 0 or 1 (got %d)", p->k_remainder);
-    const int ty = p->block_waves ? p->block_waves : 16;
+    // default: 8 waves x 1 row, the fastest shape on every survey measured
+    // (12 shots of U[96,224]^3 / 14 of U[60,100]^3 / 24 of U[128,256]^3, best
+    // chunk of each: 200 / 40 / 642 us per step; 4 waves x 2 rows 216 / 43 /
+    // 690, 16 x 1 227 / 46 / 690)
+    const int ty = p->block_waves ? p->block_waves : p->tile_j ? 16 : 8;
     const int tj = p->tile_j ? p->tile_j : ty;
     if (ty <= 0 || tj % ty != 0 || !batch_pick(p->half_width, ty, tj / ty, p->arith))
         return fail(PHC_ERR_INVALID, "no batched kernel for tile_j %d, %d waves per block", tj, ty);
@@ -430,13 +434,14 @@ phc_status phc_batch_create(const phc_batch_params *p, phc_batch **out)
     h->src.assign(p->src, p->src + 3 * h->nshots);
     h->ty = ty;
     h->nj = tj / ty;
-    h->chunk_i = p->chunk_i ? p->chunk_i : 64;
+    h->chunk_i = p->chunk_i;
     h->blocks_per_cu = p->blocks_per_cu ? p->blocks_per_cu : 1;
-    h->krem_mode = h->krem_eff = p->k_remainder;
+    h->krem_mode = p->k_remainder;
     int dev = 0;
     hipDeviceProp_t prop;
     if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
         h->cus = prop.multiProcessorCount;
+    if (h->chunk_i == 0) h->chunk_i = batch_default_chunk(h, p->dims);
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(PHC_ERR_HIP, "hipStreamCreate failed"));
     // one pool: per shot two levels, vp^2dt^2, fy, fz, rhs; each shot 256-byte aligned
@@ -499,7 +504,7 @@ phc_status phc_batch_destroy(phc_batch *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     batch_drop_graph(h);
-    for (DevBuf *b : {&h->pool, &h->shots, &h->items, &h->traces, &h->rec, &h->recoff, &h->counters})
+    for (DevBuf *b : {&h->pool, &h->shots, &h->items, &h->traces, &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -541,13 +546,11 @@ phc_status phc_batch_run(phc_batch *h, int it0, int nsteps)
                     h->nsamples);
     const size_t tbytes = sizeof(float) * (size_t)nsteps * h->nshots;
     const size_t rbytes = tbytes * h->nrec;
-    const size_t cbytes = sizeof(int) * (size_t)nsteps * BATCH_QUEUES;
-    if (h->traces.bytes < tbytes || (h->nrec > 0 && h->rec.bytes < rbytes) || h->counters.bytes < cbytes) {
+    if (h->traces.bytes < tbytes || (h->nrec > 0 && h->rec.bytes < rbytes)) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         batch_drop_graph(h);
         if (h->traces.bytes < tbytes) PHC_TRY(h->traces.alloc(tbytes));
         if (h->nrec > 0 && h->rec.bytes < rbytes) PHC_TRY(h->rec.alloc(rbytes));
-        if (h->counters.bytes < cbytes) PHC_TRY(h->counters.alloc(cbytes));
     }
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
@@ -670,43 +673,35 @@ phc_status phc_batch_autotune(phc_batch *h, int steps_per_trial, int *tile_j, in
     PHC_HIP(hipStreamSynchronize(h->stream));
     batch_drop_graph(h);
     // trials run on a copy of the pool; the shots' state is restored after
-    DevBuf save, tr, ctr;
+    DevBuf save, tr;
     PHC_TRY(save.alloc(h->pool.bytes));
     PHC_TRY(tr.alloc(sizeof(float) * h->nshots));
-    const int nctr = steps_per_trial * BATCH_QUEUES;
-    PHC_TRY(ctr.alloc(sizeof(int) * nctr));
     PHC_HIP(hipMemcpy(save.ptr, h->pool.ptr, h->pool.bytes, hipMemcpyDeviceToDevice));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     PHC_HIP(hipEventCreate(&e0));
     PHC_HIP(hipEventCreate(&e1));
-    static const int shapes[][2] = {{16, 1}, {8, 2}, {4, 2}, {4, 4}};
-    static const int chunks[] = {32, 64, 128, 256, 512, -1, -2, -3, -4};
+    static const int shapes[][2] = {{16, 1}, {8, 1}, {8, 2}, {4, 2}, {4, 4}};
+    static const int chunks[] = {8, 16, 24, 32, 48, 64, 128, -1, -2, -3, -4};
     static const int bpcs[] = {1, 2, 4};
     double best = 1e30;
-    int bty = h->ty, bnj = h->nj, bci = h->chunk_i, bbp = h->blocks_per_cu, bku = h->krem_eff;
+    int bty = h->ty, bnj = h->nj, bci = h->chunk_i, bbp = h->blocks_per_cu;
     phc_status st = PHC_OK;
-    // requested mode 0: also the partial k tiles marched as tiles (-1)
-    const int modes[2] = {h->krem_mode, -1};
-    for (int mi = 0; mi < (h->krem_mode == 0 ? 2 : 1); ++mi)
     for (const auto &sh : shapes)
         for (int ci : chunks)
             for (int bp : bpcs) {
                 if (st != PHC_OK) break;
                 if (sh[0] * bp > 32) continue;  // at most 32 waves of one shape per CU
+                if (ci > 0 && bp > bpcs[0]) continue;  // only the per-XCD schedules depend on it
                 h->ty = sh[0];
                 h->nj = sh[1];
                 h->chunk_i = ci;
                 h->blocks_per_cu = bp;
-                h->krem_eff = modes[mi];
                 if ((st = batch_build_items(h))) break;
                 float ms = 0.f;
                 for (int rep = 0; rep < 2 && st == PHC_OK; ++rep) {  // first pass warms up
-                    hipLaunchKernelGGL(fd_batch_zero_kernel, dim3((nctr + 255) / 256), dim3(256), 0, h->stream,
-                                       ctr.as<int>(), nctr);
                     if (hipEventRecord(e0, h->stream) != hipSuccess) st = fail(PHC_ERR_HIP, "event record failed");
                     for (int s = 0; s < steps_per_trial && st == PHC_OK; ++s)
-                        st = batch_launch(h, (h->cur + s) & 1, 0, 0, h->sw > 0, tr.as<float>(), 1, 0,
-                                          ctr.as<int>() + s * BATCH_QUEUES);
+                        st = batch_launch(h, (h->cur + s) & 1, 0, 0, h->sw > 0, tr.as<float>(), 1, 0, BatchSample{});
                     if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess ||
                                          hipEventSynchronize(e1) != hipSuccess ||
                                          hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
@@ -714,7 +709,7 @@ phc_status phc_batch_autotune(phc_batch *h, int steps_per_trial, int *tile_j, in
                 }
                 if (st == PHC_OK && ms < best) {
                     best = ms;
-                    bty = h->ty; bnj = h->nj; bci = h->chunk_i; bbp = h->blocks_per_cu; bku = h->krem_eff;
+                    bty = h->ty; bnj = h->nj; bci = h->chunk_i; bbp = h->blocks_per_cu;
                 }
             }
     (void)hipEventDestroy(e0);
@@ -724,8 +719,7 @@ phc_status phc_batch_autotune(phc_batch *h, int steps_per_trial, int *tile_j, in
         st = fail(PHC_ERR_HIP, "restoring the shots after tuning failed");
     save.release();
     tr.release();
-    ctr.release();
-    h->ty = bty; h->nj = bnj; h->chunk_i = bci; h->blocks_per_cu = bbp; h->krem_eff = bku;
+    h->ty = bty; h->nj = bnj; h->chunk_i = bci; h->blocks_per_cu = bbp;
     PHC_TRY(st);
     PHC_TRY(batch_build_items(h));
     if (tile_j) *tile_j = bty * bnj;

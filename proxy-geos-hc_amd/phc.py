@@ -461,7 +461,7 @@ def multi_shot_setups(nshots=64, nmin=128, nmax=384, f0_range=(5.0, 15.0), nstep
 
 class FdBatch:
     """Many FD shots (FdSetup each, same half width, coefficients, sponge and
-    sample count) advanced together by the batched persistent kernel."""
+    sample count) advanced together by the batched kernel, one launch per step."""
 
     def __init__(self, setups, arith=ARITH_FP32, init_value=1e-6, tile_j=0, block_waves=0, chunk_i=0,
                  blocks_per_cu=0, k_remainder=0):

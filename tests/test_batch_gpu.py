@@ -184,3 +184,29 @@ def test_full_size_survey_every_shot_exact(gpu, oracle):
         assert np.array_equal(rsrc[k], tr), "shot %d" % k
         assert np.array_equal(r.field(k, True), P.current()), "shot %d current" % k
     r.close()
+
+
+@pytest.mark.parametrize("nrec,n", [(1, 1), (170, 2), (171, 3), (700, 6)])
+def test_receivers_fill_sampling_blocks(gpu, nrec, n):
+    """Receivers below, at and past one sampling block's threads (3 shots x nrec
+    against 512), one of them on the source, in runs of one to a few steps (the
+    last step is sampled by a launch of its own): the single-grid traces bit
+    for bit, on the default shape."""
+    banner("sampling blocks, %d receivers per shot, %d steps" % (nrec, n))
+    setups = make_shots(gpu, dims=DIMS[:3], sponge=6, nsamples=20)
+    rng = np.random.default_rng(nrec)
+    rec = np.stack([np.stack([rng.integers(0, d, nrec) for d in (s.nx, s.ny, s.nz)], 1) for s in setups])
+    for k, s in enumerate(setups):
+        rec[k, 0] = (s.xs, s.ys, s.zs)
+    b = gpu.FdBatch(setups)
+    b.set_receivers(rec)
+    b.run(9)
+    src, rv = b.run(n)
+    for k, s in enumerate(setups):
+        one = gpu.FdSolver(s, arith=gpu.ARITH_FP32)
+        one.set_receivers(rec[k])
+        one.run(0, 9)
+        tr, orv = one.run(9, n)
+        assert np.array_equal(src[k], tr) and np.array_equal(rv[k], orv), "shot %d" % k
+        one.close()
+    b.close()
