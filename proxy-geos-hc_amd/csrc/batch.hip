@@ -49,7 +49,6 @@ struct FdGrid {
     const float *vp, *fy, *fz;
     int64_t src_off;
     int inj;
-    float rhs_next;
     float *trace;
     int ilo, ihi, jlo, jhi, klo, khi;  // every point of the shot
     int krem;
@@ -94,7 +93,7 @@ __device__ __forceinline__ void batch_sample(const BatchSample &r, const ShotDes
 template <int R, int TY, int NJ, int ARITH, typename IT>
 __global__ void __launch_bounds__(FD_TK *TY)
 fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__restrict__ items, int nitems,
-                int cur, int it, int inj, float *traces, int trace_stride, int step, BatchSample rec)
+                int cur, const int *it0, int inj, float *traces, int trace_stride, int step, BatchSample rec)
 {
     using SH = FdTileShape<R, TY, NJ>;
     __shared__ float tile[2][SH::LH][SH::LW];
@@ -104,6 +103,7 @@ fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__
                      ((int)blockIdx.x - nitems) * T + (int)(threadIdx.y * FD_TK + threadIdx.x));
         return;
     }
+    const int it = uniform_value(it0) + step;
     const int4 wi = items[blockIdx.x];
     if (wi.z >= wi.w) return;  // padding of a shorter XCD list (whole block)
     const ShotDesc &sd = shots[wi.x];
@@ -116,7 +116,7 @@ fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__
     g.fz = sd.fz;
     g.src_off = sd.src_off;
     g.inj = inj;
-    g.rhs_next = inj ? sd.rhs[it + 1] : 0.f;
+    const float rhs_next = uniform_value(inj ? sd.rhs + it + 1 : nullptr);
     g.trace = traces + (int64_t)wi.x * trace_stride + step;
     g.ilo = 0; g.ihi = sd.L.nx;
     g.jlo = 0; g.jhi = sd.L.ny;
@@ -126,17 +126,19 @@ fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__
     if (wi.y < 0) {
         const int64_t part = -1 - wi.y;
         for (int m = 0; m < BATCH_SLAB_PASSES; ++m)
-            fd_rem_points<R, ARITH, IT>(c, g, (part * BATCH_SLAB_PASSES + m) * T, T);
+            fd_rem_points<R, ARITH, IT>(c, g, rhs_next, (part * BATCH_SLAB_PASSES + m) * T);
         return;
     }
     const int tk = sd.tiles_k;
-    fd_tile<R, TY, NJ, ARITH, IT>(c, g, wi.y % tk, wi.y / tk, wi.z, wi.w, tile);
+    fd_tile<R, TY, NJ, ARITH, IT>(c, g, rhs_next, wi.y % tk, wi.y / tk, wi.z, wi.w, tile);
 }
 
-// rhs[it] into every shot's current level at its source (FDTDkernels.hpp:121-128)
-__global__ void fd_batch_inject_kernel(const ShotDesc *shots, int nshots, int cur, int it)
+// Start of a run at sample it: rhs[it] into every shot's current level at its
+// source (FDTDkernels.hpp:121-128), and it where the run's steps read it.
+__global__ void fd_batch_inject_kernel(const ShotDesc *shots, int nshots, int cur, int it, int *it0)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) *it0 = it;
     if (s >= nshots) return;
     const ShotDesc &d = shots[s];
     float *p = d.lev[cur];
@@ -149,7 +151,7 @@ __global__ void fd_batch_sample_kernel(BatchSample rec, const ShotDesc *shots, c
     batch_sample(rec, shots, traces, level, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-using BatchFn = void (*)(FdStepArgs, const ShotDesc *, const int4 *, int, int, int, int, float *, int, int,
+using BatchFn = void (*)(FdStepArgs, const ShotDesc *, const int4 *, int, int, const int *, int, float *, int, int,
                          BatchSample);
 
 template <int R, int TY, int NJ>
@@ -184,7 +186,7 @@ struct phc_batch {
     std::vector<FdLayout> L;
     std::vector<int> src;
     std::vector<ShotDesc> hdesc;
-    DevBuf pool, shots, items, traces, rec, recoff;
+    DevBuf pool, shots, items, it0, traces, rec, recoff;
     int cur = 1;      // level holding the current field (the reference's i2)
     int pending = 0;  // the previous level still owes its sponge product
     hipStream_t stream = nullptr;
@@ -195,15 +197,12 @@ struct phc_batch {
     int timing = 0;
     double last_ms = 0.0;
     int last_n = 0, last_nrec = 0;
-    hipGraphExec_t gexec = nullptr;
-    int g_it0 = -1, g_n = -1, g_cur = -1, g_pending = -1, g_nrec = -1;
+    RunGraph graph[2];  // of phc_batch_run, by the level it starts from
 };
 
 static void batch_drop_graph(phc_batch *h)
 {
-    if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
-    h->gexec = nullptr;
-    h->g_it0 = h->g_n = h->g_cur = h->g_pending = h->g_nrec = -1;
+    for (RunGraph &g : h->graph) g.drop();
 }
 
 // Planes per work item when the caller gives none.  With x planes of tile
@@ -331,8 +330,8 @@ static void batch_common(const phc_batch *h, FdStepArgs &c, int damp)
 // (previous, overwritten by the new level).  traces[shot*stride + step] gets
 // each shot's new source value before the fused injection of rhs[it+1]; `rec`
 // samples the receivers of level `cur`.
-static phc_status batch_launch(phc_batch *h, int cur, int it, int inj, int damp, float *traces, int stride,
-                               int step, const BatchSample &rec)
+static phc_status batch_launch(phc_batch *h, int cur, int inj, int damp, float *traces, int stride, int step,
+                               const BatchSample &rec)
 {
     BatchFn fn = batch_pick(h->R, h->ty, h->nj, h->arith);
     if (!fn) return fail(PHC_ERR_INVALID, "no batched kernel for %d waves x %d rows", h->ty, h->nj);
@@ -340,21 +339,19 @@ static phc_status batch_launch(phc_batch *h, int cur, int it, int inj, int damp,
     batch_common(h, c, damp);
     const int T = FD_TK * h->ty;
     hipLaunchKernelGGL(fn, dim3(h->nitems + (rec.n + T - 1) / T), dim3(FD_TK, h->ty), 0, h->stream, c,
-                       h->shots.as<ShotDesc>(), h->items.as<int4>(), h->nitems, cur, it, inj, traces, stride, step,
+                       h->shots.as<ShotDesc>(), h->items.as<int4>(), h->nitems, cur, h->it0.as<int>(), inj, traces, stride, step,
                        rec);
     PHC_HIP(hipGetLastError());
     return PHC_OK;
 }
 
-// The whole run on h->stream: injection of rhs[it0] into every current level,
-// then one batched step per sample; a step's receivers are sampled by the
-// next step's launch, the last step's by a launch of their own.  With `ev`,
-// events bracket every batched launch.
-static phc_status batch_enqueue(phc_batch *h, int it0, int nsteps, hipEvent_t *ev)
+// A run's steps on h->stream (fd_batch_inject_kernel has gone before): one
+// batched step per sample; a step's receivers are sampled by the next step's
+// launch, the last step's by a launch of their own.  Names no time sample, so
+// that a captured run serves every chunk.  With `ev`, events bracket every
+// batched launch.
+static phc_status batch_enqueue(phc_batch *h, int nsteps, hipEvent_t *ev)
 {
-    hipLaunchKernelGGL(fd_batch_inject_kernel, dim3((h->nshots + 63) / 64), dim3(64), 0, h->stream,
-                       h->shots.as<ShotDesc>(), h->nshots, h->cur, it0);
-    PHC_HIP(hipGetLastError());
     int cur = h->cur;
     BatchSample rec{h->recoff.as<int64_t>(), h->rec.as<float>(), 0, h->nrec, nsteps, 0};
     for (int s = 0; s < nsteps; ++s) {
@@ -362,7 +359,7 @@ static phc_status batch_enqueue(phc_batch *h, int it0, int nsteps, hipEvent_t *e
         rec.n = s > 0 ? h->nshots * h->nrec : 0;
         rec.step = s - 1;
         if (ev) PHC_HIP(hipEventRecord(ev[2 * s], h->stream));
-        PHC_TRY(batch_launch(h, cur, it0 + s, s + 1 < nsteps ? 1 : 0, damp, h->traces.as<float>(), nsteps, s, rec));
+        PHC_TRY(batch_launch(h, cur, s + 1 < nsteps ? 1 : 0, damp, h->traces.as<float>(), nsteps, s, rec));
         if (ev) PHC_HIP(hipEventRecord(ev[2 * s + 1], h->stream));
         cur = 1 - cur;
     }
@@ -455,7 +452,8 @@ phc_status phc_batch_create(const phc_batch_params *p, phc_batch **out)
         total = round_up(total, 64);
     }
     phc_status st;
-    if ((st = h->pool.alloc(sizeof(float) * total)) || (st = h->shots.alloc(sizeof(ShotDesc) * h->nshots)))
+    if ((st = h->pool.alloc(sizeof(float) * total)) || (st = h->shots.alloc(sizeof(ShotDesc) * h->nshots)) ||
+        (st = h->it0.alloc(sizeof(int))))
         return bail(st);
     h->hdesc.resize(h->nshots);
     for (int s = 0; s < h->nshots; ++s) {
@@ -504,7 +502,7 @@ phc_status phc_batch_destroy(phc_batch *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     batch_drop_graph(h);
-    for (DevBuf *b : {&h->pool, &h->shots, &h->items, &h->traces, &h->rec, &h->recoff})
+    for (DevBuf *b : {&h->pool, &h->shots, &h->items, &h->it0, &h->traces, &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -552,10 +550,13 @@ phc_status phc_batch_run(phc_batch *h, int it0, int nsteps)
         if (h->traces.bytes < tbytes) PHC_TRY(h->traces.alloc(tbytes));
         if (h->nrec > 0 && h->rec.bytes < rbytes) PHC_TRY(h->rec.alloc(rbytes));
     }
+    hipLaunchKernelGGL(fd_batch_inject_kernel, dim3((h->nshots + 63) / 64), dim3(64), 0, h->stream,
+                       h->shots.as<ShotDesc>(), h->nshots, h->cur, it0, h->it0.as<int>());
+    PHC_HIP(hipGetLastError());
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = batch_enqueue(h, it0, nsteps, ev.data());
+        phc_status st = batch_enqueue(h, nsteps, ev.data());
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -569,27 +570,8 @@ phc_status phc_batch_run(phc_batch *h, int it0, int nsteps)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        if (!(h->gexec && h->g_it0 == it0 && h->g_n == nsteps && h->g_cur == h->cur &&
-              h->g_pending == h->pending && h->g_nrec == h->nrec)) {
-            batch_drop_graph(h);
-            hipGraph_t graph = nullptr;
-            PHC_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-            phc_status st = batch_enqueue(h, it0, nsteps, nullptr);
-            hipError_t ce = hipStreamEndCapture(h->stream, &graph);
-            if (st != PHC_OK) {
-                if (graph) (void)hipGraphDestroy(graph);
-                return st;
-            }
-            if (ce != hipSuccess) return fail(PHC_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ce));
-            hipError_t ie = hipGraphInstantiate(&h->gexec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if (ie != hipSuccess) {
-                h->gexec = nullptr;
-                return fail(PHC_ERR_HIP, "graph instantiate failed: %s", hipGetErrorString(ie));
-            }
-            h->g_it0 = it0; h->g_n = nsteps; h->g_cur = h->cur; h->g_pending = h->pending; h->g_nrec = h->nrec;
-        }
-        PHC_HIP(hipGraphLaunch(h->gexec, h->stream));
+        PHC_TRY(run_captured(h->stream, h->graph[h->cur], nsteps, h->pending, h->nrec,
+                             [&] { return batch_enqueue(h, nsteps, nullptr); }));
     }
     if (nsteps % 2) h->cur = 1 - h->cur;
     h->pending = h->sw > 0 ? 1 : 0;
@@ -701,7 +683,7 @@ phc_status phc_batch_autotune(phc_batch *h, int steps_per_trial, int *tile_j, in
                 for (int rep = 0; rep < 2 && st == PHC_OK; ++rep) {  // first pass warms up
                     if (hipEventRecord(e0, h->stream) != hipSuccess) st = fail(PHC_ERR_HIP, "event record failed");
                     for (int s = 0; s < steps_per_trial && st == PHC_OK; ++s)
-                        st = batch_launch(h, (h->cur + s) & 1, 0, 0, h->sw > 0, tr.as<float>(), 1, 0, BatchSample{});
+                        st = batch_launch(h, (h->cur + s) & 1, 0, h->sw > 0, tr.as<float>(), 1, 0, BatchSample{});
                     if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess ||
                                          hipEventSynchronize(e1) != hipSuccess ||
                                          hipEventElapsedTime(&ms, e0, e1) != hipSuccess))

@@ -46,7 +46,7 @@ __device__ __forceinline__ void fd_block_range(const FdStepArgs &a, int &kt, int
         i0 = e.y;
         i1 = e.z;
     } else {
-        const int b = xcd_block(blockIdx.x, a.nb_main ? a.nb_main : gridDim.x - (a.rec_n > 0 ? 1 : 0));
+        const int b = xcd_block(blockIdx.x, a.nb_main ? a.nb_main : (int)gridDim.x - a.rec_blocks);
         const int nt = a.tiles_k * a.tiles_j, ic = b / nt;
         w = b - ic * nt;
         i0 = a.ilo + ic * a.chunk_i;
@@ -56,13 +56,16 @@ __device__ __forceinline__ void fd_block_range(const FdStepArgs &a, int &kt, int
     jt = w / a.tiles_k;
 }
 
-// The extra block's receiver sampling (FdStepArgs::rec_n).
+// The extra blocks' receiver sampling (FdStepArgs::rec_n).  One block for all
+// of them ran into the march's tail with thousands of receivers (4 or more
+// rounds of two dependent loads each).
 __device__ __forceinline__ void fd_sample_prev(const FdStepArgs &a)
 {
-    for (int r = (int)(threadIdx.y * blockDim.x + threadIdx.x); r < a.rec_n; r += (int)(blockDim.x * blockDim.y)) {
-        const int64_t o = a.rec_off[r];
-        a.rec_out[(int64_t)r * a.rec_stride + a.rec_step] = (o == a.src_off) ? a.rec_src[a.rec_step] : a.pn[o];
-    }
+    const int b = (int)blockIdx.x - ((int)gridDim.x - a.rec_blocks);
+    const int r = b * (int)(blockDim.x * blockDim.y) + (int)(threadIdx.y * blockDim.x + threadIdx.x);
+    if (r >= a.rec_n) return;
+    const int64_t o = a.rec_off[r];
+    a.rec_out[(int64_t)r * a.rec_stride + a.rec_step] = (o == a.src_off) ? a.rec_src[a.rec_step] : a.pn[o];
 }
 
 template <int R, int TY, int NJ, int ARITH, typename IT>
@@ -71,18 +74,19 @@ fd_step_kernel(FdStepArgs a)
 {
     using SH = FdTileShape<R, TY, NJ>;
     __shared__ float tile[2][SH::LH][SH::LW];
-    if (a.rec_n > 0 && blockIdx.x == gridDim.x - 1) {
+    if ((int)blockIdx.x >= (int)gridDim.x - a.rec_blocks) {
         fd_sample_prev(a);
         return;
     }
+    const float rhs_next = uniform_value(a.rhs_next);
     if (a.nb_main && (int)blockIdx.x >= a.nb_main) {
-        fd_rem_points<R, ARITH, IT>(a, a, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY), FD_TK * TY);
+        fd_rem_points<R, ARITH, IT>(a, a, rhs_next, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY));
         return;
     }
     int kt, jt, i0, i1;
     fd_block_range(a, kt, jt, i0, i1);
     if (i0 >= i1) return;  // padding of a shorter XCD list (whole block)
-    fd_tile<R, TY, NJ, ARITH, IT>(a, a, kt, jt, i0, i1, tile);
+    fd_tile<R, TY, NJ, ARITH, IT>(a, a, rhs_next, kt, jt, i0, i1, tile);
 }
 
 // computeOneStepPML (FDTDkernels.hpp:87-104) in one launch: the march over
@@ -94,24 +98,35 @@ fd_step_pml_kernel(FdStepArgs a)
 {
     using SH = FdTileShape<R, TY, NJ>;
     __shared__ float tile[2][SH::LH][SH::LW];
-    if (a.rec_n > 0 && blockIdx.x == gridDim.x - 1) {
+    if ((int)blockIdx.x >= (int)gridDim.x - a.rec_blocks) {
         fd_sample_prev(a);
         return;
     }
+    const float rhs_next = uniform_value(a.rhs_next);
     if (a.nb_main && (int)blockIdx.x >= a.nb_main) {
-        fd_rem_points<R, ARITH, IT, true>(a, a, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY), FD_TK * TY);
+        fd_rem_points<R, ARITH, IT, true>(a, a, rhs_next, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY));
         return;
     }
     int kt, jt, i0, i1;
     fd_block_range(a, kt, jt, i0, i1);
     if (i0 >= i1) return;  // padding of a shorter XCD list (whole block)
-    fd_tile<R, TY, NJ, ARITH, IT, true>(a, a, kt, jt, i0, i1, tile);
+    fd_tile<R, TY, NJ, ARITH, IT, true>(a, a, rhs_next, kt, jt, i0, i1, tile);
 }
 
 // addRHS (FDTDkernels.hpp:121-128): one point.
 __global__ void fd_add_rhs_kernel(float *p, const float *vp, int64_t off, const float *rhs, int it)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) p[off] = add_nc(p[off], mul_nc(vp[off], rhs[it]));
+}
+
+// Start of a run: the run's source samples into its window, the first one
+// into the current level (addRHS).
+__global__ void fd_begin_run_kernel(float *p, const float *vp, int64_t off, const float *rhs, int it0, int n,
+                                    float *window)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) window[t] = rhs[it0 + t];
+    if (t == 0) p[off] = add_nc(p[off], mul_nc(vp[off], rhs[it0]));
 }
 
 // addRHS with the sample value handed over by the caller.
@@ -234,8 +249,8 @@ struct phc_fd {
     double coef0;
     int nsamples;
     FdLayout L;
-    DevBuf lev[2], vp, fx, fy, fz, rhs, trace, rec, recoff;
-    std::vector<float> hfx, hfy, hfz, hvp, hrhs;
+    DevBuf lev[2], vp, fx, fy, fz, rhs, window, trace, rec, recoff;
+    std::vector<float> hfx, hfy, hfz, hvp;
     int pending[2] = {0, 0};
     hipStream_t stream = nullptr;
     int ty = 4, nj = 2, chunk_i = 0, index64 = 0;
@@ -260,9 +275,7 @@ struct phc_fd {
     int lb_on = 0;
     LbInfer lbi;
     DevBuf lb_w, lb_corr, lb_kvcs, lb_kslab;
-    // cached graph of the last phc_fd_run
-    hipGraphExec_t gexec = nullptr;
-    int g_it0 = -1, g_n = -1, g_cur = -1, g_damp = -1, g_nrec = -1;
+    RunGraph graph[2];  // of phc_fd_run, by the level it starts from
 };
 
 static phc_status fd_validate(const phc_fd_params *p)
@@ -352,7 +365,7 @@ static void fd_fill_args(const phc_fd *h, FdStepArgs &a, int ca, int cb)
         a.stab[d] = (float)std::exp((double)h->alpha * std::pow((double)d, 2.0));
     a.src_off = fd_off(h->L, h->xs, h->ys, h->zs);
     a.inj = 0;
-    a.rhs_next = 0.f;
+    a.rhs_next = nullptr;
     a.trace = nullptr;
     const int TJ = h->ty * h->nj;
     a.tiles_k = (h->nz + FD_TK - 1) / FD_TK;
@@ -426,9 +439,7 @@ static phc_status fd_materialize(phc_fd *h, int level)
 
 static void fd_drop_graph(phc_fd *h)
 {
-    if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
-    h->gexec = nullptr;
-    h->g_it0 = h->g_n = h->g_cur = h->g_damp = h->g_nrec = -1;
+    for (RunGraph &g : h->graph) g.drop();
 }
 
 static FdKernelFn fd_handle_kernel(const phc_fd *h)
@@ -487,7 +498,8 @@ static phc_status fd_launch_step(phc_fd *h, FdStepArgs a, bool damp)
     a.damp_prev = damp ? 1 : 0;
     int nb = 0;
     PHC_TRY(fd_plan_launch(h, a, &nb));
-    if (a.rec_n > 0) ++nb;  // the sampling block
+    a.rec_blocks = (a.rec_n + FD_TK * h->ty - 1) / (FD_TK * h->ty);
+    nb += a.rec_blocks;
     hipLaunchKernelGGL(fn, dim3(nb), dim3(FD_TK, h->ty), 0, h->stream, a);
     PHC_HIP(hipGetLastError());
     return PHC_OK;
@@ -597,7 +609,6 @@ phc_status phc_fd_create(const phc_fd_params *p, phc_fd **out)
         hipMemcpy(h->fy.ptr, h->hfy.data(), sizeof(float) * h->ny, hipMemcpyHostToDevice) ||
         hipMemcpy(h->fz.ptr, h->hfz.data(), sizeof(float) * h->nz, hipMemcpyHostToDevice))
         return bail(fail(PHC_ERR_HIP, "sponge upload failed"));
-    h->hrhs.assign(p->rhs, p->rhs + h->nsamples);
     if (h->nsamples > 0) {
         if ((st = h->rhs.alloc(sizeof(float) * h->nsamples))) return bail(st);
         if (hipMemcpy(h->rhs.ptr, p->rhs, sizeof(float) * h->nsamples, hipMemcpyHostToDevice))
@@ -612,7 +623,7 @@ phc_status phc_fd_destroy(phc_fd *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     fd_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->vp, &h->fx, &h->fy, &h->fz, &h->rhs, &h->trace,
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->vp, &h->fx, &h->fy, &h->fz, &h->rhs, &h->window, &h->trace,
                       &h->rec, &h->recoff, &h->lb_w, &h->lb_corr, &h->lb_kvcs, &h->lb_kslab, &h->pml_ex,
                       &h->pml_ey, &h->pml_ez, &h->pml_phi})
         b->release();
@@ -703,26 +714,23 @@ phc_status phc_fd_set_receivers(phc_fd *h, int nrec, const int *ijk)
 
 } // extern "C"
 
-// Enqueue the whole run on h->stream: prologue injection of rhs[it0] into the
-// current level, then one fused step per time sample (injection of the next
-// sample folded into the store), plus receiver sampling.  With `ev`, events
-// bracket every stencil launch (timing mode).
-static phc_status fd_enqueue_run(phc_fd *h, int it0, int nsteps, int c0, bool damp0, hipEvent_t *ev)
+// Enqueue a run's steps on h->stream (fd_begin_run_kernel has filled the
+// window and injected its first sample): one fused step per time sample
+// (injection of the next sample folded into the store), each step's launch
+// sampling the receivers of the one before.  Names no time sample, so that a
+// captured run serves every chunk.  With `ev`, events bracket every stencil
+// launch (timing mode).
+static phc_status fd_enqueue_run(phc_fd *h, int nsteps, int c0, bool damp0, hipEvent_t *ev)
 {
-    hipLaunchKernelGGL(fd_add_rhs_kernel, dim3(1), dim3(64), 0, h->stream, h->lev[c0].as<float>(),
-                       h->vp.as<float>(), fd_off(h->L, h->xs, h->ys, h->zs), h->rhs.as<float>(),
-                       it0);
-    PHC_HIP(hipGetLastError());
     int c = c0;
     for (int s = 0; s < nsteps; ++s) {
-        const int it = it0 + s;
         const int ca = 1 - c, cb = c;
         FdStepArgs a;
         fd_fill_args(h, a, ca, cb);
         a.trace = h->trace.as<float>() + s;
         if (s + 1 < nsteps) {
             a.inj = 1;
-            a.rhs_next = h->hrhs[it + 1];
+            a.rhs_next = h->window.as<float>() + s + 1;
         }
         if (h->nrec > 0 && s > 0) {  // the previous step's receivers, by this launch
             a.rec_off = h->recoff.as<int64_t>();
@@ -765,20 +773,31 @@ phc_status phc_fd_run(phc_fd *h, int it0, int nsteps, int *cur)
     const int c0 = *cur;
     PHC_TRY(fd_materialize(h, c0));
     const bool damp0 = h->pending[1 - c0] != 0;
-    if (h->trace.bytes < sizeof(float) * nsteps) {
+    if (h->trace.bytes < sizeof(float) * nsteps || h->window.bytes < sizeof(float) * nsteps) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         fd_drop_graph(h);
         PHC_TRY(h->trace.alloc(sizeof(float) * nsteps));
+        PHC_TRY(h->window.alloc(sizeof(float) * nsteps));
     }
     if (h->nrec > 0 && h->rec.bytes < sizeof(float) * (size_t)nsteps * h->nrec) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         fd_drop_graph(h);
         PHC_TRY(h->rec.alloc(sizeof(float) * (size_t)nsteps * h->nrec));
     }
+    {   // the schedule table is uploaded now, not inside a capture
+        FdStepArgs a;
+        fd_fill_args(h, a, 1 - c0, c0);
+        int nb = 0;
+        PHC_TRY(fd_plan_launch(h, a, &nb));
+    }
+    hipLaunchKernelGGL(fd_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
+                       h->lev[c0].as<float>(), h->vp.as<float>(), fd_off(h->L, h->xs, h->ys, h->zs),
+                       h->rhs.as<float>(), it0, nsteps, h->window.as<float>());
+    PHC_HIP(hipGetLastError());
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = fd_enqueue_run(h, it0, nsteps, c0, damp0, ev.data());
+        phc_status st = fd_enqueue_run(h, nsteps, c0, damp0, ev.data());
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -792,34 +811,8 @@ phc_status phc_fd_run(phc_fd *h, int it0, int nsteps, int *cur)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        const int damp_key = damp0 ? 1 : 0;
-        if (!(h->gexec && h->g_it0 == it0 && h->g_n == nsteps && h->g_cur == c0 &&
-              h->g_damp == damp_key && h->g_nrec == h->nrec)) {
-            fd_drop_graph(h);
-            {   // the schedule table is uploaded now, not inside the capture
-                FdStepArgs a;
-                fd_fill_args(h, a, 1 - c0, c0);
-                int nb = 0;
-                PHC_TRY(fd_plan_launch(h, a, &nb));
-            }
-            hipGraph_t graph = nullptr;
-            PHC_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-            phc_status st = fd_enqueue_run(h, it0, nsteps, c0, damp0, nullptr);
-            hipError_t ce = hipStreamEndCapture(h->stream, &graph);
-            if (st != PHC_OK) {
-                if (graph) (void)hipGraphDestroy(graph);
-                return st;
-            }
-            if (ce != hipSuccess) return fail(PHC_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ce));
-            hipError_t ie = hipGraphInstantiate(&h->gexec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if (ie != hipSuccess) {
-                h->gexec = nullptr;
-                return fail(PHC_ERR_HIP, "graph instantiate failed: %s", hipGetErrorString(ie));
-            }
-            h->g_it0 = it0; h->g_n = nsteps; h->g_cur = c0; h->g_damp = damp_key; h->g_nrec = h->nrec;
-        }
-        PHC_HIP(hipGraphLaunch(h->gexec, h->stream));
+        PHC_TRY(run_captured(h->stream, h->graph[c0], nsteps, damp0 ? 1 : 0, h->nrec,
+                             [&] { return fd_enqueue_run(h, nsteps, c0, damp0, nullptr); }));
     }
     const int cend = (nsteps % 2 == 0) ? c0 : 1 - c0;
     h->pending[cend] = 0;

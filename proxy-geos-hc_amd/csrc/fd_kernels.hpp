@@ -59,8 +59,8 @@ struct FdStepArgs {
     float stab[FD_MAX_SW + 1];  // exp(alpha d^2), d = 0..sw (read with a uniform index)
     int64_t src_off;    // offset of the source point
     int damp_prev;      // previous level is read damped (deferred applySponge)
-    int inj;            // add vp[src]*rhs_next at src after the update
-    float rhs_next;
+    int inj;            // add vp[src] * *rhs_next at src after the update
+    const float *rhs_next;  // in the run's sample window (device memory)
     float *trace;       // if set: *trace = new value at src before injection
     int tiles_k, tiles_j, chunk_i;
     // box of points this launch updates: i in [ilo, ihi) (marched in chunks
@@ -88,14 +88,14 @@ struct FdStepArgs {
     // sched[b].z); an empty range does nothing
     const int4 *sched;
     // receiver sampling of the level this launch reads as current (the
-    // previous step's result), by one extra block after the others:
-    // rec_out[r * rec_stride + rec_step] = pn[rec_off[r]], or
+    // previous step's result), by extra blocks after the others, one receiver
+    // per thread: rec_out[r * rec_stride + rec_step] = pn[rec_off[r]], or
     // rec_src[rec_step] (the value recorded before the fused injection) for a
-    // receiver on the source point (0 receivers: no extra block)
+    // receiver on the source point (0 receivers: no extra blocks)
     const int64_t *rec_off;
     float *rec_out;
     const float *rec_src;
-    int rec_n, rec_stride, rec_step;
+    int rec_n, rec_blocks, rec_stride, rec_step;
 };
 
 } // namespace phc

@@ -101,13 +101,14 @@ struct FdTileShape {
     static constexpr int LH = TJ + 2 * R;
 };
 
-// March of one tile column (k-tile kt, j-tile jt) of one grid over planes [i0, i1).
+// March of one tile column (k-tile kt, j-tile jt) of one grid over planes [i0, i1);
+// with g.inj, vp * rhs_next is added at the source point after its update.
 // PML: points outside the PML's inner box take the pml3D update (the
 // stencil values come from the same register ring and LDS tile), so one
 // launch covers the slabs and the inner box.
 template <int R, int TY, int NJ, int ARITH, typename IT, bool PML = false, class G>
-__device__ __forceinline__ void fd_tile(const FdStepArgs &a, const G &g, int kt, int jt, int i0, int i1,
-                                        float (*tile)[FdTileShape<R, TY, NJ>::LH][FdTileShape<R, TY, NJ>::LW])
+__device__ __forceinline__ void fd_tile(const FdStepArgs &a, const G &g, float rhs_next, int kt, int jt, int i0,
+                                        int i1, float (*tile)[FdTileShape<R, TY, NJ>::LH][FdTileShape<R, TY, NJ>::LW])
 {
     constexpr int TJ = TY * NJ;
     constexpr int LW = FD_TK + 2 * R;
@@ -310,7 +311,7 @@ __device__ __forceinline__ void fd_tile(const FdStepArgs &a, const G &g, int kt,
                         sto_nt(a.pml_phi, o, phin);
                         if ((int64_t)(o / S) == g.src_off) {
                             if (g.trace) *g.trace = val;
-                            if (g.inj) val = add_nc(val, mul_nc(vvj, g.rhs_next));
+                            if (g.inj) val = add_nc(val, mul_nc(vvj, rhs_next));
                         }
                         sto_nt(g.pnm1, o, val);
                         continue;
@@ -334,7 +335,7 @@ __device__ __forceinline__ void fd_tile(const FdStepArgs &a, const G &g, int kt,
                 const IT o = colq[jj] + pi;
                 if ((int64_t)(o / S) == g.src_off) {
                     if (g.trace) *g.trace = val;
-                    if (g.inj) val = add_nc(val, mul_nc(vvj, g.rhs_next));
+                    if (g.inj) val = add_nc(val, mul_nc(vvj, rhs_next));
                 }
                 sto_nt(g.pnm1, o, val);
             }
@@ -354,11 +355,10 @@ __device__ __forceinline__ void fd_tile(const FdStepArgs &a, const G &g, int kt,
 // k or a quarter tile along j: these loads are L2 hits of the rows the
 // neighbouring tiles stream).
 template <int R, int ARITH, typename IT, bool PML = false, class G>
-__device__ __forceinline__ void fd_rem_points(const FdStepArgs &a, const G &g, int64_t first, int nthreads)
+__device__ __forceinline__ void fd_rem_points(const FdStepArgs &a, const G &g, float rhs_next, int64_t first)
 {
     constexpr IT S = sizeof(IT) == 4 ? 4 : 1;
     const FdLayout &L = g.L;
-    (void)nthreads;
     int64_t t = first + (int64_t)threadIdx.y * blockDim.x + threadIdx.x;
     const int NI = g.ihi - g.ilo;
     const int64_t nA = g.krem > 0 ? (int64_t)(g.khi - g.krem) * (g.jhi - g.jlo) * NI : 0;
@@ -415,7 +415,7 @@ __device__ __forceinline__ void fd_rem_points(const FdStepArgs &a, const G &g, i
             sto_nt(a.pml_phi, o, phin);
             if ((int64_t)(o / S) == g.src_off) {
                 if (g.trace) *g.trace = val;
-                if (g.inj) val = add_nc(val, mul_nc(vvj, g.rhs_next));
+                if (g.inj) val = add_nc(val, mul_nc(vvj, rhs_next));
             }
             sto_nt(g.pnm1, o, val);
             return;
@@ -438,7 +438,7 @@ __device__ __forceinline__ void fd_rem_points(const FdStepArgs &a, const G &g, i
     }
     if ((int64_t)(o / S) == g.src_off) {
         if (g.trace) *g.trace = val;
-        if (g.inj) val = add_nc(val, mul_nc(vvj, g.rhs_next));
+        if (g.inj) val = add_nc(val, mul_nc(vvj, rhs_next));
     }
     sto_nt(g.pnm1, o, val);
 }

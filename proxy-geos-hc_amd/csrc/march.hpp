@@ -39,6 +39,20 @@ __device__ __forceinline__ float add_nc(float a, float b)
     return a + b;
 }
 
+// The value a kernel argument points to, the same for every lane and constant
+// during the launch: a scalar load (kernels issue it first, so it is there
+// long before it is used); 0 for a null pointer.
+__device__ __forceinline__ float uniform_value(const float *p)
+{
+    typedef const float __attribute__((address_space(4))) *cptr;
+    return p ? *(cptr)(uintptr_t)p : 0.f;
+}
+__device__ __forceinline__ int uniform_value(const int *p)
+{
+    typedef const int __attribute__((address_space(4))) *cptr;
+    return p ? *(cptr)(uintptr_t)p : 0;
+}
+
 // Load / store through a kernel-argument base pointer.  With 32-bit offsets
 // the offset is in bytes, so the access is scalar base + 32-bit vector offset.
 template <typename IT, typename T = float>

@@ -67,6 +67,54 @@ struct DevBuf {
     template <class T> T *as() const { return static_cast<T *>(ptr); }
 };
 
+// A captured chunk of a time loop.  Its nodes name no time sample (the chunk's
+// samples sit in a device window that a launch before the graph fills), so
+// one graph serves every chunk of the same length that starts from the same
+// levels; a handle keeps two, one per level parity.  Captured anew, a chunk
+// of 100 steps of the 196^2-node 2D mesh took 0.42 ms longer (1.19 against
+// 0.77 ms).
+struct RunGraph {
+    hipGraphExec_t exec = nullptr;
+    int n = -1, key = -1, nrec = -1;
+    void drop()
+    {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        exec = nullptr;
+        n = key = nrec = -1;
+    }
+};
+
+// Launches the graph of an n-step chunk, capturing `enqueue` first when the
+// slot holds another one (key: whatever else the nodes depend on).
+template <class F>
+phc_status run_captured(hipStream_t stream, RunGraph &g, int n, int key, int nrec, F enqueue)
+{
+    if (!(g.exec && g.n == n && g.key == key && g.nrec == nrec)) {
+        if (g.exec) PHC_HIP(hipStreamSynchronize(stream));  // the old graph may still run
+        g.drop();
+        hipGraph_t graph = nullptr;
+        PHC_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        const phc_status st = enqueue();
+        const hipError_t ce = hipStreamEndCapture(stream, &graph);
+        if (st != PHC_OK) {
+            if (graph) (void)hipGraphDestroy(graph);
+            return st;
+        }
+        if (ce != hipSuccess) return fail(PHC_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ce));
+        const hipError_t ie = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(graph);
+        if (ie != hipSuccess) {
+            g.exec = nullptr;
+            return fail(PHC_ERR_HIP, "graph instantiate failed: %s", hipGetErrorString(ie));
+        }
+        g.n = n;
+        g.key = key;
+        g.nrec = nrec;
+    }
+    PHC_HIP(hipGraphLaunch(g.exec, stream));
+    return PHC_OK;
+}
+
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
 } // namespace phc

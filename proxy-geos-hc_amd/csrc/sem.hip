@@ -54,7 +54,7 @@ struct SemSepArgs {
     int64_t src_off;   // layout offset of the source node
     int inj;
     float inj_coef;    // dt^2 c^2 of the source element (SEMsolver.cpp:41-42)
-    float rhs_next;
+    const float *rhs_next;  // in the run's sample window (device memory)
     float *trace;
     int tiles_k, tiles_j, chunk_i;
     // per-XCD schedule (null: one block per (tile, chunk of chunk_i planes)
@@ -65,13 +65,30 @@ struct SemSepArgs {
     // nodes, the tiles stop at x = krem and the blocks from nb_main on update
     // the interior nodes with x in [krem, nz - 1) one per thread
     int nb_main, krem;
+    // receiver sampling of the level this launch reads as current (the
+    // previous step's result) by rec_blocks extra blocks after the others,
+    // one receiver per thread: rec_out[r * rec_stride + rec_step]; a receiver
+    // on the source node takes rec_src[rec_step], recorded before injection
+    const int64_t *rec_off;
+    float *rec_out;
+    const float *rec_src;
+    int rec_n, rec_blocks, rec_stride, rec_step;
 };
+
+// out[r * stride + step] = level value of receiver r (the source node already
+// holds the next sample's injection: its trace has the value before).
+__device__ __forceinline__ void sem_sample_point(const float *p, const int64_t *offs, int r, float *out, int stride,
+                                                 int step, int64_t src_off, const float *src_trace)
+{
+    const int64_t o = offs[r];
+    out[(int64_t)r * stride + step] = (o == src_off) ? src_trace[step] : p[o];
+}
 
 // One node of the x-remainder slab per thread: the separable update with the
 // same operations in the same order as the march (so a node gets the same
 // bits from either path), its stencil values read from memory.
 template <int P, typename IT>
-__device__ __forceinline__ void sem_rem_points(const SemSepArgs &a, int64_t t)
+__device__ __forceinline__ void sem_rem_points(const SemSepArgs &a, float rhs_next, int64_t t)
 {
     constexpr int R = P, W = 2 * P + 1;
     constexpr IT S = sizeof(IT) == 4 ? 4 : 1;
@@ -97,7 +114,7 @@ __device__ __forceinline__ void sem_rem_points(const SemSepArgs &a, int64_t t)
     float val = fmaf(-ldo(a.qf, o), lap, 2.f * pc - ldo(a.pnm1, o));
     if ((int64_t)(o / S) == a.src_off) {
         if (a.trace) *a.trace = val;
-        if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, a.rhs_next));
+        if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, rhs_next));
     }
     sto_nt(a.pnm1, o, val);
 }
@@ -124,8 +141,16 @@ sem_sep_kernel(SemSepArgs a)
     constexpr IT S = sizeof(IT) == 4 ? 4 : 1;
     __shared__ float tile[2][LH][LW];
 
+    if ((int)blockIdx.x >= (int)gridDim.x - a.rec_blocks) {
+        const int r = ((int)blockIdx.x - ((int)gridDim.x - a.rec_blocks)) * (FD_TK * TY) +
+                      (int)(threadIdx.y * FD_TK + threadIdx.x);
+        if (r < a.rec_n)
+            sem_sample_point(a.pn, a.rec_off, r, a.rec_out, a.rec_stride, a.rec_step, a.src_off, a.rec_src);
+        return;
+    }
+    const float rhs_next = uniform_value(a.rhs_next);
     if (a.nb_main && (int)blockIdx.x >= a.nb_main) {
-        sem_rem_points<P, IT>(a, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY) +
+        sem_rem_points<P, IT>(a, rhs_next, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY) +
                                      (int64_t)threadIdx.y * FD_TK + threadIdx.x);
         return;
     }
@@ -139,7 +164,7 @@ sem_sep_kernel(SemSepArgs a)
         i1 = e.z;
         if (i0 >= i1) return;  // padding of a shorter XCD list (whole block)
     } else {
-        const int b = xcd_block(blockIdx.x, a.nb_main ? a.nb_main : gridDim.x);
+        const int b = xcd_block(blockIdx.x, a.nb_main ? a.nb_main : (int)gridDim.x - a.rec_blocks);
         const int ic = b / (a.tiles_k * a.tiles_j);
         w = b - ic * (a.tiles_k * a.tiles_j);
         i0 = ic * a.chunk_i;
@@ -274,7 +299,7 @@ sem_sep_kernel(SemSepArgs a)
                 const IT o = colq[jj] + pi;
                 if ((int64_t)(o / S) == a.src_off) {
                     if (a.trace) *a.trace = val;
-                    if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, a.rhs_next));
+                    if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, rhs_next));
                 }
                 sto_nt(a.pnm1, o, val);
             }
@@ -529,7 +554,8 @@ struct SemMarchArgs {
     int tiles_x, tiles_z, ychunk;
     int64_t src_node;
     int inj;
-    float inj_coef, rhs_next;
+    float inj_coef;
+    const float *rhs_next;  // in the run's sample window
     float *trace;
 };
 
@@ -708,7 +734,7 @@ __global__ void __launch_bounds__(NT) sem_march_kernel(SemMarchArgs a)
                         float val = fmaf(-a.dt2m[n], g, 2.f * u[slot[cc]][Z][X] - a.pnm1[n]);
                         if (n == a.src_node) {
                             if (a.trace) *a.trace = val;
-                            if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, a.rhs_next));
+                            if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, uniform_value(a.rhs_next)));
                         }
                         a.pnm1[n] = val;
                     }
@@ -725,7 +751,7 @@ __global__ void __launch_bounds__(NT) sem_march_kernel(SemMarchArgs a)
 // injection of the next time sample.
 __global__ void sem_update_kernel(float *pold, const float *pcur, float *y, const float *dt2m,
                                   int nx, int ny, int nz, int src_node, int inj, float inj_coef,
-                                  float rhs_next, float *trace)
+                                  const float *rhs_next, float *trace)
 {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nn = (int64_t)nx * ny * nz;
@@ -737,7 +763,7 @@ __global__ void sem_update_kernel(float *pold, const float *pcur, float *y, cons
     float val = fmaf(-dt2m[n], yv, 2.f * pcur[n] - pold[n]);
     if (n == src_node) {
         if (trace) *trace = val;
-        if (inj) val = add_nc(val, mul_nc(inj_coef, rhs_next));
+        if (inj) val = add_nc(val, mul_nc(inj_coef, uniform_value(rhs_next)));
     }
     pold[n] = val;
 }
@@ -762,9 +788,17 @@ __global__ void sem_sample_kernel(const float *p, const int64_t *offs, int nrec,
                                   int stride, int step, int64_t src_off, const float *src_trace)
 {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrec) return;
-    const int64_t o = offs[r];
-    out[(int64_t)r * stride + step] = (o == src_off) ? src_trace[step] : p[o];
+    if (r < nrec) sem_sample_point(p, offs, r, out, stride, step, src_off, src_trace);
+}
+
+// Start of a run: its source samples into the window, the first one into the
+// current level (SEMsolver.cpp:39-43).
+__global__ void sem_begin_run_kernel(float *p, int64_t off, float coef, const float *rhs, int it0, int n,
+                                     float *window)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) window[t] = rhs[it0 + t];
+    if (t == 0) p[off] = add_nc(p[off], mul_nc(coef, rhs[it0]));
 }
 
 using SemSepFn = void (*)(SemSepArgs);
@@ -847,7 +881,7 @@ struct phc_sem {
     int kernel;
     float dt;
     int nsamples;
-    std::vector<float> hrhs, model;
+    std::vector<float> model;
     int src_element, src_node;
     bool src_interior = true;  // boundary nodes are never updated: no fused injection
     float inj_coef;
@@ -868,13 +902,12 @@ struct phc_sem {
     DevBuf y, dt2m, geo, rhs;
     float Dm[(SEM_MAX_P + 1) * (SEM_MAX_P + 1)];
     std::vector<float> hmass;
-    // traces
-    DevBuf trace, rec, recoff;
+    // traces, and the running chunk's source samples
+    DevBuf trace, window, rec, recoff;
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
     double last_ms = 0.0;
-    hipGraphExec_t gexec = nullptr;
-    int g_it0 = -1, g_n = -1, g_i1 = -1, g_nrec = -1;
+    RunGraph graph[2];  // of phc_sem_run, by i1
 };
 
 static int64_t sem_off(const phc_sem *h, int64_t node)
@@ -887,9 +920,7 @@ static int64_t sem_off(const phc_sem *h, int64_t node)
 
 static void sem_drop_graph(phc_sem *h)
 {
-    if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
-    h->gexec = nullptr;
-    h->g_it0 = h->g_n = h->g_i1 = h->g_nrec = -1;
+    for (RunGraph &g : h->graph) g.drop();
 }
 
 // Upload a node-order host field into a level (layout conversion for the
@@ -967,10 +998,13 @@ static phc_status sem_prepare_sched(phc_sem *h)
 }
 
 // One step: level i1 <- update(level i1, level i2); optional fused injection
-// of the next sample and source trace.
-static phc_status sem_launch(phc_sem *h, int i1, int i2, int inj, float rhs_next, float *trace,
-                             hipEvent_t e0, hipEvent_t e1)
+// of the sample at rhs_next (device memory) and source trace.  rec_step >= 0:
+// the separable launch also samples level i2's receivers into that step of a
+// run of rec_stride steps.
+static phc_status sem_launch(phc_sem *h, int i1, int i2, const float *rhs_next, float *trace, hipEvent_t e0,
+                             hipEvent_t e1, int rec_step = -1, int rec_stride = 0)
 {
+    const int inj = rhs_next != nullptr;
     if (h->kernel == PHC_SEM_SEPARABLE) {
         SemSepArgs a;
         std::memset(&a, 0, sizeof(a));
@@ -1008,6 +1042,16 @@ static phc_status sem_launch(phc_sem *h, int i1, int i2, int inj, float rhs_next
             const int64_t pts = (int64_t)(h->L.nz - 1 - a.krem) * (h->L.ny - 2) * (h->L.nx - 2);
             a.nb_main = nb;
             nb += (int)((pts + FD_TK * h->ty - 1) / (FD_TK * h->ty));
+        }
+        if (rec_step >= 0) {
+            a.rec_off = h->recoff.as<int64_t>();
+            a.rec_out = h->rec.as<float>();
+            a.rec_src = h->trace.as<float>();
+            a.rec_n = h->nrec;
+            a.rec_stride = rec_stride;
+            a.rec_step = rec_step;
+            a.rec_blocks = (h->nrec + FD_TK * h->ty - 1) / (FD_TK * h->ty);
+            nb += a.rec_blocks;
         }
         SemSepFn fn = sem_pick_sep(h->p, h->ty, h->nj, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32));
         if (!fn) return fail(PHC_ERR_INVALID, "no separable kernel for p=%d", h->p);
@@ -1129,7 +1173,6 @@ static phc_status sem_source(phc_sem *h, int src_element, int nsamples, const fl
     const int sx = (int)(sn % h->nx), sz = (int)((sn / h->nx) % h->nz), sy = (int)(sn / ((int64_t)h->nx * h->nz));
     h->src_interior = sx >= 1 && sx < h->nx - 1 && sz >= 1 && sz < h->nz - 1 && sy >= 1 && sy < h->ny - 1;
     h->nsamples = nsamples;
-    h->hrhs.assign(rhs, rhs + nsamples);
     PHC_TRY(h->rhs.alloc(sizeof(float) * std::max(1, nsamples)));
     if (nsamples > 0) PHC_HIP(hipMemcpy(h->rhs.ptr, rhs, sizeof(float) * nsamples, hipMemcpyHostToDevice));
     return PHC_OK;
@@ -1222,7 +1265,6 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
     h->kernel = p->kernel;
     h->dt = p->dt;
     h->nsamples = p->nsamples;
-    h->hrhs.assign(p->rhs, p->rhs + p->nsamples);
     h->model.assign(p->model, p->model + nE);
     h->src_element = p->src_element;
     {
@@ -1352,7 +1394,7 @@ phc_status phc_sem_destroy(phc_sem *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     sem_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->y, &h->dt2m, &h->geo, &h->rhs, &h->trace,
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->y, &h->dt2m, &h->geo, &h->rhs, &h->window, &h->trace,
                       &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1379,7 +1421,7 @@ phc_status phc_sem_compute_one_step(phc_sem *h, int time_sample, int i1, int i2)
     if (time_sample < 0 || time_sample >= h->nsamples)
         return fail(PHC_ERR_INVALID, "time sample %d outside 0..%d", time_sample, h->nsamples - 1);
     PHC_TRY(sem_inject(h, i2, time_sample));
-    return sem_launch(h, i1, i2, 0, 0.f, nullptr, nullptr, nullptr);
+    return sem_launch(h, i1, i2, nullptr, nullptr, nullptr, nullptr);
 }
 
 phc_status phc_sem_compute_one_step_rhs(phc_sem *h, int i1, int i2, int nrhs, const int *rhs_element,
@@ -1406,7 +1448,7 @@ phc_status phc_sem_compute_one_step_rhs(phc_sem *h, int i1, int i2, int nrhs, co
                            sem_off(h, sem_first_node(h, e)), ((h->dt * h->dt) * c) * c, rhs_value[r]);
         PHC_HIP(hipGetLastError());
     }
-    return sem_launch(h, i1, i2, 0, 0.f, nullptr, nullptr, nullptr);
+    return sem_launch(h, i1, i2, nullptr, nullptr, nullptr, nullptr);
 }
 
 phc_status phc_sem_set_source(phc_sem *h, int src_element, int nsamples, const float *rhs)
@@ -1417,32 +1459,39 @@ phc_status phc_sem_set_source(phc_sem *h, int src_element, int nsamples, const f
     return sem_source(h, src_element, nsamples, rhs);
 }
 
-static phc_status sem_enqueue_run(phc_sem *h, int it0, int nsteps, int i1, int i2,
-                                  std::vector<hipEvent_t> *ev)
+// A run's steps on h->stream (sem_begin_run_kernel has filled the window and
+// injected its first sample).  Names no time sample, so that a captured run
+// serves every chunk.  The separable step's launch samples the receivers of
+// the step before; the element kernels' receivers, and the last step's, are
+// sampled by launches of their own.
+static phc_status sem_enqueue_run(phc_sem *h, int nsteps, int i1, int i2, std::vector<hipEvent_t> *ev)
 {
-    PHC_TRY(sem_inject(h, i2, it0));
+    const int64_t src = sem_off(h, h->src_node);
+    const float *win = h->window.as<float>();
+    const bool fused = h->kernel == PHC_SEM_SEPARABLE && h->nrec > 0;
     for (int s = 0; s < nsteps; ++s) {
-        const int it = it0 + s;
-        const bool more = s + 1 < nsteps;
+        const int rs = fused ? s - 1 : -1;
+        hipEvent_t e0 = ev ? (*ev)[2 * s] : nullptr, e1 = ev ? (*ev)[2 * s + 1] : nullptr;
         if (h->src_interior) {
-            PHC_TRY(sem_launch(h, i1, i2, more ? 1 : 0, more ? h->hrhs[it + 1] : 0.f,
-                               h->trace.as<float>() + s, ev ? (*ev)[2 * s] : nullptr,
-                               ev ? (*ev)[2 * s + 1] : nullptr));
+            PHC_TRY(sem_launch(h, i1, i2, s + 1 < nsteps ? win + s + 1 : nullptr, h->trace.as<float>() + s, e0, e1,
+                               rs, nsteps));
         } else {
             // source on a (never updated) boundary node: inject in place each
             // step, as SEMsolver.cpp:39-43 does, and read the node back
-            if (s > 0) PHC_TRY(sem_inject(h, i2, it));
-            PHC_TRY(sem_launch(h, i1, i2, 0, 0.f, nullptr, ev ? (*ev)[2 * s] : nullptr,
-                               ev ? (*ev)[2 * s + 1] : nullptr));
+            if (s > 0) {
+                hipLaunchKernelGGL(sem_inject_kernel, dim3(1), dim3(64), 0, h->stream, h->lev[i2].as<float>(), src,
+                                   h->inj_coef, win, s);
+                PHC_HIP(hipGetLastError());
+            }
+            PHC_TRY(sem_launch(h, i1, i2, nullptr, nullptr, e0, e1, rs, nsteps));
             hipLaunchKernelGGL(sem_copy_point_kernel, dim3(1), dim3(64), 0, h->stream, h->lev[i1].as<float>(),
-                               sem_off(h, h->src_node), h->trace.as<float>() + s);
+                               src, h->trace.as<float>() + s);
             PHC_HIP(hipGetLastError());
         }
-        if (h->nrec > 0) {
+        if (h->nrec > 0 && (!fused || s == nsteps - 1)) {
             hipLaunchKernelGGL(sem_sample_kernel, dim3((h->nrec + 255) / 256), dim3(256), 0, h->stream,
                                h->lev[i1].as<float>(), h->recoff.as<int64_t>(), h->nrec,
-                               h->rec.as<float>(), nsteps, s, sem_off(h, h->src_node),
-                               h->trace.as<float>());
+                               h->rec.as<float>(), nsteps, s, src, h->trace.as<float>());
             PHC_HIP(hipGetLastError());
         }
         std::swap(i1, i2);
@@ -1463,20 +1512,25 @@ phc_status phc_sem_run(phc_sem *h, int it0, int nsteps, int *i1p, int *i2p)
         return fail(PHC_ERR_INVALID, "steps %d..%d outside the %d source samples", it0,
                     it0 + nsteps - 1, h->nsamples);
     PHC_TRY(sem_prepare_sched(h));  // before any capture
-    if (h->trace.bytes < sizeof(float) * nsteps) {
+    if (h->trace.bytes < sizeof(float) * nsteps || h->window.bytes < sizeof(float) * nsteps) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         sem_drop_graph(h);
         PHC_TRY(h->trace.alloc(sizeof(float) * nsteps));
+        PHC_TRY(h->window.alloc(sizeof(float) * nsteps));
     }
     if (h->nrec > 0 && h->rec.bytes < sizeof(float) * (size_t)nsteps * h->nrec) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         sem_drop_graph(h);
         PHC_TRY(h->rec.alloc(sizeof(float) * (size_t)nsteps * h->nrec));
     }
+    hipLaunchKernelGGL(sem_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
+                       h->lev[i2].as<float>(), sem_off(h, h->src_node), h->inj_coef, h->rhs.as<float>(), it0, nsteps,
+                       h->window.as<float>());
+    PHC_HIP(hipGetLastError());
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = sem_enqueue_run(h, it0, nsteps, i1, i2, &ev);
+        phc_status st = sem_enqueue_run(h, nsteps, i1, i2, &ev);
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -1490,26 +1544,8 @@ phc_status phc_sem_run(phc_sem *h, int it0, int nsteps, int *i1p, int *i2p)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        if (!(h->gexec && h->g_it0 == it0 && h->g_n == nsteps && h->g_i1 == i1 && h->g_nrec == h->nrec)) {
-            sem_drop_graph(h);
-            hipGraph_t graph = nullptr;
-            PHC_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-            phc_status st = sem_enqueue_run(h, it0, nsteps, i1, i2, nullptr);
-            hipError_t ce = hipStreamEndCapture(h->stream, &graph);
-            if (st != PHC_OK) {
-                if (graph) (void)hipGraphDestroy(graph);
-                return st;
-            }
-            if (ce != hipSuccess) return fail(PHC_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ce));
-            hipError_t ie = hipGraphInstantiate(&h->gexec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if (ie != hipSuccess) {
-                h->gexec = nullptr;
-                return fail(PHC_ERR_HIP, "graph instantiate failed: %s", hipGetErrorString(ie));
-            }
-            h->g_it0 = it0; h->g_n = nsteps; h->g_i1 = i1; h->g_nrec = h->nrec;
-        }
-        PHC_HIP(hipGraphLaunch(h->gexec, h->stream));
+        PHC_TRY(run_captured(h->stream, h->graph[i1], nsteps, 0, h->nrec,
+                             [&] { return sem_enqueue_run(h, nsteps, i1, i2, nullptr); }));
     }
     h->last_n = nsteps;
     h->last_nrec = h->nrec;
@@ -1589,7 +1625,7 @@ phc_status phc_sem_apply_stiffness(phc_sem *h, const float *p, float *y)
     std::swap(h->lev[1], s1);
     phc_status st = sem_put(h, h->lev[0], p);
     if (st == PHC_OK) st = sem_put(h, h->lev[1], p);
-    if (st == PHC_OK) st = sem_launch(h, 0, 1, 0, 0.f, nullptr, nullptr, nullptr);
+    if (st == PHC_OK) st = sem_launch(h, 0, 1, nullptr, nullptr, nullptr, nullptr);
     std::vector<float> out((size_t)h->nn);
     if (st == PHC_OK) st = sem_get(h, h->lev[0], out.data());
     std::swap(h->lev[0], s0);
@@ -1709,7 +1745,7 @@ extern "C" phc_status phc_sem_autotune(phc_sem *h, int steps_per_trial, const ch
                 for (int rep = 0; rep < 2 && st == PHC_OK; ++rep) {
                     if (hipEventRecord(e0, h->stream) != hipSuccess) st = fail(PHC_ERR_HIP, "event record failed");
                     for (int s = 0; s < steps_per_trial && st == PHC_OK; ++s)
-                        st = sem_launch(h, s & 1, 1 - (s & 1), 0, 0.f, nullptr, nullptr, nullptr);
+                        st = sem_launch(h, s & 1, 1 - (s & 1), nullptr, nullptr, nullptr, nullptr);
                     if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess ||
                                          hipEventSynchronize(e1) != hipSuccess ||
                                          hipEventElapsedTime(&ms, e0, e1) != hipSuccess))

@@ -76,10 +76,27 @@ struct Sem2dArgs {
     int64_t src_off;    // layout offset of the source node
     int inj;
     float inj_coef;     // dt^2 c^2 of the source element (SEMsolver.cpp:41-42)
-    float rhs_next;
+    const float *rhs_next;  // in the run's sample window (device memory)
     float *trace;
     int chunk, nchunks;
+    // receiver sampling of the level this launch reads as current (the
+    // previous step's result) by extra blocks after the nb_main marching ones
+    int nb_main;
+    const int64_t *rec_off;
+    float *rec_out;
+    const float *rec_src;
+    int rec_n, rec_stride, rec_step;
 };
+
+// out[r * stride + step] = level value of receiver r.  The source node
+// already holds the next sample's injection, so a receiver there takes the
+// source trace (the value before injection) instead.
+__device__ __forceinline__ void sem2d_sample_point(const float *p, const int64_t *offs, int r, float *out, int stride,
+                                                   int step, int64_t src_off, const float *src_trace)
+{
+    const int64_t o = offs[r];
+    out[(int64_t)r * stride + step] = (o == src_off) ? src_trace[step] : p[o];
+}
 
 template <int P, typename IT>
 __global__ void __launch_bounds__(64 * S2_WAVES) sem2d_step_kernel(Sem2dArgs a)
@@ -89,6 +106,13 @@ __global__ void __launch_bounds__(64 * S2_WAVES) sem2d_step_kernel(Sem2dArgs a)
     constexpr IT S = sizeof(IT) == 4 ? 4 : 1;
     __shared__ float srow[S2_WAVES][RW];
 
+    if ((int)blockIdx.x >= a.nb_main) {
+        const int r = ((int)blockIdx.x - a.nb_main) * (64 * S2_WAVES) + (int)threadIdx.x;
+        if (r < a.rec_n)
+            sem2d_sample_point(a.pn, a.rec_off, r, a.rec_out, a.rec_stride, a.rec_step, a.src_off, a.rec_src);
+        return;
+    }
+    const float rhs_next = uniform_value(a.rhs_next);
     const Sem2Layout &L = a.L;
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -179,7 +203,7 @@ __global__ void __launch_bounds__(64 * S2_WAVES) sem2d_step_kernel(Sem2dArgs a)
             const IT o = col + zo;
             if ((int64_t)(o / S) == a.src_off) {
                 if (a.trace) *a.trace = val;
-                if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, a.rhs_next));
+                if (a.inj) val = add_nc(val, mul_nc(a.inj_coef, rhs_next));
             }
             sto_nt(a.pnm1, o, val);
         }
@@ -197,16 +221,22 @@ __global__ void sem2d_add_value_kernel(float *p, int64_t off, float coef, float 
     if (threadIdx.x == 0 && blockIdx.x == 0) p[off] = add_nc(p[off], mul_nc(coef, value));
 }
 
-// Receiver samples after a step.  The source node already holds the next
-// sample's injection, so a receiver there takes the source trace (the value
-// before injection) instead.
+// Receivers of a run's last step (the others are sampled by the step launches).
 __global__ void sem2d_sample_kernel(const float *p, const int64_t *offs, int nrec, float *out, int stride,
                                     int step, int64_t src_off, const float *src_trace)
 {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrec) return;
-    const int64_t o = offs[r];
-    out[(int64_t)r * stride + step] = (o == src_off) ? src_trace[step] : p[o];
+    if (r < nrec) sem2d_sample_point(p, offs, r, out, stride, step, src_off, src_trace);
+}
+
+// Start of a run: its source samples into the window, the first one into the
+// current level (SEMsolver.cpp:39-43).
+__global__ void sem2d_begin_run_kernel(float *p, int64_t off, float coef, const float *rhs, int it0, int n,
+                                       float *window)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) window[t] = rhs[it0 + t];
+    if (t == 0) p[off] = add_nc(p[off], mul_nc(coef, rhs[it0]));
 }
 
 using Sem2dFn = void (*)(Sem2dArgs);
@@ -239,7 +269,7 @@ struct phc_sem2d {
     int64_t nn;
     float dt;
     int nsamples;
-    std::vector<float> hrhs, model;
+    std::vector<float> model;
     int src_element, src_node;
     float inj_coef;
     hipStream_t stream = nullptr;
@@ -249,12 +279,11 @@ struct phc_sem2d {
     float cx[S2_MAX_P + 2][S2_W], cz[S2_MAX_P + 2][S2_W];
     std::vector<float> hmass, hsh;  // FP32 lumped mass and boundary term per node
     int chunk = 0;
-    DevBuf trace, rec, recoff;
+    DevBuf trace, window, rec, recoff;  // window: the running chunk's source samples
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
     double last_ms = 0.0;
-    hipGraphExec_t gexec = nullptr;
-    int g_it0 = -1, g_n = -1, g_i1 = -1, g_nrec = -1;
+    RunGraph graph[2];  // of phc_sem2d_run, by i1
 };
 
 static int64_t s2_off(const phc_sem2d *h, int64_t node)
@@ -265,9 +294,7 @@ static int64_t s2_off(const phc_sem2d *h, int64_t node)
 
 static void s2_drop_graph(phc_sem2d *h)
 {
-    if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
-    h->gexec = nullptr;
-    h->g_it0 = h->g_n = h->g_i1 = h->g_nrec = -1;
+    for (RunGraph &g : h->graph) g.drop();
 }
 
 static phc_status s2_put(phc_sem2d *h, DevBuf &dst, const float *host)
@@ -299,8 +326,11 @@ static int s2_default_chunk(const phc_sem2d *h)
     return std::min(c, h->nz);
 }
 
-static phc_status s2_launch(phc_sem2d *h, int i1, int i2, int inj, float rhs_next, float *trace,
-                            hipEvent_t e0, hipEvent_t e1)
+// One step; rhs_next (device memory, may be null): sample injected after it;
+// rec_step >= 0: also samples level i2's receivers into that step of a run of
+// rec_stride steps.
+static phc_status s2_launch(phc_sem2d *h, int i1, int i2, const float *rhs_next, float *trace, hipEvent_t e0,
+                            hipEvent_t e1, int rec_step = -1, int rec_stride = 0)
 {
     Sem2dArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -316,17 +346,27 @@ static phc_status s2_launch(phc_sem2d *h, int i1, int i2, int inj, float rhs_nex
     std::memcpy(a.cx, h->cx, sizeof(a.cx));
     std::memcpy(a.cz, h->cz, sizeof(a.cz));
     a.src_off = s2_off(h, h->src_node);
-    a.inj = inj;
+    a.inj = rhs_next != nullptr;
     a.inj_coef = h->inj_coef;
     a.rhs_next = rhs_next;
     a.trace = trace;
     a.chunk = h->chunk > 0 ? h->chunk : s2_default_chunk(h);
     a.nchunks = (h->nz + a.chunk - 1) / a.chunk;
     const int waves = h->L.tiles_x * a.nchunks;
+    a.nb_main = (waves + S2_WAVES - 1) / S2_WAVES;
+    if (rec_step >= 0) {
+        a.rec_off = h->recoff.as<int64_t>();
+        a.rec_out = h->rec.as<float>();
+        a.rec_src = h->trace.as<float>();
+        a.rec_n = h->nrec;
+        a.rec_stride = rec_stride;
+        a.rec_step = rec_step;
+    }
+    const int nb = a.nb_main + (a.rec_n + 64 * S2_WAVES - 1) / (64 * S2_WAVES);
     Sem2dFn fn = sem2d_pick(h->p, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32));
     if (!fn) return fail(PHC_ERR_INVALID, "no 2D SEM kernel for p=%d", h->p);
     if (e0) PHC_HIP(hipEventRecord(e0, h->stream));
-    hipLaunchKernelGGL(fn, dim3((waves + S2_WAVES - 1) / S2_WAVES), dim3(64 * S2_WAVES), 0, h->stream, a);
+    hipLaunchKernelGGL(fn, dim3(nb), dim3(64 * S2_WAVES), 0, h->stream, a);
     PHC_HIP(hipGetLastError());
     if (e1) PHC_HIP(hipEventRecord(e1, h->stream));
     return PHC_OK;
@@ -347,7 +387,7 @@ phc_status phc_sem2d_destroy(phc_sem2d *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     s2_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->sig, &h->rhs, &h->trace, &h->rec, &h->recoff})
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->sig, &h->rhs, &h->window, &h->trace, &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -390,7 +430,6 @@ phc_status phc_sem2d_create(const phc_sem_params *p, phc_sem2d **out)
     h->nn = nx * nz;
     h->dt = p->dt;
     h->nsamples = p->nsamples;
-    h->hrhs.assign(p->rhs, p->rhs + p->nsamples);
     h->model.assign(p->model, p->model + (size_t)p->ex * p->ez);
     h->src_element = p->src_element;
     {
@@ -504,7 +543,7 @@ phc_status phc_sem2d_compute_one_step(phc_sem2d *h, int time_sample, int i1, int
     if (time_sample < 0 || time_sample >= h->nsamples)
         return fail(PHC_ERR_INVALID, "time sample %d outside 0..%d", time_sample, h->nsamples - 1);
     PHC_TRY(s2_inject(h, i2, time_sample));
-    return s2_launch(h, i1, i2, 0, 0.f, nullptr, nullptr, nullptr);
+    return s2_launch(h, i1, i2, nullptr, nullptr, nullptr, nullptr);
 }
 
 phc_status phc_sem2d_compute_one_step_rhs(phc_sem2d *h, int i1, int i2, int nrhs, const int *rhs_element,
@@ -531,7 +570,7 @@ phc_status phc_sem2d_compute_one_step_rhs(phc_sem2d *h, int i1, int i2, int nrhs
                            s2_off(h, node), ((h->dt * h->dt) * c) * c, rhs_value[r]);
         PHC_HIP(hipGetLastError());
     }
-    return s2_launch(h, i1, i2, 0, 0.f, nullptr, nullptr, nullptr);
+    return s2_launch(h, i1, i2, nullptr, nullptr, nullptr, nullptr);
 }
 
 phc_status phc_sem2d_set_source(phc_sem2d *h, int src_element, int nsamples, const float *rhs)
@@ -547,27 +586,29 @@ phc_status phc_sem2d_set_source(phc_sem2d *h, int src_element, int nsamples, con
     const float c = h->model[src_element];
     h->inj_coef = ((h->dt * h->dt) * c) * c;
     h->nsamples = nsamples;
-    h->hrhs.assign(rhs, rhs + nsamples);
     PHC_TRY(h->rhs.alloc(sizeof(float) * std::max(1, nsamples)));
     if (nsamples > 0) PHC_HIP(hipMemcpy(h->rhs.ptr, rhs, sizeof(float) * nsamples, hipMemcpyHostToDevice));
     return PHC_OK;
 }
 
-static phc_status s2_enqueue_run(phc_sem2d *h, int it0, int nsteps, int i1, int i2, std::vector<hipEvent_t> *ev)
+// A run's steps on h->stream (sem2d_begin_run_kernel has filled the window and
+// injected its first sample), each step's launch sampling the receivers of
+// the one before.  Names no time sample, so that a captured run serves every
+// chunk.
+static phc_status s2_enqueue_run(phc_sem2d *h, int nsteps, int i1, int i2, std::vector<hipEvent_t> *ev)
 {
-    PHC_TRY(s2_inject(h, i2, it0));
+    const float *win = h->window.as<float>();
     for (int s = 0; s < nsteps; ++s) {
-        const int it = it0 + s;
-        const bool more = s + 1 < nsteps;
-        PHC_TRY(s2_launch(h, i1, i2, more ? 1 : 0, more ? h->hrhs[it + 1] : 0.f, h->trace.as<float>() + s,
-                          ev ? (*ev)[2 * s] : nullptr, ev ? (*ev)[2 * s + 1] : nullptr));
-        if (h->nrec > 0) {
-            hipLaunchKernelGGL(sem2d_sample_kernel, dim3((h->nrec + 255) / 256), dim3(256), 0, h->stream,
-                               h->lev[i1].as<float>(), h->recoff.as<int64_t>(), h->nrec, h->rec.as<float>(),
-                               nsteps, s, s2_off(h, h->src_node), h->trace.as<float>());
-            PHC_HIP(hipGetLastError());
-        }
+        PHC_TRY(s2_launch(h, i1, i2, s + 1 < nsteps ? win + s + 1 : nullptr, h->trace.as<float>() + s,
+                          ev ? (*ev)[2 * s] : nullptr, ev ? (*ev)[2 * s + 1] : nullptr, h->nrec > 0 ? s - 1 : -1,
+                          nsteps));
         std::swap(i1, i2);
+    }
+    if (h->nrec > 0) {
+        hipLaunchKernelGGL(sem2d_sample_kernel, dim3((h->nrec + 255) / 256), dim3(256), 0, h->stream,
+                           h->lev[i2].as<float>(), h->recoff.as<int64_t>(), h->nrec, h->rec.as<float>(), nsteps,
+                           nsteps - 1, s2_off(h, h->src_node), h->trace.as<float>());
+        PHC_HIP(hipGetLastError());
     }
     return PHC_OK;
 }
@@ -584,20 +625,25 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
     if (it0 < 0 || it0 + nsteps > h->nsamples)
         return fail(PHC_ERR_INVALID, "steps %d..%d outside the %d source samples", it0, it0 + nsteps - 1,
                     h->nsamples);
-    if (h->trace.bytes < sizeof(float) * nsteps) {
+    if (h->trace.bytes < sizeof(float) * nsteps || h->window.bytes < sizeof(float) * nsteps) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         s2_drop_graph(h);
         PHC_TRY(h->trace.alloc(sizeof(float) * nsteps));
+        PHC_TRY(h->window.alloc(sizeof(float) * nsteps));
     }
     if (h->nrec > 0 && h->rec.bytes < sizeof(float) * (size_t)nsteps * h->nrec) {
         PHC_HIP(hipStreamSynchronize(h->stream));
         s2_drop_graph(h);
         PHC_TRY(h->rec.alloc(sizeof(float) * (size_t)nsteps * h->nrec));
     }
+    hipLaunchKernelGGL(sem2d_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
+                       h->lev[i2].as<float>(), s2_off(h, h->src_node), h->inj_coef, h->rhs.as<float>(), it0, nsteps,
+                       h->window.as<float>());
+    PHC_HIP(hipGetLastError());
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = s2_enqueue_run(h, it0, nsteps, i1, i2, &ev);
+        phc_status st = s2_enqueue_run(h, nsteps, i1, i2, &ev);
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -611,26 +657,8 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        if (!(h->gexec && h->g_it0 == it0 && h->g_n == nsteps && h->g_i1 == i1 && h->g_nrec == h->nrec)) {
-            s2_drop_graph(h);
-            hipGraph_t graph = nullptr;
-            PHC_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-            phc_status st = s2_enqueue_run(h, it0, nsteps, i1, i2, nullptr);
-            hipError_t ce = hipStreamEndCapture(h->stream, &graph);
-            if (st != PHC_OK) {
-                if (graph) (void)hipGraphDestroy(graph);
-                return st;
-            }
-            if (ce != hipSuccess) return fail(PHC_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ce));
-            hipError_t ie = hipGraphInstantiate(&h->gexec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if (ie != hipSuccess) {
-                h->gexec = nullptr;
-                return fail(PHC_ERR_HIP, "graph instantiate failed: %s", hipGetErrorString(ie));
-            }
-            h->g_it0 = it0; h->g_n = nsteps; h->g_i1 = i1; h->g_nrec = h->nrec;
-        }
-        PHC_HIP(hipGraphLaunch(h->gexec, h->stream));
+        PHC_TRY(run_captured(h->stream, h->graph[i1], nsteps, 0, h->nrec,
+                             [&] { return s2_enqueue_run(h, nsteps, i1, i2, nullptr); }));
     }
     h->last_n = nsteps;
     h->last_nrec = h->nrec;
@@ -757,7 +785,7 @@ phc_status phc_sem2d_autotune(phc_sem2d *h, int steps_per_trial, int *chunk)
         for (int rep = 0; rep < 2 && st == PHC_OK; ++rep) {
             if (hipEventRecord(e0, h->stream) != hipSuccess) st = fail(PHC_ERR_HIP, "event record failed");
             for (int s = 0; s < steps_per_trial && st == PHC_OK; ++s)
-                st = s2_launch(h, s & 1, 1 - (s & 1), 0, 0.f, nullptr, nullptr, nullptr);
+                st = s2_launch(h, s & 1, 1 - (s & 1), nullptr, nullptr, nullptr, nullptr);
             if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                                  hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
                 st = fail(PHC_ERR_HIP, "trial timing failed");
