@@ -74,7 +74,8 @@ typedef struct {
     float sponge_alpha;
     float init_value;  /* initial value of both levels and of the halo (1e-6) */
     int arith;         /* PHC_FD_ARITH_* */
-    /* kernel tiling; 0 selects the built-in default for the radius */
+    /* kernel tiling; all 0: chosen from the grid (radius 4: the shapes with 4
+     * rows per wavefront, four points per lane) */
     int tile_j;        /* output rows per block along j (block_waves x 1, 2 or 4) */
     int block_waves;   /* wavefronts per block: 4, 8 or 16 */
     int chunk_i;       /* planes per block along the marching axis i; -m
@@ -85,8 +86,9 @@ typedef struct {
     int index64;       /* 1: force 64-bit element offsets (default: 32-bit when
                         * every array is below 4 GiB) */
     int k_remainder;   /* a last, partial 64-point tile along k: 0 (default)
-                        * updated point by point when it holds at most 32
-                        * points, as a whole tile otherwise; likewise a last
+                        * a tile with 4 rows per wavefront; otherwise updated
+                        * point by point when it holds at most 32
+                        * points, as a whole tile else; likewise a last
                         * tile along j holding at most a quarter of tile_j
                         * rows; 1 always point by point; -1 always as a tile.
                         * Same values either way. */

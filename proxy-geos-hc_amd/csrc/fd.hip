@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "fd_kernels.hpp"
+#include "fd_quad.hpp"
 #include "fd_tile.hpp"
 #include "lb.hpp"
 #include "march.hpp"
@@ -113,6 +114,29 @@ fd_step_pml_kernel(FdStepArgs a)
     fd_tile<R, TY, NJ, ARITH, IT, true>(a, a, rhs_next, kt, jt, i0, i1, tile);
 }
 
+// The radius-4 step with 4 rows per wavefront and 4 points per lane
+// (fd_quad.hpp), with or without the PML.
+template <int TY, int ARITH, typename IT, bool PML, bool NT>
+__global__ void __launch_bounds__(FD_TK *TY) __attribute__((amdgpu_waves_per_eu(3)))
+fd_quad_kernel(FdStepArgs a)
+{
+    using SH = FdQuadShape<TY>;
+    __shared__ fd_f4 tile[2][SH::LH][SH::LQ];
+    if ((int)blockIdx.x >= (int)gridDim.x - a.rec_blocks) {
+        fd_sample_prev(a);
+        return;
+    }
+    const float rhs_next = uniform_value(a.rhs_next);
+    if (a.nb_main && (int)blockIdx.x >= a.nb_main) {
+        fd_rem_points<4, ARITH, IT, PML>(a, a, rhs_next, (int64_t)(blockIdx.x - a.nb_main) * (FD_TK * TY));
+        return;
+    }
+    int kt, jt, i0, i1;
+    fd_block_range(a, kt, jt, i0, i1);
+    if (i0 >= i1) return;  // padding of a shorter XCD list (whole block)
+    fd_quad<TY, ARITH, IT, PML, NT>(a, a, rhs_next, kt, jt, i0, i1, tile);
+}
+
 // addRHS (FDTDkernels.hpp:121-128): one point.
 __global__ void fd_add_rhs_kernel(float *p, const float *vp, int64_t off, const float *rhs, int it)
 {
@@ -187,15 +211,35 @@ static FdKernelFn pick_arith(int arith, bool idx32, bool pml)
                  : fd_step_kernel<R, TY, NJ, PHC_FD_ARITH_FP32, int64_t>;
 }
 
-// Block shapes: TY wavefronts per block, NJ rows per thread (tile_j = TY*NJ).
+template <int TY, int ARITH, bool PML>
+static FdKernelFn pick_quad_access(bool idx32, bool nt)
+{
+    // arrays of 4 GiB and more never fit the cache
+    if (!idx32) return fd_quad_kernel<TY, ARITH, int64_t, PML, true>;
+    return nt ? fd_quad_kernel<TY, ARITH, uint32_t, PML, true> : fd_quad_kernel<TY, ARITH, uint32_t, PML, false>;
+}
+
+template <int TY>
+static FdKernelFn pick_quad(int arith, bool idx32, bool pml, bool nt)
+{
+    if (arith == PHC_FD_ARITH_REF)
+        return pml ? pick_quad_access<TY, PHC_FD_ARITH_REF, true>(idx32, nt)
+                   : pick_quad_access<TY, PHC_FD_ARITH_REF, false>(idx32, nt);
+    return pml ? pick_quad_access<TY, PHC_FD_ARITH_FP32, true>(idx32, nt)
+               : pick_quad_access<TY, PHC_FD_ARITH_FP32, false>(idx32, nt);
+}
+
+// Block shapes: TY wavefronts per block, NJ rows per wavefront (tile_j =
+// TY*NJ): NJ = 1 or 2 rows per thread, 4: the four-points-per-lane tile.
 // Radius 4 (the 8th-order operator and order-4 SEM) gets the full set; the
 // other radii one shape.
 template <int R>
-static FdKernelFn pick_shape(int ty, int nj, int arith, bool idx32, bool pml)
+static FdKernelFn pick_shape(int ty, int nj, int arith, bool idx32, bool pml, bool nt)
 {
     if (ty == 4 && nj == 2) return pick_arith<R, 4, 2>(arith, idx32, pml);
     if constexpr (R == 4) {
-        if (ty == 4 && nj == 4) return pick_arith<R, 4, 4>(arith, idx32, pml);
+        if (ty == 4 && nj == 4) return pick_quad<4>(arith, idx32, pml, nt);
+        if (ty == 8 && nj == 4) return pick_quad<8>(arith, idx32, pml, nt);
         if (ty == 8 && nj == 1) return pick_arith<R, 8, 1>(arith, idx32, pml);
         if (ty == 8 && nj == 2) return pick_arith<R, 8, 2>(arith, idx32, pml);
         if (ty == 16 && nj == 1) return pick_arith<R, 16, 1>(arith, idx32, pml);
@@ -205,16 +249,18 @@ static FdKernelFn pick_shape(int ty, int nj, int arith, bool idx32, bool pml)
 }
 
 // Kernel for half width R and block shape, arithmetic mode, 32-bit offsets
-// when every array is < 4 GiB, with or without the PML slabs.
-FdKernelFn fd_pick_kernel(int R, int ty, int nj, int arith, bool idx32, bool pml)
+// when every array is < 4 GiB, with or without the PML slabs; nt: non-temporal
+// accesses to the streamed arrays (the four-points-per-lane shapes; the others
+// always have them).
+FdKernelFn fd_pick_kernel(int R, int ty, int nj, int arith, bool idx32, bool pml, bool nt = true)
 {
     switch (R) {
-    case 1: return pick_shape<1>(ty, nj, arith, idx32, pml);
-    case 2: return pick_shape<2>(ty, nj, arith, idx32, pml);
-    case 3: return pick_shape<3>(ty, nj, arith, idx32, pml);
-    case 4: return pick_shape<4>(ty, nj, arith, idx32, pml);
-    case 5: return pick_shape<5>(ty, nj, arith, idx32, pml);
-    case 6: return pick_shape<6>(ty, nj, arith, idx32, pml);
+    case 1: return pick_shape<1>(ty, nj, arith, idx32, pml, nt);
+    case 2: return pick_shape<2>(ty, nj, arith, idx32, pml, nt);
+    case 3: return pick_shape<3>(ty, nj, arith, idx32, pml, nt);
+    case 4: return pick_shape<4>(ty, nj, arith, idx32, pml, nt);
+    case 5: return pick_shape<5>(ty, nj, arith, idx32, pml, nt);
+    case 6: return pick_shape<6>(ty, nj, arith, idx32, pml, nt);
     default: return nullptr;
     }
 }
@@ -442,10 +488,29 @@ static void fd_drop_graph(phc_fd *h)
     for (RunGraph &g : h->graph) g.drop();
 }
 
+// Whether a step's three arrays exceed what the 256 MB memory-side cache
+// keeps between steps: below, cached accesses to pnm1 and vp find them there
+// (150^3: 18.3 -> 16.7 us per step, 264^3, 263 MB: 62.5 -> 60.9); above, they
+// push out the pn rows that neighbouring tiles share (304^3, 411 MB: 82 ->
+// 100 us; measured on the one-point tile).
+static bool fd_streams_past_cache(const FdLayout &L) { return 12 * L.total > (int64_t)300e6; }
+
 static FdKernelFn fd_handle_kernel(const phc_fd *h)
 {
     return fd_pick_kernel(h->R, h->ty, h->nj, h->arith, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32),
-                          h->pml_on != 0);
+                          h->pml_on != 0, fd_streams_past_cache(h->L));
+}
+
+// Blocks of a shape resident per CU (the quad kernels hold 3 waves per SIMD:
+// their amdgpu_waves_per_eu, and 23 KB of LDS at most).
+static int fd_resident(FdKernelFn fn, int ty, int nj)
+{
+    if (nj == 4) return 12 / ty;
+    int per_cu = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(fn), FD_TK * ty, 0) !=
+            hipSuccess || per_cu < 1)
+        per_cu = 1;
+    return per_cu;
 }
 
 // The per-XCD schedule (chunk_i = -m) for the tiles `a` plans: ranges of
@@ -461,12 +526,8 @@ static phc_status fd_prepare_sched(phc_fd *h, const FdStepArgs &a)
     if (h->sched_key == key && h->sched.ptr) return PHC_OK;
     FdKernelFn fn = fd_handle_kernel(h);
     if (!fn) return fail(PHC_ERR_INVALID, "no kernel for R=%d block_waves=%d rows/thread=%d", h->R, h->ty, h->nj);
-    int per_cu = 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(fn), FD_TK * h->ty, 0) !=
-            hipSuccess || per_cu < 1)
-        per_cu = 1;
     std::vector<int4> tab;
-    build_xcd_schedule(a.ihi - a.ilo, a.ilo, ncol, std::max(h->cus / 8, 1) * per_cu, -h->chunk_i, 1, tab);
+    build_xcd_schedule(a.ihi - a.ilo, a.ilo, ncol, std::max(h->cus / 8, 1) * fd_resident(fn, h->ty, h->nj), -h->chunk_i, 1, tab);
     PHC_HIP(hipStreamSynchronize(h->stream));  // queued launches may still read the old table
     fd_drop_graph(h);
     PHC_TRY(h->sched.alloc(sizeof(int4) * tab.size()));
@@ -489,6 +550,40 @@ static phc_status fd_plan_launch(phc_fd *h, FdStepArgs &a, int *nb)
         *nb = h->sched_nb + slab;
     }
     return PHC_OK;
+}
+
+// Block shape and per-XCD split where the caller gives none: the pair whose
+// busiest CU has the least work (xcd_schedule_cost, where the figures are).
+// Radius 4 chooses between the four-points-per-lane shapes, 16 or 32 rows;
+// the one-point shapes were slower at every size (best of all shapes and
+// chunks at 96^3, 150^3, 203 x 178 x 261, 264^3, 336 x 300 x 290, 401^3,
+// 480 x 380 x 480, 512^3: 9.1, 17.1, 38.1, 62.9, 90.3, 204, 274, 358 us
+// against 7.5, 14.3, 29.2, 58.9, 88.7, 198, 258, 347).  A partial last k tile
+// stays a tile there (point by point it cost 10-30% more at 96^3 to 264^3).
+static void fd_default_shape(phc_fd *h)
+{
+    static const int quad[][2] = {{8, 4}, {4, 4}}, other[][2] = {{4, 2}};
+    const auto *shapes = h->R == 4 ? quad : other;
+    const int n = h->R == 4 ? 2 : 1;
+    double best = -1.0;
+    for (int s = 0; s < n; ++s) {
+        const int ty = shapes[s][0], nj = shapes[s][1], TJ = ty * nj;
+        FdKernelFn fn = fd_pick_kernel(h->R, ty, nj, h->arith, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32),
+                                       false, fd_streams_past_cache(h->L));
+        const int ncol = ((h->nz + FD_TK - 1) / FD_TK) * ((h->ny + TJ - 1) / TJ);
+        const int cux = std::max(h->cus / 8, 1), slots = cux * fd_resident(fn, ty, nj);
+        std::vector<int4> tab;
+        for (int m = 1; m <= 4; ++m) {
+            build_xcd_schedule(h->nx, 0, ncol, slots, m, 1, tab);
+            const double c = xcd_schedule_cost(tab, cux, TJ, 0.35 * 2 * h->R, 2 * h->R);
+            if (best < 0.0 || c < best) {
+                best = c;
+                h->ty = ty;
+                h->nj = nj;
+                h->chunk_i = -m;
+            }
+        }
+    }
 }
 
 static phc_status fd_launch_step(phc_fd *h, FdStepArgs a, bool damp)
@@ -568,8 +663,6 @@ phc_status phc_fd_create(const phc_fd_params *p, phc_fd **out)
     for (int l = 0; l <= p->lz; ++l) h->cz[l] = p->coefz[l];
     h->coef0 = p->coef0;
     h->nsamples = p->nsamples;
-    // default shape: the fastest measured at 512^3 for radius 4 (16 waves,
-    // 16 rows, whole i-extent per block); other radii have one shape
     const int dty = (h->R == 4) ? 16 : 4, dtj = (h->R == 4) ? 16 : 8;
     h->ty = p->block_waves ? p->block_waves : dty;
     h->nj = (p->tile_j ? p->tile_j : (p->block_waves ? 2 * h->ty : dtj)) / h->ty;
@@ -587,6 +680,8 @@ phc_status phc_fd_create(const phc_fd_params *p, phc_fd **out)
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
             h->cus = cus;
     }
+    if (!p->block_waves && !p->tile_j && !p->chunk_i) fd_default_shape(h);
+    if (h->nj == 4 && h->krem_mode == 0) h->krem_eff = -1;
     const size_t bytes = sizeof(float) * (size_t)h->L.total;
     if ((st = h->lev[0].alloc(bytes)) || (st = h->lev[1].alloc(bytes)) || (st = h->vp.alloc(bytes)))
         return bail(st);
@@ -1106,7 +1201,7 @@ extern "C" phc_status phc_fd_autotune(phc_fd *h, int steps_per_trial, const char
         hipEvent_t e0, e1;
         PHC_HIP(hipEventCreate(&e0));
         PHC_HIP(hipEventCreate(&e1));
-        const int shapes[][2] = {{4, 8}, {4, 16}, {8, 8}, {8, 16}, {16, 16}, {16, 32}};
+        const int shapes[][2] = {{4, 8}, {4, 16}, {8, 8}, {8, 16}, {8, 32}, {16, 16}, {16, 32}};
         const int chunks[] = {64, 128, 256, 512, 1024, -1, -2, -3, -4};
         double best = 1e30;
         int bty = h->ty, bnj = h->nj, bci = h->chunk_i, bku = h->krem_eff;

@@ -53,4 +53,30 @@ inline void build_xcd_schedule(int planes, int plane0, int ncol, int slots_per_x
         for (size_t l = 0; l < lists[x].size(); ++l) tab[8 * l + x] = lists[x][l];
 }
 
+// Work of the busiest CU under a schedule table, in rows x planes: an XCD's
+// entries go in order to its least loaded CU; an entry of n planes costs
+// (n + lead) x (rows + halo).  lead: planes' worth of a march's first loads
+// (2R + 1 planes of ring and the descriptor reads, with no stencil to hide
+// them); halo: rows' worth of a tile's 2R halo rows, which come from L2.
+// Blocks that share a CU share its throughput, so the sum is what counts, not
+// the number of rounds.  Used to choose a block shape and split: among the
+// tables of one grid the measured step follows it (FD, MI355X: 304^3 (4 waves
+// x 16 rows, split 1) 2594 -> 81.8 us against (8 x 32, 2) 2923 -> 86.9; 401^3
+// (8 x 32, 2) 5846 -> 198, (4 x 16, 2) 6147 -> 213, (8 x 32, 1) 6160 -> 208;
+// 480 x 380 x 480 (8 x 32, 2) 6820 -> 258, (8 x 32, 1) 7099 -> 267; 512^3
+// (8 x 32, 3) 9187 -> 347, (2) 9466 -> 370, (1) 10022 -> 378).
+inline double xcd_schedule_cost(const std::vector<int4> &tab, int cus_per_xcd, double rows, double halo, double lead)
+{
+    double worst = 0.0;
+    std::vector<double> load(std::max(cus_per_xcd, 1));
+    for (int x = 0; x < 8; ++x) {
+        std::fill(load.begin(), load.end(), 0.0);
+        for (size_t b = x; b < tab.size(); b += 8)
+            if (tab[b].y < tab[b].z)
+                *std::min_element(load.begin(), load.end()) += (tab[b].z - tab[b].y + lead) * (rows + halo);
+        worst = std::max(worst, *std::max_element(load.begin(), load.end()));
+    }
+    return worst;
+}
+
 } // namespace phc
