@@ -225,7 +225,7 @@ typedef struct {
     int src_element;       /* element holding the source (SEMproxy.cpp:101-106) */
     int kernel;            /* PHC_SEM_* */
     int weights_ref;       /* 1: the reference's 8-decimal GLL weights; 0: exact */
-    int tile_j, block_waves, chunk_i; /* separable kernel tiling (0: default); chunk_i = -m,
+    int tile_j, block_waves, chunk_i; /* separable kernel tiling (all 0: default); chunk_i = -m,
                                          m = 1..4: per-XCD schedule of 8 >> (m-1) plane
                                          ranges x 2^(m-1) column bands */
     int index64;           /* 1: 64-bit offsets in the separable and 2D kernels even

@@ -1341,6 +1341,18 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
         h->ty = p->block_waves ? p->block_waves : 16;
         h->nj = p->tile_j ? p->tile_j / h->ty : 1;
         h->chunk_i = p->chunk_i ? p->chunk_i : h->ny;
+        // where the caller gives no shape: 8 waves x 1 row on the per-XCD
+        // schedule of 4 plane ranges x 2 column bands.  One whole-axis march
+        // per 16-row column (a caller's shape without a chunk) left most CUs
+        // idle: 14 blocks at 101^3 order 2.  Best shape and chunk of each
+        // mesh / this default / before, us per step: 101^3 order 2
+        // 7.8 / 8.1 / 53.5, 321^3 order 4 88 / 88 / 201, 186 x 111 x 146
+        // order 5 16.6 / 17.6 / 78.8, 271 x 301 x 241 order 3 62.5 / 65.6 /
+        // 155, 130 x 142 x 116 order 1 12.4 / 14.2 / 66
+        if (!p->block_waves && !p->tile_j && !p->chunk_i) {
+            h->ty = 8;
+            h->chunk_i = -2;
+        }
         h->index64 = p->index64 ? 1 : 0;
         h->krem_mode = p->k_remainder;
         if (h->krem_mode < -1 || h->krem_mode > 1)

@@ -278,7 +278,7 @@ struct phc_sem2d {
     int index64 = 0;               // 64-bit offsets even for arrays < 4 GiB
     float cx[S2_MAX_P + 2][S2_W], cz[S2_MAX_P + 2][S2_W];
     std::vector<float> hmass, hsh;  // FP32 lumped mass and boundary term per node
-    int chunk = 0;
+    int chunk = 0, cus = 256;
     DevBuf trace, window, rec, recoff;  // window: the running chunk's source samples
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
@@ -320,10 +320,14 @@ static phc_status s2_get(phc_sem2d *h, const DevBuf &src, float *host)
 
 static int s2_default_chunk(const phc_sem2d *h)
 {
-    // enough waves to fill the chip (about 4 per SIMD), chunks of at least 8 rows
-    const int64_t want = 4096;
-    int c = (int)std::max<int64_t>(8, (int64_t)h->L.tiles_x * h->nz / want);
-    return std::min(c, h->nz);
+    // with x rows per wavefront slot, short chunks re-read the 2P rows that
+    // prime the ring and long ones leave slots idle at the end, so the best
+    // length grows with sqrt(x); 2.5 fits the best measured (x = 0.1, 2.9,
+    // 4.4, 9.8, 12.5, 31: 1, 4, 6, 12, 8, 8 rows; past 16 rows the step at
+    // 8001^2, x = 123, no longer gains).  Before, at least 8 rows: 7.2 us per
+    // step on the 196^2 mesh against 3.3, 67 against 52 on 4001^2.
+    const double x = (double)h->L.tiles_x * h->nz / (h->cus * 32.0);
+    return std::clamp((int)std::lround(2.5 * std::sqrt(x)), 1, std::min(16, h->nz));
 }
 
 // One step; rhs_next (device memory, may be null): sample injected after it;
@@ -520,6 +524,12 @@ phc_status phc_sem2d_create(const phc_sem_params *p, phc_sem2d **out)
     rows(ax, h->cx);
     rows(az, h->cz);
     h->chunk = p->chunk_i > 0 ? std::min(p->chunk_i, h->nz) : 0;
+    {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+            h->cus = cus;
+    }
     h->index64 = p->index64 ? 1 : 0;
     *out = h;
     return PHC_OK;
