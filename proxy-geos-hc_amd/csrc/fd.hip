@@ -30,6 +30,7 @@
 #include "lb.hpp"
 #include "march.hpp"
 #include "phc_common.hpp"
+#include "readback.hpp"
 #include "xcd_sched.hpp"
 
 namespace phc {
@@ -295,8 +296,8 @@ struct phc_fd {
     double coef0;
     int nsamples;
     FdLayout L;
-    DevBuf lev[2], vp, fx, fy, fz, rhs, window, trace, rec, recoff;
-    std::vector<float> hfx, hfy, hfz, hvp;
+    DevBuf lev[2], vp, fx, fy, fz, rhs, window, trace, rec, recoff, readback;
+    std::vector<float> hfx, hfy, hfz;
     int pending[2] = {0, 0};
     hipStream_t stream = nullptr;
     int ty = 4, nj = 2, chunk_i = 0, index64 = 0;
@@ -363,18 +364,6 @@ static phc_status fd_validate(const phc_fd_params *p)
         if (!(p->vp[n] >= 0.f) || !std::isfinite(p->vp[n]))
             return fail(PHC_ERR_INVALID, "vp^2 dt^2 at %lld is negative or not finite",
                         (long long)n);
-    return PHC_OK;
-}
-
-static phc_status fd_upload_interior(phc_fd *h, const float *host_idx3, float *dev)
-{
-    // host array in IDX3 order (k fastest, no halo) -> device layout
-    std::vector<float> buf((size_t)h->L.total, 0.f);
-    for (int i = 0; i < h->nx; ++i)
-        for (int j = 0; j < h->ny; ++j)
-            std::memcpy(&buf[(size_t)fd_off(h->L, i, j, 0)],
-                        host_idx3 + ((int64_t)i * h->ny + j) * h->nz, sizeof(float) * h->nz);
-    PHC_HIP(hipMemcpy(dev, buf.data(), sizeof(float) * h->L.total, hipMemcpyHostToDevice));
     return PHC_OK;
 }
 
@@ -686,14 +675,11 @@ phc_status phc_fd_create(const phc_fd_params *p, phc_fd **out)
     if ((st = h->lev[0].alloc(bytes)) || (st = h->lev[1].alloc(bytes)) || (st = h->vp.alloc(bytes)))
         return bail(st);
     // both levels (and their halo and padding) start at init_value
-    {
-        std::vector<float> init((size_t)h->L.total, p->init_value);
-        if (hipMemcpy(h->lev[0].ptr, init.data(), bytes, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(h->lev[1].ptr, init.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
-            return bail(fail(PHC_ERR_HIP, "initial upload failed"));
-    }
-    if ((st = fd_upload_interior(h, p->vp, h->vp.as<float>()))) return bail(st);
-    h->hvp.assign(p->vp, p->vp + (size_t)h->nx * h->ny * h->nz);
+    if ((st = fill_field(h->stream, h->lev[0].as<float>(), h->L.total, p->init_value)) ||
+        (st = fill_field(h->stream, h->lev[1].as<float>(), h->L.total, p->init_value)) ||
+        (st = fill_field(h->stream, h->vp.as<float>(), h->L.total, 0.f)) ||
+        (st = write_field(h->stream, h->readback, h->vp.as<float>(), h->L, 0, 0, 0, p->vp)))
+        return bail(st);
     fd_axis_damping(h->nx, h->sw, h->alpha, h->hfx);
     fd_axis_damping(h->ny, h->sw, h->alpha, h->hfy);
     fd_axis_damping(h->nz, h->sw, h->alpha, h->hfz);
@@ -718,7 +704,7 @@ phc_status phc_fd_destroy(phc_fd *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     fd_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->vp, &h->fx, &h->fy, &h->fz, &h->rhs, &h->window, &h->trace,
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->vp, &h->fx, &h->fy, &h->fz, &h->rhs, &h->window, &h->readback, &h->trace,
                       &h->rec, &h->recoff, &h->lb_w, &h->lb_corr, &h->lb_kvcs, &h->lb_kslab, &h->pml_ex,
                       &h->pml_ey, &h->pml_ez, &h->pml_phi})
         b->release();
@@ -930,42 +916,34 @@ phc_status phc_fd_get_traces(phc_fd *h, float *src, float *rec)
     return PHC_OK;
 }
 
+// The sponge product a level owes (deferred applySponge).
+static FieldDamping fd_owed(const phc_fd *h, int level)
+{
+    FieldDamping d;
+    if (h->pending[level] && h->sw > 0) {
+        d.sw = h->sw;
+        d.fx = h->fx.as<float>();
+        d.fy = h->fy.as<float>();
+        d.fz = h->fz.as<float>();
+    }
+    return d;
+}
+
 phc_status phc_fd_get_field(phc_fd *h, int level, float *host)
 {
     if (!h || !host) return fail(PHC_ERR_INVALID, "handle or host buffer is NULL");
     if (level < 0 || level > 1) return fail(PHC_ERR_INVALID, "level %d is not 0 or 1", level);
-    PHC_HIP(hipStreamSynchronize(h->stream));
-    std::vector<float> buf((size_t)h->L.total);
-    PHC_HIP(hipMemcpy(buf.data(), h->lev[level].ptr, sizeof(float) * h->L.total, hipMemcpyDeviceToHost));
     // IDX3_l order with the reference's per-axis halos (FDTDmacros.hpp:14)
-    const int LX = h->lh[0], LY = h->lh[1], LZ = h->lh[2];
-    const int NYe = h->ny + 2 * LY, NZe = h->nz + 2 * LZ;
-    for (int i = -LX; i < h->nx + LX; ++i)
-        for (int j = -LY; j < h->ny + LY; ++j) {
-            float *dst = host + ((int64_t)(i + LX) * NYe + (j + LY)) * NZe;
-            const float *srcp = &buf[(size_t)fd_off(h->L, i, j, -LZ)];
-            std::memcpy(dst, srcp, sizeof(float) * NZe);
-            const bool row_in = i >= 0 && i < h->nx && j >= 0 && j < h->ny;
-            if (h->pending[level] && row_in)
-                for (int k = 0; k < h->nz; ++k) dst[k + LZ] = dst[k + LZ] * fd_sponge_at(h, i, j, k);
-        }
-    return PHC_OK;
+    const float *const f[3] = {h->hfx.data(), h->hfy.data(), h->hfz.data()};
+    return read_field(h->stream, h->readback, h->lev[level].as<float>(), h->L, h->lh[0], h->lh[1], h->lh[2],
+                      fd_owed(h, level), f, host);
 }
 
 phc_status phc_fd_set_field(phc_fd *h, int level, const float *host)
 {
     if (!h || !host) return fail(PHC_ERR_INVALID, "handle or host buffer is NULL");
     if (level < 0 || level > 1) return fail(PHC_ERR_INVALID, "level %d is not 0 or 1", level);
-    PHC_HIP(hipStreamSynchronize(h->stream));
-    std::vector<float> buf((size_t)h->L.total);
-    PHC_HIP(hipMemcpy(buf.data(), h->lev[level].ptr, sizeof(float) * h->L.total, hipMemcpyDeviceToHost));
-    const int LX = h->lh[0], LY = h->lh[1], LZ = h->lh[2];
-    const int NYe = h->ny + 2 * LY, NZe = h->nz + 2 * LZ;
-    for (int i = -LX; i < h->nx + LX; ++i)
-        for (int j = -LY; j < h->ny + LY; ++j)
-            std::memcpy(&buf[(size_t)fd_off(h->L, i, j, -LZ)],
-                        host + ((int64_t)(i + LX) * NYe + (j + LY)) * NZe, sizeof(float) * NZe);
-    PHC_HIP(hipMemcpy(h->lev[level].ptr, buf.data(), sizeof(float) * h->L.total, hipMemcpyHostToDevice));
+    PHC_TRY(write_field(h->stream, h->readback, h->lev[level].as<float>(), h->L, h->lh[0], h->lh[1], h->lh[2], host));
     h->pending[level] = 0;
     return PHC_OK;
 }
@@ -991,14 +969,9 @@ phc_status phc_fd_get_slice_xz(phc_fd *h, int level, int j, float *host)
 {
     if (!h || !host) return fail(PHC_ERR_INVALID, "handle or host buffer is NULL");
     if (j < 0 || j >= h->ny) return fail(PHC_ERR_INVALID, "slice j=%d outside 0..%d", j, h->ny - 1);
-    const int LX = h->lh[0], LY = h->lh[1], LZ = h->lh[2];
-    std::vector<float> full((size_t)(h->nx + 2 * LX) * (h->ny + 2 * LY) * (h->nz + 2 * LZ));
-    PHC_TRY(phc_fd_get_field(h, level, full.data()));
-    const int NYe = h->ny + 2 * LY, NZe = h->nz + 2 * LZ;
-    for (int k = 0; k < h->nz; ++k)
-        for (int i = 0; i < h->nx; ++i)
-            host[(int64_t)k * h->nx + i] = full[((int64_t)(i + LX) * NYe + (j + LY)) * NZe + (k + LZ)];
-    return PHC_OK;
+    if (level < 0 || level > 1) return fail(PHC_ERR_INVALID, "level %d is not 0 or 1", level);
+    const float *const f[3] = {h->hfx.data(), h->hfy.data(), h->hfz.data()};
+    return read_slice_xz(h->stream, h->readback, h->lev[level].as<float>(), h->L, j, fd_owed(h, level), f, host);
 }
 
 phc_status phc_fd_check_finite(phc_fd *h, int level)

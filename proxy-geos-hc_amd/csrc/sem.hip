@@ -37,6 +37,7 @@
 #include "march.hpp"
 #include "xcd_sched.hpp"
 #include "phc_common.hpp"
+#include "readback.hpp"
 #include "sem_setup.hpp"
 
 namespace phc {
@@ -903,7 +904,7 @@ struct phc_sem {
     float Dm[(SEM_MAX_P + 1) * (SEM_MAX_P + 1)];
     std::vector<float> hmass;
     // traces, and the running chunk's source samples
-    DevBuf trace, window, rec, recoff;
+    DevBuf trace, window, rec, recoff, readback;
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
     double last_ms = 0.0;
@@ -923,17 +924,12 @@ static void sem_drop_graph(phc_sem *h)
     for (RunGraph &g : h->graph) g.drop();
 }
 
-// Upload a node-order host field into a level (layout conversion for the
+// A node-order host field into a level (layout conversion for the
 // separable path; halo stays zero).
 static phc_status sem_put(phc_sem *h, DevBuf &dst, const float *host)
 {
     if (h->kernel == PHC_SEM_SEPARABLE) {
-        std::vector<float> buf((size_t)h->L.total, 0.f);
-        for (int iy = 0; iy < h->ny; ++iy)
-            for (int iz = 0; iz < h->nz; ++iz)
-                std::memcpy(&buf[(size_t)fd_off(h->L, iy, iz, 0)],
-                            host + ((int64_t)iy * h->nz + iz) * h->nx, sizeof(float) * h->nx);
-        PHC_HIP(hipMemcpy(dst.ptr, buf.data(), sizeof(float) * buf.size(), hipMemcpyHostToDevice));
+        return write_field(h->stream, h->readback, dst.as<float>(), h->L, 0, 0, 0, host);
     } else {
         PHC_HIP(hipMemcpy(dst.ptr, host, sizeof(float) * h->nn, hipMemcpyHostToDevice));
     }
@@ -942,15 +938,10 @@ static phc_status sem_put(phc_sem *h, DevBuf &dst, const float *host)
 
 static phc_status sem_get(phc_sem *h, const DevBuf &src, float *host)
 {
-    PHC_HIP(hipStreamSynchronize(h->stream));
     if (h->kernel == PHC_SEM_SEPARABLE) {
-        std::vector<float> buf((size_t)h->L.total);
-        PHC_HIP(hipMemcpy(buf.data(), src.ptr, sizeof(float) * buf.size(), hipMemcpyDeviceToHost));
-        for (int iy = 0; iy < h->ny; ++iy)
-            for (int iz = 0; iz < h->nz; ++iz)
-                std::memcpy(host + ((int64_t)iy * h->nz + iz) * h->nx,
-                            &buf[(size_t)fd_off(h->L, iy, iz, 0)], sizeof(float) * h->nx);
+        return read_field(h->stream, h->readback, src.as<float>(), h->L, 0, 0, 0, FieldDamping{}, nullptr, host);
     } else {
+        PHC_HIP(hipStreamSynchronize(h->stream));
         PHC_HIP(hipMemcpy(host, src.ptr, sizeof(float) * h->nn, hipMemcpyDeviceToHost));
     }
     return PHC_OK;
@@ -1310,8 +1301,8 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
         const size_t bytes = sizeof(float) * (size_t)h->L.total;
         if ((st = h->lev[0].alloc(bytes)) || (st = h->lev[1].alloc(bytes)) || (st = h->qf.alloc(bytes)))
             return bail(st);
-        PHC_HIP(hipMemset(h->lev[0].ptr, 0, bytes));
-        PHC_HIP(hipMemset(h->lev[1].ptr, 0, bytes));
+        for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf})
+            if ((st = fill_field(h->stream, b->as<float>(), h->L.total, 0.f))) return bail(st);
         // Q = dt^2 Wx Wz Wy / M on interior nodes, 0 elsewhere
         std::vector<float> Qn((size_t)h->nn, 0.f);
         for (int iy = 1; iy < h->ny - 1; ++iy)
@@ -1406,7 +1397,7 @@ phc_status phc_sem_destroy(phc_sem *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     sem_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->y, &h->dt2m, &h->geo, &h->rhs, &h->window, &h->trace,
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->y, &h->dt2m, &h->geo, &h->rhs, &h->window, &h->readback, &h->trace,
                       &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1635,8 +1626,11 @@ phc_status phc_sem_apply_stiffness(phc_sem *h, const float *p, float *y)
     // swap the levels' buffers for the scratch ones for one launch
     std::swap(h->lev[0], s0);
     std::swap(h->lev[1], s1);
-    phc_status st = sem_put(h, h->lev[0], p);
-    if (st == PHC_OK) st = sem_put(h, h->lev[1], p);
+    phc_status st = PHC_OK;
+    for (DevBuf *b : {&h->lev[0], &h->lev[1]}) {
+        if (st == PHC_OK && sep) st = fill_field(h->stream, b->as<float>(), h->L.total, 0.f);  // the halo
+        if (st == PHC_OK) st = sem_put(h, *b, p);
+    }
     if (st == PHC_OK) st = sem_launch(h, 0, 1, nullptr, nullptr, nullptr, nullptr);
     std::vector<float> out((size_t)h->nn);
     if (st == PHC_OK) st = sem_get(h, h->lev[0], out.data());

@@ -34,6 +34,7 @@
 
 #include "march.hpp"
 #include "phc_common.hpp"
+#include "readback.hpp"
 #include "sem_setup.hpp"
 
 namespace phc {
@@ -279,7 +280,7 @@ struct phc_sem2d {
     float cx[S2_MAX_P + 2][S2_W], cz[S2_MAX_P + 2][S2_W];
     std::vector<float> hmass, hsh;  // FP32 lumped mass and boundary term per node
     int chunk = 0, cus = 256;
-    DevBuf trace, window, rec, recoff;  // window: the running chunk's source samples
+    DevBuf trace, window, rec, recoff, readback;  // window: the running chunk's source samples
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
     double last_ms = 0.0;
@@ -309,13 +310,11 @@ static phc_status s2_put(phc_sem2d *h, DevBuf &dst, const float *host)
 
 static phc_status s2_get(phc_sem2d *h, const DevBuf &src, float *host)
 {
-    PHC_HIP(hipStreamSynchronize(h->stream));
-    std::vector<float> buf((size_t)h->L.total);
-    PHC_HIP(hipMemcpy(buf.data(), src.ptr, sizeof(float) * buf.size(), hipMemcpyDeviceToHost));
-    for (int iz = 0; iz < h->nz; ++iz)
-        std::memcpy(host + (int64_t)iz * h->nx, &buf[(size_t)s2_off(h, (int64_t)iz * h->nx)],
-                    sizeof(float) * h->nx);
-    return PHC_OK;
+    FdLayout L{};  // one plane of nz rows of nx nodes
+    L.nx = 1; L.ny = h->nz; L.nz = h->nx;
+    L.pitch_k = h->L.pitch;
+    L.origin = h->L.origin;
+    return read_field(h->stream, h->readback, src.as<float>(), L, 0, 0, 0, FieldDamping{}, nullptr, host);
 }
 
 static int s2_default_chunk(const phc_sem2d *h)
@@ -391,7 +390,7 @@ phc_status phc_sem2d_destroy(phc_sem2d *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     s2_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->sig, &h->rhs, &h->window, &h->trace, &h->rec, &h->recoff})
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->sig, &h->rhs, &h->window, &h->readback, &h->trace, &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
