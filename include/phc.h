@@ -375,7 +375,7 @@ typedef struct {
     float sponge_alpha;
     float init_value;         /* initial value of both levels */
     int arith;                /* PHC_FD_ARITH_* */
-    int tile_j, block_waves;  /* 0 = default (8 x 8) */
+    int tile_j, block_waves;  /* 0 = default (16 rows, 4 waves) */
     int chunk_i;              /* planes per work item at most, 0 = chosen from
                                * the shots' sizes; -m (m = 1..4): each shot's
                                * per-XCD schedule (as phc_fd_params.chunk_i),

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "fd_kernels.hpp"
+#include "fd_quad.hpp"
 #include "fd_tile.hpp"
 #include "xcd_sched.hpp"
 #include "march.hpp"
@@ -88,26 +89,28 @@ __device__ __forceinline__ void batch_sample(const BatchSample &r, const ShotDes
 // resident per CU, so one block's first loads (9 planes of ring, about 3 us
 // with the descriptor reads) run beside the others' marches; resident blocks
 // that claimed their items from a queue one after the other left that
-// latency and the claim's open: 12 shots of U[96,224]^3, best shape of each,
-// 200 us per step against 240 (47.7 M points: 3.8 against 3.2 TB/s).
-template <int R, int TY, int NJ, int ARITH, typename IT>
-__global__ void __launch_bounds__(FD_TK *TY)
-fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__restrict__ items, int nitems,
-                int cur, const int *it0, int inj, float *traces, int trace_stride, int step, BatchSample rec)
+// latency and the claim's open: 12 shots of U[96,224]^3, best one-point shape
+// of each, 200 us per step against 240 (47.7 M points: 3.8 against 3.2 TB/s;
+// 182 with four points per lane, 4.2 TB/s).
+//
+// fd_batch_item fills the grid of the block's item; false: nothing to march
+// (a sampling block, padding, or slab points, which it has updated).
+template <int R, int TY, int ARITH, typename IT>
+__device__ __forceinline__ bool fd_batch_item(const FdStepArgs &c, const ShotDesc *__restrict__ shots,
+                                              const int4 *__restrict__ items, int nitems, int cur, const int *it0,
+                                              int inj, float *traces, int trace_stride, int step,
+                                              const BatchSample &rec, FdGrid &g, float &rhs_next, int4 &tile)
 {
-    using SH = FdTileShape<R, TY, NJ>;
-    __shared__ float tile[2][SH::LH][SH::LW];
     constexpr int T = FD_TK * TY;
     if ((int)blockIdx.x >= nitems) {
         batch_sample(rec, shots, traces, cur,
                      ((int)blockIdx.x - nitems) * T + (int)(threadIdx.y * FD_TK + threadIdx.x));
-        return;
+        return false;
     }
     const int it = uniform_value(it0) + step;
     const int4 wi = items[blockIdx.x];
-    if (wi.z >= wi.w) return;  // padding of a shorter XCD list (whole block)
+    if (wi.z >= wi.w) return false;  // padding of a shorter XCD list (whole block)
     const ShotDesc &sd = shots[wi.x];
-    FdGrid g;
     g.L = sd.L;
     g.pn = sd.lev[cur];
     g.pnm1 = sd.lev[1 - cur];
@@ -116,7 +119,7 @@ fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__
     g.fz = sd.fz;
     g.src_off = sd.src_off;
     g.inj = inj;
-    const float rhs_next = uniform_value(inj ? sd.rhs + it + 1 : nullptr);
+    rhs_next = uniform_value(inj ? sd.rhs + it + 1 : nullptr);
     g.trace = traces + (int64_t)wi.x * trace_stride + step;
     g.ilo = 0; g.ihi = sd.L.nx;
     g.jlo = 0; g.jhi = sd.L.ny;
@@ -127,10 +130,41 @@ fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__
         const int64_t part = -1 - wi.y;
         for (int m = 0; m < BATCH_SLAB_PASSES; ++m)
             fd_rem_points<R, ARITH, IT>(c, g, rhs_next, (part * BATCH_SLAB_PASSES + m) * T);
-        return;
+        return false;
     }
-    const int tk = sd.tiles_k;
-    fd_tile<R, TY, NJ, ARITH, IT>(c, g, rhs_next, wi.y % tk, wi.y / tk, wi.z, wi.w, tile);
+    tile = make_int4(wi.y % sd.tiles_k, wi.y / sd.tiles_k, wi.z, wi.w);
+    return true;
+}
+
+template <int R, int TY, int NJ, int ARITH, typename IT>
+__global__ void __launch_bounds__(FD_TK *TY)
+fd_batch_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__restrict__ items, int nitems,
+                int cur, const int *it0, int inj, float *traces, int trace_stride, int step, BatchSample rec)
+{
+    using SH = FdTileShape<R, TY, NJ>;
+    __shared__ float tile[2][SH::LH][SH::LW];
+    FdGrid g;
+    float rhs_next;
+    int4 w;
+    if (fd_batch_item<R, TY, ARITH, IT>(c, shots, items, nitems, cur, it0, inj, traces, trace_stride, step, rec, g,
+                                        rhs_next, w))
+        fd_tile<R, TY, NJ, ARITH, IT>(c, g, rhs_next, w.x, w.y, w.z, w.w, tile);
+}
+
+// The shapes with 4 rows per wavefront: four points per lane (fd_quad.hpp).
+template <int TY, int ARITH, bool NT>
+__global__ void __launch_bounds__(FD_TK *TY) __attribute__((amdgpu_waves_per_eu(3)))
+fd_batch_quad_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int4 *__restrict__ items, int nitems,
+                     int cur, const int *it0, int inj, float *traces, int trace_stride, int step, BatchSample rec)
+{
+    using SH = FdQuadShape<TY>;
+    __shared__ fd_f4 tile[2][SH::LH][SH::LQ];
+    FdGrid g;
+    float rhs_next;
+    int4 w;
+    if (fd_batch_item<4, TY, ARITH, uint32_t>(c, shots, items, nitems, cur, it0, inj, traces, trace_stride, step,
+                                              rec, g, rhs_next, w))
+        fd_quad<TY, ARITH, uint32_t, false, NT>(c, g, rhs_next, w.x, w.y, w.z, w.w, tile);
 }
 
 // Start of a run at sample it: rhs[it] into every shot's current level at its
@@ -161,14 +195,25 @@ static BatchFn batch_arith(int arith)
                                      : fd_batch_kernel<R, TY, NJ, PHC_FD_ARITH_FP32, uint32_t>;
 }
 
-static BatchFn batch_pick(int R, int ty, int nj, int arith)
+template <int TY>
+static BatchFn batch_quad(int arith, bool nt)
+{
+    if (arith == PHC_FD_ARITH_REF)
+        return nt ? fd_batch_quad_kernel<TY, PHC_FD_ARITH_REF, true> : fd_batch_quad_kernel<TY, PHC_FD_ARITH_REF, false>;
+    return nt ? fd_batch_quad_kernel<TY, PHC_FD_ARITH_FP32, true> : fd_batch_quad_kernel<TY, PHC_FD_ARITH_FP32, false>;
+}
+
+// nt: non-temporal accesses to the streamed arrays (the four-points-per-lane
+// shapes; the others always have them).
+static BatchFn batch_pick(int R, int ty, int nj, int arith, bool nt = true)
 {
     if (R != 4) return nullptr;
     if (ty == 16 && nj == 1) return batch_arith<4, 16, 1>(arith);
     if (ty == 8 && nj == 1) return batch_arith<4, 8, 1>(arith);
     if (ty == 8 && nj == 2) return batch_arith<4, 8, 2>(arith);
     if (ty == 4 && nj == 2) return batch_arith<4, 4, 2>(arith);
-    if (ty == 4 && nj == 4) return batch_arith<4, 4, 4>(arith);
+    if (ty == 4 && nj == 4) return batch_quad<4>(arith, nt);
+    if (ty == 8 && nj == 4) return batch_quad<8>(arith, nt);
     return nullptr;
 }
 
@@ -205,19 +250,21 @@ static void batch_drop_graph(phc_batch *h)
     for (RunGraph &g : h->graph) g.drop();
 }
 
-// Planes per work item when the caller gives none.  With x planes of tile
-// columns per resident block, items of c planes waste about (2R+1)/c of the
-// time on ring lead-ins (loads without a stencil) and c/2x on the part-empty
-// last round, so the best c grows with sqrt(x).  The factor 3 fits the best
-// chunk lengths measured (x = 20, 66, 112, 321: 16, 24, 32, 48).
+// Planes per work item when the caller gives none: 24, fewer where a resident
+// block then gets less than a few items' worth of planes.  Items of c planes
+// waste about (2R+1)/c of the time on ring lead-ins (loads without a stencil)
+// and c/2x on the part-empty last round, x = planes of tile columns per
+// resident block.  Measured (4 waves x 16 rows; x = 13, 15, 44, 75, 214): 24
+// planes 34.1, 29.2, 88.8, 188, 612 us per step, the best of 8-128 planes
+// 31.7, 29.2, 88.8, 186, 609; at x = 1.1, 8 planes 9.6, 24 planes 16.1.
 static int batch_default_chunk(const phc_batch *h, const int *dims)
 {
     const int TJ = h->ty * h->nj;
     double planes = 0.0;
     for (int s = 0; s < h->nshots; ++s)
         planes += (double)((dims[3 * s + 2] + FD_TK - 1) / FD_TK) * ((dims[3 * s + 1] + TJ - 1) / TJ) * dims[3 * s];
-    const double slots = (double)h->cus * std::max(32 / (h->ty * h->nj), 1);
-    return std::clamp((int)std::lround(3.0 * std::sqrt(planes / slots)), 8, 64);
+    const double slots = (double)h->cus * (h->nj == 4 ? 12 / h->ty : std::max(32 / (h->ty * h->nj), 1));
+    return std::clamp((int)std::lround(7.0 * planes / slots), 8, 24);
 }
 
 // Work items of every shot for the current shape, one list per XCD,
@@ -333,7 +380,8 @@ static void batch_common(const phc_batch *h, FdStepArgs &c, int damp)
 static phc_status batch_launch(phc_batch *h, int cur, int inj, int damp, float *traces, int stride, int step,
                                const BatchSample &rec)
 {
-    BatchFn fn = batch_pick(h->R, h->ty, h->nj, h->arith);
+    // a pool past what the 256 MB memory-side cache keeps streams past it
+    BatchFn fn = batch_pick(h->R, h->ty, h->nj, h->arith, h->pool.bytes > (size_t)300e6);
     if (!fn) return fail(PHC_ERR_INVALID, "no batched kernel for %d waves x %d rows", h->ty, h->nj);
     FdStepArgs c;
     batch_common(h, c, damp);
@@ -399,12 +447,14 @@ phc_status phc_batch_create(const phc_batch_params *p, phc_batch **out)
         return fail(PHC_ERR_INVALID, "bad chunk_i (planes per item, or -1..-4) or blocks_per_cu");
     if (p->k_remainder < -1 || p->k_remainder > 1)
         return fail(PHC_ERR_INVALID, "k_remainder must be -1, 0 or 1 (got %d)", p->k_remainder);
-    // default: 8 waves x 1 row, the fastest shape on every survey measured
-    // (12 shots of U[96,224]^3 / 14 of U[60,100]^3 / 24 of U[128,256]^3, best
-    // chunk of each: 200 / 40 / 642 us per step; 4 waves x 2 rows 216 / 43 /
-    // 690, 16 x 1 227 / 46 / 690)
-    const int ty = p->block_waves ? p->block_waves : p->tile_j ? 16 : 8;
-    const int tj = p->tile_j ? p->tile_j : ty;
+    // default: 4 waves x 16 rows, four points per lane, the fastest shape on
+    // every survey measured (12 shots of U[96,224]^3 / 8 of U[106,190]^3 / 14
+    // of U[60,100]^3 / 24 of U[128,256]^3, best chunk of each: 182 / 89 / 29 /
+    // 609 us per step; 8 waves x 32 rows 202 / 102 / 33 / 633; 8 waves x 1 row
+    // 199 / 103 / 40 / 642; 4 waves x 2 rows 216 / 113 / 43 / 690)
+    const bool shape = p->block_waves || p->tile_j;
+    const int ty = p->block_waves ? p->block_waves : shape ? 16 : 4;
+    const int tj = p->tile_j ? p->tile_j : shape ? ty : 16;
     if (ty <= 0 || tj % ty != 0 || !batch_pick(p->half_width, ty, tj / ty, p->arith))
         return fail(PHC_ERR_INVALID, "no batched kernel for tile_j %d, %d waves per block", tj, ty);
     for (int s = 0; s < p->nshots; ++s) {
@@ -662,7 +712,7 @@ phc_status phc_batch_autotune(phc_batch *h, int steps_per_trial, int *tile_j, in
     hipEvent_t e0 = nullptr, e1 = nullptr;
     PHC_HIP(hipEventCreate(&e0));
     PHC_HIP(hipEventCreate(&e1));
-    static const int shapes[][2] = {{16, 1}, {8, 1}, {8, 2}, {4, 2}, {4, 4}};
+    static const int shapes[][2] = {{16, 1}, {8, 1}, {8, 2}, {8, 4}, {4, 2}, {4, 4}};
     static const int chunks[] = {8, 16, 24, 32, 48, 64, 128, -1, -2, -3, -4};
     static const int bpcs[] = {1, 2, 4};
     double best = 1e30;

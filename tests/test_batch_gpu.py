@@ -210,3 +210,31 @@ def test_receivers_fill_sampling_blocks(gpu, nrec, n):
         assert np.array_equal(src[k], tr) and np.array_equal(rv[k], orv), "shot %d" % k
         one.close()
     b.close()
+
+
+@pytest.mark.parametrize("tile_j,waves,chunk_i,krem", [(16, 4, 7, 0), (32, 8, 9, 0), (32, 8, -2, 0), (16, 4, 24, 1),
+                                                       (8, 8, 5, 0)])
+def test_quad_shapes_bit_exact(gpu, oracle, tile_j, waves, chunk_i, krem):
+    """Four points per lane (4 rows per wavefront) and the 8-wave one-row shape:
+    rows that end inside a quad, reference rounding = the oracle, FP32 = the
+    single-grid one-point tile, bit for bit."""
+    banner("quad shapes tile_j=%d waves=%d chunk=%d krem=%d" % (tile_j, waves, chunk_i, krem))
+    dims = [(12, 33, 66), (9, 15, 61), (30, 17, 131), (5, 4, 3)]
+    setups = make_shots(gpu, dims=dims, sponge=5, nsamples=30)
+    kw = dict(tile_j=tile_j, block_waves=waves, chunk_i=chunk_i, k_remainder=krem)
+    for arith in (gpu.ARITH_REF, gpu.ARITH_FP32):
+        b = gpu.FdBatch(setups, arith=arith, **kw)
+        src, _ = b.run(21)
+        for k, s in enumerate(setups):
+            if arith == gpu.ARITH_REF:
+                P = oracle_of(oracle, s)
+                tr, _ = P.run(21)
+                cur, prev = P.current(), P.previous()
+            else:
+                one = gpu.FdSolver(s, arith=arith, tile_j=8, block_waves=8, chunk_i=6)
+                tr, _ = one.run(0, 21)
+                cur, prev = one.current(), one.previous()
+                one.close()
+            assert np.array_equal(src[k], tr), "shot %d" % k
+            assert np.array_equal(b.field(k, True), cur) and np.array_equal(b.field(k, False), prev), "shot %d" % k
+        b.close()
