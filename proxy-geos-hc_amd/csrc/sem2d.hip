@@ -240,6 +240,186 @@ __global__ void sem2d_begin_run_kernel(float *p, int64_t off, float coef, const 
     if (t == 0) p[off] = add_nc(p[off], mul_nc(coef, rhs[it0]));
 }
 
+// T steps in one launch, for meshes whose step is bound by the launch and its
+// latency chain, not by memory (196^2 nodes: 0.6 MB per step).  A block of 16
+// wavefronts owns a TX(x) x TZ(z) tile and holds the tile plus P T nodes on
+// each side, the halo that T steps of a radius-P stencil reach: lane = column,
+// RZ consecutive rows per wavefront.  A node's current, previous and Q values
+// stay in registers; the current level goes through an LDS plane (double
+// buffer, one barrier per step) for the neighbours.  Each step computes the
+// rows that the steps left still need; halo nodes are computed by every block
+// that needs them, with the same operations in the same order as the one-step
+// kernel, so every node gets the same bits.  The levels are read from one pair
+// of buffers and written to another, since other blocks still read the halo.
+// 196^2 nodes of order 3: 6.2 us for 4 steps, 2.9 us for one alone
+// (s2_plan_multi has the other meshes).
+constexpr int S2_MW = 16;  // wavefronts per block
+
+struct Sem2dMultiArgs {
+    Sem2dArgs s;              // levels, model, layout, rows by class, source, receivers
+    float *out_n, *out_nm1;   // levels after the T steps: current, previous
+    int src_x, src_z;
+    const float *window;      // the run's samples; the launch's first step is step0 of nsteps
+    int step0, nsteps;
+    float *trace;
+    const int *rec_node;      // receivers' ix + iz nx
+    int tiles_x;
+};
+
+template <int P, int T, int RZ>
+__global__ void __launch_bounds__(64 * S2_MW) sem2d_multi_kernel(Sem2dMultiArgs m)
+{
+    constexpr int W = 2 * P + 1;
+    constexpr int H = S2_MW * RZ, PT = P * T;      // rows held; halo rows and columns per side
+    constexpr int TX = 64 - 2 * PT, TZ = H - 2 * PT;
+    static_assert(TX > 0 && TZ > 0, "the halo must leave a tile");
+    constexpr int NR = 2;                          // receivers per thread
+    __shared__ float plane[2][(H + 2 * P) * 64 + 2 * P];
+    __shared__ float src_before[2];  // value at the source node before its injection
+    const Sem2dArgs &a = m.s;
+    const Sem2Layout &L = a.L;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x0 = (int)(blockIdx.x % m.tiles_x) * TX - PT, z0 = (int)(blockIdx.x / m.tiles_x) * TZ - PT;
+    const int x = x0 + lane, zr = z0 + wv * RZ;  // the lane's column, the wavefront's first row
+    const bool xin = x >= 0 && x < L.nx;
+    const bool xown = lane >= PT && lane < PT + TX;
+    for (int t = threadIdx.x; t < 2 * ((H + 2 * P) * 64 + 2 * P); t += 64 * S2_MW) (&plane[0][0])[t] = 0.f;
+
+    float cur[RZ], old[RZ], q[RZ], sg[RZ];
+    bool in[RZ], edge[RZ];
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+        const int z = zr + r;
+        in[r] = xin && z >= 0 && z < L.nz;
+        const int64_t o = L.origin + (int64_t)(in[r] ? z : 0) * L.pitch + (in[r] ? x : 0);
+        cur[r] = in[r] ? a.pn[o] : 0.f;
+        old[r] = in[r] ? a.pnm1[o] : 0.f;
+        q[r] = in[r] ? a.qf[o] : 0.f;
+        edge[r] = in[r] && (z == 0 || z == L.nz - 1 || x == 0 || x == L.nx - 1);
+        sg[r] = !edge[r] ? 0.f : (z == 0) ? a.sig_z0[x] : (z == L.nz - 1) ? a.sig_z1[x]
+                               : (x == 0) ? a.sig_x0[z] : a.sig_x1[z];
+    }
+    float cxr[W];
+    {
+        const int cls = (x == 0) ? P : (x == L.nx - 1) ? P + 1 : (xin ? x % P : 0);
+#pragma unroll
+        for (int d = 0; d < W; ++d) cxr[d] = a.cx[cls][d];
+    }
+    int cls[RZ];  // rows' classes along z (uniform over the wavefront)
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+        const int z = zr + r;
+        cls[r] = (z == 0) ? P : (z == L.nz - 1) ? P + 1 : (z > 0 && z < L.nz) ? z % P : 0;
+    }
+    // receivers this block owns: their place in the plane
+    int rpos[NR];
+    bool rsrc[NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+        const int r = (int)threadIdx.x + k * 64 * S2_MW;
+        rpos[k] = -1;
+        rsrc[k] = false;
+        if (r < a.rec_n) {
+            const int node = m.rec_node[r], rx = node % L.nx - x0, rz = node / L.nx - z0;
+            if (rx >= PT && rx < PT + TX && rz >= PT && rz < PT + TZ) {
+                rpos[k] = P + (rz + P) * 64 + rx;
+                rsrc[k] = node == m.src_x + m.src_z * L.nx;
+            }
+        }
+    }
+    auto sample = [&](int t) {  // receivers after step t of the launch
+#pragma unroll
+        for (int k = 0; k < NR; ++k)
+            if (rpos[k] >= 0)
+                a.rec_out[(int64_t)((int)threadIdx.x + k * 64 * S2_MW) * a.rec_stride + m.step0 + t] =
+                    rsrc[k] ? src_before[t & 1] : plane[(t + 1) & 1][rpos[k]];
+    };
+    __syncthreads();
+    const int at = P + (wv * RZ + P) * 64 + lane;  // plane index of the lane's first row
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) plane[0][at + r * 64] = cur[r];
+
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        __syncthreads();
+        if (t > 0) sample(t - 1);
+        const float *pl = plane[t & 1];
+        float *pw = plane[(t + 1) & 1];
+        float zv[RZ + 2 * P];  // the lane's column, rows zr - P .. zr + RZ - 1 + P
+#pragma unroll
+        for (int r = 0; r < RZ + 2 * P; ++r)
+            zv[r] = (r >= P && r < P + RZ) ? cur[r - P] : pl[at + (r - P) * 64];
+#pragma unroll
+        for (int r = 0; r < RZ; ++r) {
+            const int row = wv * RZ + r;
+            // rows the remaining steps do not need any more
+            if (row < P * (t + 1) || row >= H - P * (t + 1)) continue;
+            const float pc = cur[r];
+            float lap = 0.f;
+#pragma unroll
+            for (int d = 0; d < W; ++d) {
+                if (d == P) continue;
+                lap = fmaf(a.cz[cls[r]][d], zv[r + d] - pc, lap);
+                lap = fmaf(cxr[d], pl[at + r * 64 + d - P] - pc, lap);
+            }
+            float val;
+            if (!edge[r]) val = fmaf(-q[r], lap, 2.f * pc - old[r]);
+            else val = fmaf(-q[r], lap, fmaf(1.f - sg[r], -old[r], 2.f * pc)) / (1.f + sg[r]);
+            if (x == m.src_x && zr + r == m.src_z) {
+                const int s = m.step0 + t;
+                src_before[t & 1] = val;
+                if (xown && row >= PT && row < PT + TZ) m.trace[s] = val;
+                if (s + 1 < m.nsteps) val = add_nc(val, mul_nc(a.inj_coef, m.window[s + 1]));
+            }
+            if (!in[r]) val = 0.f;
+            old[r] = pc;
+            cur[r] = val;
+            pw[at + r * 64] = val;
+        }
+    }
+    __syncthreads();
+    sample(T - 1);
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+        const int row = wv * RZ + r;
+        if (!in[r] || !xown || row < PT || row >= PT + TZ) continue;
+        const int64_t o = L.origin + (int64_t)(zr + r) * L.pitch + x;
+        m.out_n[o] = cur[r];
+        m.out_nm1[o] = old[r];
+    }
+}
+
+using Sem2dMultiFn = void (*)(Sem2dMultiArgs);
+
+template <int P, int T>
+static Sem2dMultiFn s2_multi_rows(int rz)
+{
+    if constexpr (2 * P * T + 16 <= 64) {
+        if constexpr (2 * S2_MW >= 2 * P * T + 8) if (rz == 2) return sem2d_multi_kernel<P, T, 2>;
+        if constexpr (3 * S2_MW >= 2 * P * T + 8) if (rz == 3) return sem2d_multi_kernel<P, T, 3>;
+        if constexpr (4 * S2_MW >= 2 * P * T + 8) if (rz == 4) return sem2d_multi_kernel<P, T, 4>;
+    }
+    return nullptr;
+}
+
+// Kernel of T = 4 or 8 steps with rz rows per wavefront, null if the halo
+// leaves less than 16 columns or 8 rows.
+static Sem2dMultiFn sem2d_pick_multi(int p, int t, int rz)
+{
+    switch (p * 10 + t) {
+    case 14: return s2_multi_rows<1, 4>(rz);
+    case 18: return s2_multi_rows<1, 8>(rz);
+    case 24: return s2_multi_rows<2, 4>(rz);
+    case 28: return s2_multi_rows<2, 8>(rz);
+    case 34: return s2_multi_rows<3, 4>(rz);
+    case 38: return s2_multi_rows<3, 8>(rz);
+    case 44: return s2_multi_rows<4, 4>(rz);
+    case 54: return s2_multi_rows<5, 4>(rz);
+    default: return nullptr;
+    }
+}
+
 using Sem2dFn = void (*)(Sem2dArgs);
 
 template <int P>
@@ -284,7 +464,12 @@ struct phc_sem2d {
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
     double last_ms = 0.0;
-    RunGraph graph[2];  // of phc_sem2d_run, by i1
+    // several steps per launch (small meshes): steps per launch (0: off), rows
+    // per wavefront, the second pair of levels, the receivers' nodes
+    int multi_t = 0, multi_rz = 0;
+    DevBuf alt[2], recnode;
+    int flipped = 0;    // lev and alt have changed places an odd number of times
+    RunGraph graph[4];  // of phc_sem2d_run, by i1 and flipped
 };
 
 static int64_t s2_off(const phc_sem2d *h, int64_t node)
@@ -329,13 +514,34 @@ static int s2_default_chunk(const phc_sem2d *h)
     return std::clamp((int)std::lround(2.5 * std::sqrt(x)), 1, std::min(16, h->nz));
 }
 
-// One step; rhs_next (device memory, may be null): sample injected after it;
-// rec_step >= 0: also samples level i2's receivers into that step of a run of
-// rec_stride steps.
-static phc_status s2_launch(phc_sem2d *h, int i1, int i2, const float *rhs_next, float *trace, hipEvent_t e0,
-                            hipEvent_t e1, int rec_step = -1, int rec_stride = 0)
+// Steps per launch (T) and rows per wavefront (RZ) for a mesh.  A launch costs
+// about 4 us and T RZ (0.2 + 0.04 P) us per round of one block per CU; a
+// single step 2.7 us and 4.6 us per million nodes.  Several steps per launch
+// are taken where the estimate is under 0.8 of the single step's; measured, us
+// per step, single / chosen: 196^2 order 3 2.86 / 1.56, 451^2 order 3
+// 4.1 / 2.3, 1201^2 order 3 9.7 / 7.0, 401^2 order 1 3.4 / 1.0, 501^2 order 2
+// 4.2 / 1.6, 401^2 order 4 4.0 / 2.6, 201^2 order 5 3.0 / 2.2; past the line
+// 381 x 476 order 5 4.4 (4.6 with 4 steps per launch), 751^2 order 5 6.3 (8.9).
+static void s2_plan_multi(phc_sem2d *h)
 {
-    Sem2dArgs a;
+    h->multi_t = h->multi_rz = 0;
+    double best = 0.8 * (2.7 + 4.6e-6 * (double)h->nn);
+    for (int t : {8, 4})
+        for (int rz : {2, 3, 4}) {
+            if (!sem2d_pick_multi(h->p, t, rz)) continue;
+            const int tx = 64 - 2 * h->p * t, tz = S2_MW * rz - 2 * h->p * t;
+            const double rounds = (double)((h->nx + tx - 1) / tx) * ((h->nz + tz - 1) / tz) / h->cus;
+            const double cost = (4.0 + t * rz * (0.2 + 0.04 * h->p) * std::max(1.0, rounds)) / t;
+            if (cost < best) {
+                best = cost;
+                h->multi_t = t;
+                h->multi_rz = rz;
+            }
+        }
+}
+
+static void s2_fill_args(const phc_sem2d *h, Sem2dArgs &a, int i1, int i2)
+{
     std::memset(&a, 0, sizeof(a));
     a.pn = h->lev[i2].as<float>();
     a.pnm1 = h->lev[i1].as<float>();
@@ -349,8 +555,18 @@ static phc_status s2_launch(phc_sem2d *h, int i1, int i2, const float *rhs_next,
     std::memcpy(a.cx, h->cx, sizeof(a.cx));
     std::memcpy(a.cz, h->cz, sizeof(a.cz));
     a.src_off = s2_off(h, h->src_node);
-    a.inj = rhs_next != nullptr;
     a.inj_coef = h->inj_coef;
+}
+
+// One step; rhs_next (device memory, may be null): sample injected after it;
+// rec_step >= 0: also samples level i2's receivers into that step of a run of
+// rec_stride steps.
+static phc_status s2_launch(phc_sem2d *h, int i1, int i2, const float *rhs_next, float *trace, hipEvent_t e0,
+                            hipEvent_t e1, int rec_step = -1, int rec_stride = 0)
+{
+    Sem2dArgs a;
+    s2_fill_args(h, a, i1, i2);
+    a.inj = rhs_next != nullptr;
     a.rhs_next = rhs_next;
     a.trace = trace;
     a.chunk = h->chunk > 0 ? h->chunk : s2_default_chunk(h);
@@ -390,7 +606,7 @@ phc_status phc_sem2d_destroy(phc_sem2d *h)
     if (!h) return PHC_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     s2_drop_graph(h);
-    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->qf, &h->sig, &h->rhs, &h->window, &h->readback, &h->trace, &h->rec, &h->recoff})
+    for (DevBuf *b : {&h->lev[0], &h->lev[1], &h->alt[0], &h->alt[1], &h->recnode, &h->qf, &h->sig, &h->rhs, &h->window, &h->readback, &h->trace, &h->rec, &h->recoff})
         b->release();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -530,6 +746,10 @@ phc_status phc_sem2d_create(const phc_sem_params *p, phc_sem2d **out)
             h->cus = cus;
     }
     h->index64 = p->index64 ? 1 : 0;
+    if (!h->chunk && !h->index64) s2_plan_multi(h);
+    if (h->multi_t)
+        for (DevBuf &b : h->alt)
+            if ((st = b.alloc(bytes)) || (st = fill_field(h->stream, b.as<float>(), h->L.total, 0.f))) return bail(st);
     *out = h;
     return PHC_OK;
 }
@@ -604,22 +824,57 @@ phc_status phc_sem2d_set_source(phc_sem2d *h, int src_element, int nsamples, con
 // injected its first sample), each step's launch sampling the receivers of
 // the one before.  Names no time sample, so that a captured run serves every
 // chunk.
+// Where a mesh takes several steps per launch, whole launches come first
+// (reading lev and writing alt, or the reverse), single steps after them; the
+// levels end in lev, or in alt after an odd number of launches.
 static phc_status s2_enqueue_run(phc_sem2d *h, int nsteps, int i1, int i2, std::vector<hipEvent_t> *ev)
 {
     const float *win = h->window.as<float>();
-    for (int s = 0; s < nsteps; ++s) {
-        PHC_TRY(s2_launch(h, i1, i2, s + 1 < nsteps ? win + s + 1 : nullptr, h->trace.as<float>() + s,
-                          ev ? (*ev)[2 * s] : nullptr, ev ? (*ev)[2 * s + 1] : nullptr, h->nrec > 0 ? s - 1 : -1,
-                          nsteps));
+    const int t = ev || h->nrec > 2 * 64 * S2_MW ? 0 : h->multi_t, launches = t ? nsteps / t : 0;
+    for (int l = 0; l < launches; ++l) {
+        Sem2dMultiArgs m;
+        s2_fill_args(h, m.s, i1, i2);
+        DevBuf *from = (l & 1) ? h->alt : h->lev, *to = (l & 1) ? h->lev : h->alt;
+        m.s.pn = from[i2].as<float>();
+        m.s.pnm1 = from[i1].as<float>();
+        m.out_n = to[i2].as<float>();
+        m.out_nm1 = to[i1].as<float>();
+        m.src_x = h->src_node % h->nx;
+        m.src_z = h->src_node / h->nx;
+        m.window = win;
+        m.step0 = l * t;
+        m.nsteps = nsteps;
+        m.trace = h->trace.as<float>();
+        m.rec_node = h->recnode.as<int>();
+        m.s.rec_out = h->rec.as<float>();
+        m.s.rec_n = h->nrec;
+        m.s.rec_stride = nsteps;
+        const int tx = 64 - 2 * h->p * t, tz = S2_MW * h->multi_rz - 2 * h->p * t;
+        m.tiles_x = (h->nx + tx - 1) / tx;
+        hipLaunchKernelGGL(sem2d_pick_multi(h->p, t, h->multi_rz), dim3(m.tiles_x * ((h->nz + tz - 1) / tz)),
+                           dim3(64 * S2_MW), 0, h->stream, m);
+        PHC_HIP(hipGetLastError());
+    }
+    if (launches & 1)
+        for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
+    phc_status st = PHC_OK;
+    for (int s = launches * t; s < nsteps && st == PHC_OK; ++s) {
+        // the launches above have sampled their own steps
+        const int rs = h->nrec > 0 && s > launches * t ? s - 1 : -1;
+        st = s2_launch(h, i1, i2, s + 1 < nsteps ? win + s + 1 : nullptr, h->trace.as<float>() + s,
+                       ev ? (*ev)[2 * s] : nullptr, ev ? (*ev)[2 * s + 1] : nullptr, rs, nsteps);
         std::swap(i1, i2);
     }
-    if (h->nrec > 0) {
+    if (st == PHC_OK && h->nrec > 0 && launches * t < nsteps) {
         hipLaunchKernelGGL(sem2d_sample_kernel, dim3((h->nrec + 255) / 256), dim3(256), 0, h->stream,
                            h->lev[i2].as<float>(), h->recoff.as<int64_t>(), h->nrec, h->rec.as<float>(), nsteps,
                            nsteps - 1, s2_off(h, h->src_node), h->trace.as<float>());
-        PHC_HIP(hipGetLastError());
+        if (hipGetLastError() != hipSuccess) st = fail(PHC_ERR_HIP, "receiver sampling launch failed");
     }
-    return PHC_OK;
+    // enqueueing leaves the handle as it was: the caller moves it on
+    if (launches & 1)
+        for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
+    return st;
 }
 
 phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
@@ -666,8 +921,12 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        PHC_TRY(run_captured(h->stream, h->graph[i1], nsteps, 0, h->nrec,
+        PHC_TRY(run_captured(h->stream, h->graph[i1 + 2 * h->flipped], nsteps, 0, h->nrec,
                              [&] { return s2_enqueue_run(h, nsteps, i1, i2, nullptr); }));
+        if (h->multi_t && h->nrec <= 2 * 64 * S2_MW && (nsteps / h->multi_t) % 2) {
+            for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
+            h->flipped ^= 1;
+        }
     }
     h->last_n = nsteps;
     h->last_nrec = h->nrec;
@@ -691,6 +950,8 @@ phc_status phc_sem2d_set_receivers(phc_sem2d *h, int nrec, const int *nodes)
     if (nrec > 0) {
         PHC_TRY(h->recoff.alloc(sizeof(int64_t) * nrec));
         PHC_HIP(hipMemcpy(h->recoff.ptr, offs.data(), sizeof(int64_t) * nrec, hipMemcpyHostToDevice));
+        PHC_TRY(h->recnode.alloc(sizeof(int) * nrec));
+        PHC_HIP(hipMemcpy(h->recnode.ptr, nodes, sizeof(int) * nrec, hipMemcpyHostToDevice));
     }
     return PHC_OK;
 }
