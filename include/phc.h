@@ -225,14 +225,16 @@ typedef struct {
     int src_element;       /* element holding the source (SEMproxy.cpp:101-106) */
     int kernel;            /* PHC_SEM_* */
     int weights_ref;       /* 1: the reference's 8-decimal GLL weights; 0: exact */
-    int tile_j, block_waves, chunk_i; /* separable kernel tiling (all 0: default); chunk_i = -m,
-                                         m = 1..4: per-XCD schedule of 8 >> (m-1) plane
-                                         ranges x 2^(m-1) column bands */
+    int tile_j, block_waves, chunk_i; /* separable kernel tiling: block_waves (4, 8, 16) x 1 or 2
+                                         rows, 4 or 8 x 4 rows (four nodes per lane); all 0: from
+                                         the mesh; chunk_i = -m, m = 1..4: per-XCD schedule of
+                                         8 >> (m-1) plane ranges x 2^(m-1) column bands */
     int index64;           /* 1: 64-bit offsets in the separable and 2D kernels even
                               when every array is < 4 GiB (testing) */
     int k_remainder;       /* separable kernel: a last, partial 64-node tile along x
                               updated node by node when it holds at most 32 nodes (0,
-                              default), always (1), or marched as a tile (-1) */
+                              default; with four nodes per lane never), always (1), or
+                              marched as a tile (-1) */
 } phc_sem_params;
 
 phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out);

@@ -158,7 +158,7 @@ fd_batch_quad_kernel(FdStepArgs c, const ShotDesc *__restrict__ shots, const int
                      int cur, const int *it0, int inj, float *traces, int trace_stride, int step, BatchSample rec)
 {
     using SH = FdQuadShape<TY>;
-    __shared__ fd_f4 tile[2][SH::LH][SH::LQ];
+    __shared__ quad_f4 tile[2][SH::LH][SH::LQ];
     FdGrid g;
     float rhs_next;
     int4 w;

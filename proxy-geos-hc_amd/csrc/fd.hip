@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(FD_TK *TY) __attribute__((amdgpu_waves_per_eu(
 fd_quad_kernel(FdStepArgs a)
 {
     using SH = FdQuadShape<TY>;
-    __shared__ fd_f4 tile[2][SH::LH][SH::LQ];
+    __shared__ quad_f4 tile[2][SH::LH][SH::LQ];
     if ((int)blockIdx.x >= (int)gridDim.x - a.rec_blocks) {
         fd_sample_prev(a);
         return;

@@ -4,32 +4,10 @@
 // shapes with 4 rows per wavefront.
 #pragma once
 
-#include <type_traits>
-#include <utility>
-
 #include "fd_tile.hpp"
+#include "quad.hpp"
 
 namespace phc {
-
-typedef float fd_f4 __attribute__((ext_vector_type(4)));
-
-template <bool NT, typename IT>
-__device__ __forceinline__ fd_f4 ldq(const float *base, IT off)
-{
-    if constexpr (NT) return ldo_nt<IT, fd_f4>((const fd_f4 *)base, sizeof(IT) == 4 ? off : off / 4);
-    else return ldo<IT, fd_f4>((const fd_f4 *)base, sizeof(IT) == 4 ? off : off / 4);
-}
-
-template <bool NT, typename IT>
-__device__ __forceinline__ void stq(float *base, IT off, fd_f4 v)
-{
-    if constexpr (NT) {
-        sto_nt<IT, fd_f4>((fd_f4 *)base, sizeof(IT) == 4 ? off : off / 4, v);
-    } else {
-        if constexpr (sizeof(IT) == 4) *(fd_f4 *)((char *)base + off) = v;
-        else ((fd_f4 *)base)[off / 4] = v;
-    }
-}
 
 // A block of TY wavefronts owns a 64(k) x 4 TY(j) column and marches along i
 // as fd_tile does (register ring along i, halo ring, LDS plane, unconditional
@@ -48,13 +26,6 @@ __device__ __forceinline__ void stq(float *base, IT off, fd_f4 v)
 // Every point takes the same operations in the same order as in fd_tile, so
 // both give the same bits.  NT: the streamed pnm1 and vp with non-temporal
 // accesses (working sets past the cache), else cached ones.
-// plane(u, ib + u) for u = 0, 1, ... while ib + u < end.
-template <class F, int... U>
-__device__ __forceinline__ void fd_turn(F &plane, int ib, int end, std::integer_sequence<int, U...>)
-{
-    (void)((ib + U < end && (plane(std::integral_constant<int, U>{}, ib + U), true)) && ...);
-}
-
 template <int TY>
 struct FdQuadShape {
     static constexpr int TJ = 4 * TY;
@@ -64,7 +35,7 @@ struct FdQuadShape {
 
 template <int TY, int ARITH, typename IT, bool PML, bool NT, class G>
 __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float rhs_next, int kt, int jt, int i0,
-                                        int i1, fd_f4 (*tile)[FdQuadShape<TY>::LH][FdQuadShape<TY>::LQ])
+                                        int i1, quad_f4 (*tile)[FdQuadShape<TY>::LH][FdQuadShape<TY>::LQ])
 {
     constexpr int R = 4;
     constexpr int TJ = 4 * TY;
@@ -119,7 +90,7 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
 
     // sponge factors of the lane's points on planes inside the undamped i
     // range (sin) and whether they take the plane's factor outside it (sfx)
-    fd_f4 sin;
+    quad_f4 sin;
     bool sfx[4];
     const bool inJ = j >= a.sw && j < L.ny - a.sw;
 #pragma unroll
@@ -172,7 +143,7 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
     }
     const int nval = min(4, L.nz - k);  // points of the quad inside the grid (<= 0: none)
 
-    fd_f4 q[Q], fh[NH][F], pm[2], vv[2], ph[2];
+    quad_f4 q[Q], fh[NH][F], pm[2], vv[2], ph[2];
     float ex[2][3];
 
     auto load_halo = [&](int slot, int p) {
@@ -193,7 +164,7 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
         }
     };
     auto stage = [&](int buf, int qslot, int hslot) {
-        fd_f4(*tl)[LQ] = tile[buf];
+        quad_f4(*tl)[LQ] = tile[buf];
         tl[row + R][qd + 1] = q[qslot];
 #pragma unroll
         for (int m = 0; m < NH; ++m)
@@ -219,17 +190,17 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
             load_aux((u + 1) & 1, min(i + 1, L.nx - 1));
         }
         if (jk) {
-            const fd_f4(*tl)[LQ] = tile[u & 1];
+            const quad_f4(*tl)[LQ] = tile[u & 1];
             const int r = row + R;
-            const fd_f4 pc = q[(u + R) % Q];
-            const fd_f4 pmr = pm[u & 1], vq = vv[u & 1];
-            fd_f4 up[R + 1], dn[R + 1];
+            const quad_f4 pc = q[(u + R) % Q];
+            const quad_f4 pmr = pm[u & 1], vq = vv[u & 1];
+            quad_f4 up[R + 1], dn[R + 1];
 #pragma unroll
             for (int l = 1; l <= R; ++l) {
                 up[l] = tl[r + l][qd + 1];
                 dn[l] = tl[r - l][qd + 1];
             }
-            const fd_f4 zl = tl[r][qd], zr = tl[r][qd + 2];
+            const quad_f4 zl = tl[r][qd], zr = tl[r][qd + 2];
             float z[12];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -268,9 +239,9 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
                     for (int c = 0; c < 4; ++c) lap[c] = fmaf(a.cz[l], z[4 + c + l] + z[4 + c - l], lap[c]);
                 }
             }
-            fd_f4 val;
+            quad_f4 val;
             {
-                fd_f4 s = {1.f, 1.f, 1.f, 1.f};
+                quad_f4 s = {1.f, 1.f, 1.f, 1.f};
                 if (a.sw > 0) {
                     if (i >= a.sw && i < L.nx - a.sw) {
                         s = sin;
@@ -297,7 +268,7 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
                 const bool pslab_i = i < a.px3 || i >= a.px4;
                 if (pslab_i || qslab) {
                     const float exm = ex[u & 1][0], ex0 = ex[u & 1][1], exp_ = ex[u & 1][2];
-                    fd_f4 phn = ph[u & 1];
+                    quad_f4 phn = ph[u & 1];
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         float e, tg, v, pn;
@@ -329,7 +300,7 @@ __device__ __forceinline__ void fd_quad(const FdStepArgs &a, const G &g, float r
         stage((u + 1) & 1, (u + 1 + R) % Q, (u + 1) % F);
         lds_barrier();
     };
-    for (int ib = i0; ib < i1; ib += Q) fd_turn(plane, ib, i1, std::make_integer_sequence<int, Q>{});
+    for (int ib = i0; ib < i1; ib += Q) march_turn(plane, ib, i1, std::make_integer_sequence<int, Q>{});
 }
 
 } // namespace phc

@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "fd_kernels.hpp"
+#include "quad.hpp"
 #include "march.hpp"
 #include "xcd_sched.hpp"
 #include "phc_common.hpp"
@@ -308,6 +309,220 @@ sem_sep_kernel(SemSepArgs a)
             lds_barrier();
         }
     }
+}
+
+// The separable step with four nodes per lane, for the shapes with 4 rows per
+// wavefront: the FD step's quad tile (fd_quad.hpp) with the separable
+// operator's coefficients.  A lane holds 4 consecutive x nodes of one row; at
+// orders 1, 2 and 4 a component's coefficient row along x is the same in
+// every lane (its index mod p is the component's), at 3 and 5 it depends on
+// the lane and is held in registers.  Every node takes the same operations in
+// the same order as in sem_sep_kernel, so both give the same bits.
+// Bound by the LDS reads and instructions of a node below the memory-side
+// cache's size, by memory above it.  One node per lane (best shape) / four, us
+// per step: 151^3 order 2 20.5 / 16.5, 151^3 order 3 22.5 / 16.7, 241^3 order
+// 4 52.9 / 42.2, 186 x 111 x 146 order 5 21.8 / 19.0, 401^3 order 4 (774 MB,
+// 16 B per node) 211 / 198.
+template <int P>
+struct SemQuadShape {
+    static constexpr int HQ = (P + 3) / 4;               // halo quads per side of a row
+    static constexpr int LQ = FD_TK / 4 + 2 * HQ;        // quads of an LDS row
+    static constexpr int U = P == 4 ? 20 : 2 * P + 2;    // planes per turn (order 4: the march's row is u % 4)
+};
+
+template <int P, int TY, typename IT, bool NT>
+__global__ void __launch_bounds__(FD_TK *TY) __attribute__((amdgpu_waves_per_eu(P == 5 ? 2 : 3)))
+sem_quad_kernel(SemSepArgs a)
+{
+    constexpr int R = P, W = 2 * P + 1, TJ = 4 * TY, LH = TJ + 2 * R;
+    constexpr int HQ = SemQuadShape<P>::HQ, LQ = SemQuadShape<P>::LQ;
+    constexpr int T = FD_TK * TY;
+    constexpr int NROW = 2 * R * (FD_TK / 4), NHQ = NROW + 2 * HQ * TJ;  // halo quads: rows, then row ends
+    constexpr int NH = (NHQ + T - 1) / T;
+    constexpr int Q = 2 * R + 2, F = R + 1, U = SemQuadShape<P>::U;
+    constexpr IT S = sizeof(IT) == 4 ? 4 : 1;
+    constexpr bool UNI = 4 % P == 0;  // a component's x row is the same in every lane
+    __shared__ quad_f4 tile[2][LH][LQ];
+
+    if ((int)blockIdx.x >= (int)gridDim.x - a.rec_blocks) {
+        const int r = ((int)blockIdx.x - ((int)gridDim.x - a.rec_blocks)) * T +
+                      (int)(threadIdx.y * FD_TK + threadIdx.x);
+        if (r < a.rec_n)
+            sem_sample_point(a.pn, a.rec_off, r, a.rec_out, a.rec_stride, a.rec_step, a.src_off, a.rec_src);
+        return;
+    }
+    const float rhs_next = uniform_value(a.rhs_next);
+    if (a.nb_main && (int)blockIdx.x >= a.nb_main) {
+        sem_rem_points<P, IT>(a, rhs_next, (int64_t)(blockIdx.x - a.nb_main) * T +
+                                               (int64_t)threadIdx.y * FD_TK + threadIdx.x);
+        return;
+    }
+    const FdLayout &L = a.L;
+    int w, i0, i1;
+    if (a.sched) {
+        const int4 e = a.sched[blockIdx.x];
+        w = e.x;
+        i0 = e.y;
+        i1 = e.z;
+        if (i0 >= i1) return;  // padding of a shorter XCD list (whole block)
+    } else {
+        const int b = xcd_block(blockIdx.x, a.nb_main ? a.nb_main : (int)gridDim.x - a.rec_blocks);
+        const int ic = b / (a.tiles_k * a.tiles_j);
+        w = b - ic * (a.tiles_k * a.tiles_j);
+        i0 = ic * a.chunk_i;
+        i1 = min(i0 + a.chunk_i, L.nx);
+    }
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int k0 = (w % a.tiles_k) * FD_TK, j0 = 1 + (w / a.tiles_k) * TJ;  // rows 0 and ny-1 are Dirichlet
+    const int qd = tx & 15, row = ty * 4 + (tx >> 4);
+    const int k = k0 + 4 * qd, j = j0 + row;
+    const IT pitch = (IT)L.pitch_j * S;
+
+    const bool jk = j < L.ny - 1 && k < L.nz - 1;  // the lane updates at least one node of [1, nz-1)
+    const bool ld = j < L.ny + R && k < L.nz + R;
+    const IT colq = (IT)fd_off(L, 0, ld ? j : 0, ld ? k : 0) * S;
+    int hrow[NH], hq[NH];
+    IT colh[NH];
+    bool hst[NH];
+#pragma unroll
+    for (int m = 0; m < NH; ++m) {
+        const int h = ty * FD_TK + tx + T * m;
+        int jh, kh;
+        if (h < NROW) {
+            const int hr = h >> 4;
+            jh = hr < R ? j0 - R + hr : j0 + TJ + hr - R;
+            kh = k0 + 4 * (h & 15);
+            hrow[m] = hr < R ? hr : TJ + hr;
+            hq[m] = (h & 15) + HQ;
+        } else {
+            const int e = h - NROW, s = e % (2 * HQ);
+            jh = j0 + e / (2 * HQ);
+            kh = s < HQ ? k0 + 4 * (s - HQ) : k0 + FD_TK + 4 * (s - HQ);
+            hrow[m] = e / (2 * HQ) + R;
+            hq[m] = s < HQ ? s : FD_TK / 4 + s;
+        }
+        hst[m] = h < NHQ;
+        const bool l = hst[m] && jh < L.ny + R && kh < L.nz + R;
+        colh[m] = (IT)fd_off(L, 0, l ? jh : 0, l ? kh : 0) * S;
+    }
+    float czr[W], cxv[UNI ? 1 : 4][W];
+    {
+        const int mz = j % P;
+#pragma unroll
+        for (int d = 0; d < W; ++d) czr[d] = a.cz[mz][d];
+        if constexpr (!UNI) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int mx = (k + c) % P;
+#pragma unroll
+                for (int d = 0; d < W; ++d) cxv[c][d] = a.cx[mx][d];
+            }
+        }
+    }
+    int src_i = -1, src_c = 0;
+    {
+        const int64_t d = a.src_off - (int64_t)(colq / S);
+        if (jk && d >= 0) {
+            int64_t pi, c;
+            if constexpr (sizeof(IT) == 4) {
+                pi = (uint32_t)d / (uint32_t)L.pitch_j;
+                c = (uint32_t)d % (uint32_t)L.pitch_j;
+            } else {
+                pi = d / L.pitch_j;
+                c = d % L.pitch_j;
+            }
+            if (c < 4 && k + c >= 1 && k + c < L.nz - 1) {  // a boundary source is not injected by the step
+                src_i = (int)pi;
+                src_c = (int)c;
+            }
+        }
+    }
+    bool kin[4];  // interior along x
+#pragma unroll
+    for (int c = 0; c < 4; ++c) kin[c] = k + c >= 1 && k + c < L.nz - 1;
+
+    quad_f4 q[Q], fh[NH][F], pm[2], qv[2];
+    auto load_halo = [&](int slot, int p) {
+        const IT po = (IT)p * pitch;
+#pragma unroll
+        for (int m = 0; m < NH; ++m) fh[m][slot] = ldq<false>(a.pn, colh[m] + po);
+    };
+    auto load_aux = [&](int set, int p) {
+        const IT po = (IT)p * pitch;
+        pm[set] = ldq<NT>(a.pnm1, colq + po);
+        qv[set] = ldq<NT>(a.qf, colq + po);
+    };
+    auto stage = [&](int buf, int qslot, int hslot) {
+        quad_f4(*tl)[LQ] = tile[buf];
+        tl[row + R][qd + HQ] = q[qslot];
+#pragma unroll
+        for (int m = 0; m < NH; ++m)
+            if (hst[m]) tl[hrow[m]][hq[m]] = fh[m][hslot];
+    };
+#pragma unroll
+    for (int l = 0; l <= 2 * R; ++l) q[l] = ldq<false>(a.pn, colq + (IT)(i0 - R + l) * pitch);
+#pragma unroll
+    for (int d = 0; d <= R; ++d) load_halo(d, i0 + d);
+    load_aux(0, i0);
+    stage(0, R, 0);
+    lds_barrier();
+
+    auto plane = [&](auto uc, int i) __attribute__((always_inline)) {
+        constexpr int u = decltype(uc)::value;
+        {
+            const int pq = min(i + 1 + R, L.nx + R - 1);
+            q[(u + 1 + 2 * R) % Q] = ldq<false>(a.pn, colq + (IT)pq * pitch);
+            load_halo((u + F) % F, pq);
+            load_aux((u + 1) & 1, min(i + 1, L.nx - 1));
+        }
+        if (jk && i >= 1 && i < L.nx - 1) {
+            const quad_f4(*tl)[LQ] = tile[u & 1];
+            const int my = (P == 4) ? (u % P) : (i % P);
+            const int r = row + R;
+            const quad_f4 pc = q[(u + R) % Q];
+            quad_f4 zr[W];
+            float x[4 * (2 * HQ + 1)];
+#pragma unroll
+            for (int d = 0; d < W; ++d)
+                if (d != R) zr[d] = tl[r - R + d][qd + HQ];
+#pragma unroll
+            for (int s = 0; s < 2 * HQ + 1; ++s) {
+                const quad_f4 v = s == HQ ? pc : tl[r][qd + s];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) x[4 * s + c] = v[c];
+            }
+            float lap[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int d = 0; d < W; ++d) {
+                if (d == R) continue;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) lap[c] = fmaf(a.cy[my][d], q[(u + d) % Q][c] - pc[c], lap[c]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) lap[c] = fmaf(czr[d], zr[d][c] - pc[c], lap[c]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    lap[c] = fmaf(UNI ? a.cx[c % P][d] : cxv[UNI ? 0 : c][d], x[4 * HQ + c - R + d] - pc[c], lap[c]);
+            }
+            quad_f4 val;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) val[c] = fmaf(-qv[u & 1][c], lap[c], 2.f * pc[c] - pm[u & 1][c]);
+            if (src_i == i) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (src_c == c) {
+                        if (a.trace) *a.trace = val[c];
+                        if (a.inj) val[c] = add_nc(val[c], mul_nc(a.inj_coef, rhs_next));
+                    }
+            }
+            // boundary nodes and what lies beyond the row keep their values
+#pragma unroll
+            for (int c = 0; c < 4; ++c) val[c] = kin[c] ? val[c] : pm[u & 1][c];
+            stq<NT>(a.pnm1, colq + (IT)i * pitch, val);
+        }
+        stage((u + 1) & 1, (u + 1 + R) % Q, (u + 1) % F);
+        lds_barrier();
+    };
+    for (int ib = i0; ib < i1; ib += U) march_turn(plane, ib, i1, std::make_integer_sequence<int, U>{});
 }
 
 // ------------------------------------------------------------ element path
@@ -810,9 +1025,18 @@ static SemSepFn sep_idx(bool idx32)
     return idx32 ? sem_sep_kernel<P, TY, NJ, uint32_t> : sem_sep_kernel<P, TY, NJ, int64_t>;
 }
 
-template <int P>
-static SemSepFn sep_shape(int ty, int nj, bool idx32)
+template <int P, int TY>
+static SemSepFn quad_idx(bool idx32, bool nt)
 {
+    if (!idx32) return sem_quad_kernel<P, TY, int64_t, true>;
+    return nt ? sem_quad_kernel<P, TY, uint32_t, true> : sem_quad_kernel<P, TY, uint32_t, false>;
+}
+
+template <int P>
+static SemSepFn sep_shape(int ty, int nj, bool idx32, bool nt)
+{
+    if (ty == 8 && nj == 4) return quad_idx<P, 8>(idx32, nt);
+    if (ty == 4 && nj == 4) return quad_idx<P, 4>(idx32, nt);
     if (ty == 16 && nj == 1) return sep_idx<P, 16, 1>(idx32);
     if (ty == 16 && nj == 2) return sep_idx<P, 16, 2>(idx32);
     if (ty == 8 && nj == 2) return sep_idx<P, 8, 2>(idx32);
@@ -822,14 +1046,14 @@ static SemSepFn sep_shape(int ty, int nj, bool idx32)
     return nullptr;
 }
 
-static SemSepFn sem_pick_sep(int p, int ty, int nj, bool idx32)
+static SemSepFn sem_pick_sep(int p, int ty, int nj, bool idx32, bool nt)
 {
     switch (p) {
-    case 1: return sep_shape<1>(ty, nj, idx32);
-    case 2: return sep_shape<2>(ty, nj, idx32);
-    case 3: return sep_shape<3>(ty, nj, idx32);
-    case 4: return sep_shape<4>(ty, nj, idx32);
-    case 5: return sep_shape<5>(ty, nj, idx32);
+    case 1: return sep_shape<1>(ty, nj, idx32, nt);
+    case 2: return sep_shape<2>(ty, nj, idx32, nt);
+    case 3: return sep_shape<3>(ty, nj, idx32, nt);
+    case 4: return sep_shape<4>(ty, nj, idx32, nt);
+    case 5: return sep_shape<5>(ty, nj, idx32, nt);
     default: return nullptr;
     }
 }
@@ -959,9 +1183,75 @@ static void sem_build_sched(int nx, int ncol, int slots, int m, std::vector<int4
 static int sem_tiles_k(const phc_sem *h, int *krem)
 {
     const int span = std::max(h->L.nz - 1, 1), full = span / FD_TK, rem = span - full * FD_TK;
-    const bool use = h->krem_mode >= 0 && full > 0 && rem > 0 && (h->krem_mode == 1 || rem <= FD_TK / 2);
+    // mode 0 with four nodes per lane: a tile (as nodes it cost 1-13% more at
+    // 76^3 and 151^3 order 3, nothing elsewhere)
+    const bool use = h->krem_mode >= (h->nj == 4 ? 1 : 0) && full > 0 && rem > 0 &&
+                     (h->krem_mode == 1 || rem <= FD_TK / 2);
     if (krem) *krem = use ? FD_TK * full : 0;
     return use ? full : (span + FD_TK - 1) / FD_TK;
+}
+
+static SemSepFn sem_handle_kernel(const phc_sem *h)
+{
+    // non-temporal pnm1 and coefficients (quad kernels) from where the three
+    // arrays no longer stay in the 256 MB memory-side cache, as in the FD step
+    return sem_pick_sep(h->p, h->ty, h->nj, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32),
+                        12 * h->L.total > (int64_t)300e6);
+}
+
+// Blocks of the handle's shape resident per CU.
+static int sem_resident(const phc_sem *h)
+{
+    int per_cu = 1;
+    SemSepFn fn = sem_handle_kernel(h);
+    if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(fn),
+                                                            FD_TK * h->ty, 0) != hipSuccess || per_cu < 1)
+        per_cu = 1;
+    return per_cu;
+}
+
+// Block shape and per-XCD split where the caller gives none.
+// Below 600,000 nodes 8 waves x 1 row, split 2: four nodes per lane leave too
+// few wavefronts there (51^3 order 5: 9.6 against 10.9 us per step, 81^3 order
+// 4: 9.7 / 10.3; 101^3, at once above the line: order 1 10.2 / 8.7, order 2
+// 11.9 / 9.5, order 5 15.3 / 14.3).  Above, 4 waves x 16 rows, split 1, the
+// best or within 5% of the best table entry from 101^3 to 321^3 (order 1
+// alone prefers chunks of 12-24 planes by up to 14%).  From 500 MB of arrays
+// the shape and split with the least work on the busiest CU, as in the FD
+// step: us per step of 8 x 1 / 4 x 16 split 1 / chosen: 341^3 order 2 122 /
+// 117 / 111, 331 x 346 x 331 order 3 127 / 112 / 104, 353 x 361 x 345 order 4
+// 148 / 141 / 122, 351 x 361 x 351 order 5 186 / 138 / 126, 481^3-sized orders
+// 3, 4, 5 373, 346, 377 / - / 295, 281, 279; below the line that choice loses
+// (321^3 order 4 95.6 against 90.0, 261^3 order 2 71 against 55).
+static void sem_default_shape(phc_sem *h)
+{
+    h->ty = 8;
+    h->nj = 1;
+    h->chunk_i = -2;
+    if (h->nn < 600000) return;
+    h->ty = 4;
+    h->nj = 4;
+    h->chunk_i = -1;
+    if (12 * h->L.total < (int64_t)500e6) return;
+    double best = -1.0;
+    int ty = 4, m = 1;
+    for (int t : {8, 4}) {
+        h->ty = t;
+        const int TJ = 4 * t, ncol = sem_tiles_k(h, nullptr) * ((std::max(h->L.ny - 2, 1) + TJ - 1) / TJ);
+        const int cux = std::max(h->cus / 8, 1), slots = cux * sem_resident(h);
+        std::vector<int4> tab;
+        for (int s = 1; s <= 4; ++s) {
+            sem_build_sched(h->L.nx, ncol, slots, s, tab);
+            const double c = xcd_schedule_cost(tab, cux, TJ, 0.35 * 2 * h->p, 2 * h->p);
+            if (best < 0.0 || c < best) {
+                best = c;
+                ty = t;
+                m = s;
+            }
+        }
+    }
+    h->ty = ty;
+    h->chunk_i = -m;
 }
 
 static phc_status sem_prepare_sched(phc_sem *h)
@@ -972,13 +1262,8 @@ static phc_status sem_prepare_sched(phc_sem *h)
     const int ncol = sem_tiles_k(h, nullptr) * ((std::max(h->L.ny - 2, 1) + TJ - 1) / TJ);
     // blocks of this shape resident per CU (the table deals one round of
     // them per XCD at a time)
-    int per_cu = 1;
-    SemSepFn fn = sem_pick_sep(h->p, h->ty, h->nj, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32));
-    if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(fn),
-                                                            FD_TK * h->ty, 0) != hipSuccess || per_cu < 1)
-        per_cu = 1;
     std::vector<int4> tab;
-    sem_build_sched(h->L.nx, ncol, std::max(h->cus / 8, 1) * per_cu, -h->chunk_i, tab);
+    sem_build_sched(h->L.nx, ncol, std::max(h->cus / 8, 1) * sem_resident(h), -h->chunk_i, tab);
     PHC_HIP(hipStreamSynchronize(h->stream));  // queued launches may still read the old table
     sem_drop_graph(h);
     PHC_TRY(h->sched.alloc(sizeof(int4) * tab.size()));
@@ -1044,7 +1329,7 @@ static phc_status sem_launch(phc_sem *h, int i1, int i2, const float *rhs_next, 
             a.rec_blocks = (h->nrec + FD_TK * h->ty - 1) / (FD_TK * h->ty);
             nb += a.rec_blocks;
         }
-        SemSepFn fn = sem_pick_sep(h->p, h->ty, h->nj, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32));
+        SemSepFn fn = sem_handle_kernel(h);
         if (!fn) return fail(PHC_ERR_INVALID, "no separable kernel for p=%d", h->p);
         if (e0) PHC_HIP(hipEventRecord(e0, h->stream));
         hipLaunchKernelGGL(fn, dim3(nb), dim3(FD_TK, h->ty), 0, h->stream, a);
@@ -1332,18 +1617,6 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
         h->ty = p->block_waves ? p->block_waves : 16;
         h->nj = p->tile_j ? p->tile_j / h->ty : 1;
         h->chunk_i = p->chunk_i ? p->chunk_i : h->ny;
-        // where the caller gives no shape: 8 waves x 1 row on the per-XCD
-        // schedule of 4 plane ranges x 2 column bands.  One whole-axis march
-        // per 16-row column (a caller's shape without a chunk) left most CUs
-        // idle: 14 blocks at 101^3 order 2.  Best shape and chunk of each
-        // mesh / this default / before, us per step: 101^3 order 2
-        // 7.8 / 8.1 / 53.5, 321^3 order 4 88 / 88 / 201, 186 x 111 x 146
-        // order 5 16.6 / 17.6 / 78.8, 271 x 301 x 241 order 3 62.5 / 65.6 /
-        // 155, 130 x 142 x 116 order 1 12.4 / 14.2 / 66
-        if (!p->block_waves && !p->tile_j && !p->chunk_i) {
-            h->ty = 8;
-            h->chunk_i = -2;
-        }
         h->index64 = p->index64 ? 1 : 0;
         h->krem_mode = p->k_remainder;
         if (h->krem_mode < -1 || h->krem_mode > 1)
@@ -1351,7 +1624,7 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
         if (h->chunk_i < -4)
             return bail(fail(PHC_ERR_INVALID, "chunk_i %d: planes per chunk, or -1..-4 for the per-XCD schedule",
                              h->chunk_i));
-        if (!sem_pick_sep(P, h->ty, h->nj, true))
+        if (!sem_pick_sep(P, h->ty, h->nj, true, true))
             return bail(fail(PHC_ERR_INVALID, "no separable kernel for p=%d with %d waves x %d rows",
                              P, h->ty, h->nj));
         int dev = 0;
@@ -1359,6 +1632,7 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
             prop.multiProcessorCount > 0)
             h->cus = prop.multiProcessorCount;
+        if (!p->block_waves && !p->tile_j && !p->chunk_i) sem_default_shape(h);
     } else {
         const size_t bytes = sizeof(float) * (size_t)h->nn;
         if ((st = h->lev[0].alloc(bytes)) || (st = h->lev[1].alloc(bytes)) || (st = h->y.alloc(bytes)) ||
@@ -1709,7 +1983,7 @@ extern "C" phc_status phc_sem_autotune(phc_sem *h, int steps_per_trial, const ch
                     continue;
                 const bool chunk_ok = c > 0 || (c >= -4 && c <= -1);
                 if (!std::strcmp(tag, "sem") && ex == h->ex && ey == h->ey && ez == h->ez && pp == h->p &&
-                    km == h->krem_mode && a > 0 && b % a == 0 && chunk_ok && sem_pick_sep(h->p, a, b / a, true)) {
+                    km == h->krem_mode && a > 0 && b % a == 0 && chunk_ok && sem_pick_sep(h->p, a, b / a, true, true)) {
                     h->ty = a; h->nj = b / a; h->chunk_i = c;
                     hit = true;
                 }
@@ -1730,7 +2004,7 @@ extern "C" phc_status phc_sem_autotune(phc_sem *h, int steps_per_trial, const ch
         phc_status st = PHC_OK;
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
             st = fail(PHC_ERR_HIP, "event create failed");
-        const int shapes[][2] = {{16, 16}, {16, 32}, {8, 16}, {8, 8}, {4, 8}, {4, 4}};
+        const int shapes[][2] = {{16, 16}, {16, 32}, {8, 32}, {8, 16}, {8, 8}, {4, 16}, {4, 8}, {4, 4}};
         // chunk lengths that split the march axis evenly (n chunks, multiples
         // of 4 planes): a short last chunk would be mostly ring priming
         std::vector<int> chunks;
@@ -1744,7 +2018,7 @@ extern "C" phc_status phc_sem_autotune(phc_sem *h, int steps_per_trial, const ch
         int bty = h->ty, bnj = h->nj, bci = h->chunk_i;
         for (auto &sh : shapes) {
             if (st != PHC_OK) break;
-            if (!sem_pick_sep(h->p, sh[0], sh[1] / sh[0], true)) continue;
+            if (!sem_pick_sep(h->p, sh[0], sh[1] / sh[0], true, true)) continue;
             for (int c : chunks) {
                 h->ty = sh[0]; h->nj = sh[1] / sh[0]; h->chunk_i = c;
                 float ms = 0.f;
