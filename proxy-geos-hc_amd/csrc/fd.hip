@@ -1199,7 +1199,18 @@ extern "C" phc_status phc_fd_autotune(phc_fd *h, int steps_per_trial, const char
                         a.pnm1 = s0.as<float>();
                         if (s & 1) { a.pn = s0.as<float>(); a.pnm1 = s1.as<float>(); }
                         if (h->pml_on) a.pml_phi = s2.as<float>();
-                        st = fd_launch_step(h, a, false);
+                        // a learned layer's passes are part of the trial: they push
+                        // the levels out of the caches, and the shape that is best
+                        // for the march alone loses (264^3 with the layer, us per
+                        // step: 8 waves x 32 rows, split 1 105.3, 4 x 8, split 1
+                        // 102.9; alone 59.6 and 60.8)
+                        if (h->lb_on && lb_enqueue_correct(h->lbi, h->L, a.pn, a.pnm1, h->vp.as<float>(), h->stream,
+                                                           nullptr, nullptr) != hipSuccess)
+                            st = fail(PHC_ERR_HIP, "trial launch failed");
+                        if (st == PHC_OK) st = fd_launch_step(h, a, false);
+                        if (st == PHC_OK && h->lb_on &&
+                            lb_enqueue_apply(h->lbi, h->L, a.pnm1, h->stream) != hipSuccess)
+                            st = fail(PHC_ERR_HIP, "trial launch failed");
                     }
                     if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess ||
                                          hipEventSynchronize(e1) != hipSuccess ||
