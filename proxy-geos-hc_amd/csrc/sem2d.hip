@@ -747,9 +747,14 @@ phc_status phc_sem2d_create(const phc_sem_params *p, phc_sem2d **out)
     }
     h->index64 = p->index64 ? 1 : 0;
     if (!h->chunk && !h->index64) s2_plan_multi(h);
+    if (h->multi_t && (h->alt[0].alloc(bytes) || h->alt[1].alloc(bytes))) {
+        for (DevBuf &b : h->alt) b.release();
+        (void)hipGetLastError();
+        h->multi_t = 0;  // no room for the second pair of levels: single steps
+    }
     if (h->multi_t)
         for (DevBuf &b : h->alt)
-            if ((st = b.alloc(bytes)) || (st = fill_field(h->stream, b.as<float>(), h->L.total, 0.f))) return bail(st);
+            if ((st = fill_field(h->stream, b.as<float>(), h->L.total, 0.f))) return bail(st);
     *out = h;
     return PHC_OK;
 }
