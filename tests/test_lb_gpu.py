@@ -182,6 +182,33 @@ def test_learned_steps_match_cpu_emulation(gpu, oracle):
     assert np.array_equal(sol2.previous(), sol.previous())
 
 
+def test_autotune_with_the_layer_leaves_the_run_unchanged(gpu):
+    """The tuner's trials run the learned step on copies: the levels keep
+    their bits and the tuned shape (FP32 shapes agree bit for bit) gives the
+    same run as an untuned one."""
+    banner("autotune with a learned layer")
+    rng = np.random.default_rng(17)
+    s = thin_solver(gpu, 40, 60)
+    lb = gpu.LearnedBoundary(seed=2)
+    lb.set_params(rng.normal(0, 0.15, (lo.FACES, lo.NP)).astype(np.float32))
+    out = []
+    for tune in (False, True):
+        sol = gpu.FdSolver(s, arith=gpu.ARITH_FP32, init_value=0.0)
+        sol.set_learned_boundary(lb, halo=0.0)
+        sol.run(0, 30)
+        before = [sol.current(), sol.previous()]
+        if tune:
+            sol.autotune(steps_per_trial=2)
+            assert np.array_equal(sol.current(), before[0])
+            assert np.array_equal(sol.previous(), before[1])
+        sol.run(30, 20)
+        out.append([sol.current(), sol.previous()])
+        sol.close()
+    assert np.isfinite(out[0][0]).all() and np.max(np.abs(out[0][0])) > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def test_learned_steps_full_size_264(gpu, oracle):
     """The learned grid of the bench (256^3 region + 4-point layer = 264^3):
     from a smooth field that fills the layers, 3 learned steps (reference
