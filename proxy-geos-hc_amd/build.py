@@ -87,8 +87,8 @@ def build_host():
 
 
 def build_checks():
-    """Host check programs under tests/cpp/ (the drop-in classes' semantics),
-    linked against libphc.so; and, where the reference tree is present, the
+    """Host check programs under tests/cpp/ (the drop-in classes' semantics,
+    linked against libphc.so; the shim that refuses HIP calls); and, where the reference tree is present, the
     reference's own drivers built unchanged on the drop-in headers
     (oracle/ref_drivers.mk, outputs in oracle/_ref/)."""
     outs = []
@@ -98,6 +98,11 @@ def build_checks():
         _run(["g++", "-O2", "-std=c++17", "-Wall", "-I" + INCLUDE, "-I" + HOST, src, "-o", exe,
               "-L" + PKG, "-lphc", "-Wl,-rpath,$ORIGIN/../../proxy-geos-hc_amd"])
         outs.append(exe)
+    src = os.path.join(ROOT, "tests", "cpp", "hip_faults.c")
+    if os.path.exists(src):
+        lib = os.path.join(os.path.dirname(src), "libhip_faults.so")
+        _run(["gcc", "-O2", "-Wall", "-fPIC", "-shared", src, "-o", lib, "-ldl"])
+        outs.append(lib)
     ref = os.environ.get("PHC_REFERENCE", "/root/reference")
     if os.path.isdir(os.path.join(ref, "src", "fd")):
         _run(["make", "-s", "-B", "-f", os.path.join(ORACLE, "ref_drivers.mk"), "REF=" + ref])

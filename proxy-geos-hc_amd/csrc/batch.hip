@@ -600,13 +600,18 @@ phc_status phc_batch_run(phc_batch *h, int it0, int nsteps)
         if (h->traces.bytes < tbytes) PHC_TRY(h->traces.alloc(tbytes));
         if (h->nrec > 0 && h->rec.bytes < rbytes) PHC_TRY(h->rec.alloc(rbytes));
     }
-    hipLaunchKernelGGL(fd_batch_inject_kernel, dim3((h->nshots + 63) / 64), dim3(64), 0, h->stream,
-                       h->shots.as<ShotDesc>(), h->nshots, h->cur, it0, h->it0.as<int>());
-    PHC_HIP(hipGetLastError());
+    // changes the current level: launched once nothing but launches can fail
+    auto begin = [&]() -> phc_status {
+        hipLaunchKernelGGL(fd_batch_inject_kernel, dim3((h->nshots + 63) / 64), dim3(64), 0, h->stream,
+                           h->shots.as<ShotDesc>(), h->nshots, h->cur, it0, h->it0.as<int>());
+        PHC_HIP(hipGetLastError());
+        return PHC_OK;
+    };
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = batch_enqueue(h, nsteps, ev.data());
+        phc_status st = begin();
+        if (st == PHC_OK) st = batch_enqueue(h, nsteps, ev.data());
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -620,8 +625,10 @@ phc_status phc_batch_run(phc_batch *h, int it0, int nsteps)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        PHC_TRY(run_captured(h->stream, h->graph[h->cur], nsteps, h->pending, h->nrec,
-                             [&] { return batch_enqueue(h, nsteps, nullptr); }));
+        PHC_TRY(prepare_captured(h->stream, h->graph[h->cur], nsteps, h->pending, h->nrec,
+                                 [&] { return batch_enqueue(h, nsteps, nullptr); }));
+        PHC_TRY(begin());
+        PHC_HIP(hipGraphLaunch(h->graph[h->cur].exec, h->stream));
     }
     if (nsteps % 2) h->cur = 1 - h->cur;
     h->pending = h->sw > 0 ? 1 : 0;

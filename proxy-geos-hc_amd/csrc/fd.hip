@@ -871,14 +871,19 @@ phc_status phc_fd_run(phc_fd *h, int it0, int nsteps, int *cur)
         int nb = 0;
         PHC_TRY(fd_plan_launch(h, a, &nb));
     }
-    hipLaunchKernelGGL(fd_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
-                       h->lev[c0].as<float>(), h->vp.as<float>(), fd_off(h->L, h->xs, h->ys, h->zs),
-                       h->rhs.as<float>(), it0, nsteps, h->window.as<float>());
-    PHC_HIP(hipGetLastError());
+    // changes the current level: launched once nothing but launches can fail
+    auto begin = [&]() -> phc_status {
+        hipLaunchKernelGGL(fd_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
+                           h->lev[c0].as<float>(), h->vp.as<float>(), fd_off(h->L, h->xs, h->ys, h->zs),
+                           h->rhs.as<float>(), it0, nsteps, h->window.as<float>());
+        PHC_HIP(hipGetLastError());
+        return PHC_OK;
+    };
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = fd_enqueue_run(h, nsteps, c0, damp0, ev.data());
+        phc_status st = begin();
+        if (st == PHC_OK) st = fd_enqueue_run(h, nsteps, c0, damp0, ev.data());
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -892,8 +897,10 @@ phc_status phc_fd_run(phc_fd *h, int it0, int nsteps, int *cur)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        PHC_TRY(run_captured(h->stream, h->graph[c0], nsteps, damp0 ? 1 : 0, h->nrec,
-                             [&] { return fd_enqueue_run(h, nsteps, c0, damp0, nullptr); }));
+        PHC_TRY(prepare_captured(h->stream, h->graph[c0], nsteps, damp0 ? 1 : 0, h->nrec,
+                                 [&] { return fd_enqueue_run(h, nsteps, c0, damp0, nullptr); }));
+        PHC_TRY(begin());
+        PHC_HIP(hipGraphLaunch(h->graph[c0].exec, h->stream));
     }
     const int cend = (nsteps % 2 == 0) ? c0 : 1 - c0;
     h->pending[cend] = 0;

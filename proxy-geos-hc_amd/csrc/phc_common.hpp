@@ -84,10 +84,12 @@ struct RunGraph {
     }
 };
 
-// Launches the graph of an n-step chunk, capturing `enqueue` first when the
-// slot holds another one (key: whatever else the nodes depend on).
+// Has the slot hold the graph of an n-step chunk, capturing `enqueue` when it
+// holds another one (key: whatever else the nodes depend on).  Launches
+// nothing: a run changes its levels only after this has succeeded, so that one
+// that could not be captured can be called again.
 template <class F>
-phc_status run_captured(hipStream_t stream, RunGraph &g, int n, int key, int nrec, F enqueue)
+phc_status prepare_captured(hipStream_t stream, RunGraph &g, int n, int key, int nrec, F enqueue)
 {
     if (!(g.exec && g.n == n && g.key == key && g.nrec == nrec)) {
         if (g.exec) PHC_HIP(hipStreamSynchronize(stream));  // the old graph may still run
@@ -111,7 +113,6 @@ phc_status run_captured(hipStream_t stream, RunGraph &g, int n, int key, int nre
         g.key = key;
         g.nrec = nrec;
     }
-    PHC_HIP(hipGraphLaunch(g.exec, stream));
     return PHC_OK;
 }
 

@@ -1800,14 +1800,19 @@ phc_status phc_sem_run(phc_sem *h, int it0, int nsteps, int *i1p, int *i2p)
         sem_drop_graph(h);
         PHC_TRY(h->rec.alloc(sizeof(float) * (size_t)nsteps * h->nrec));
     }
-    hipLaunchKernelGGL(sem_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
-                       h->lev[i2].as<float>(), sem_off(h, h->src_node), h->inj_coef, h->rhs.as<float>(), it0, nsteps,
-                       h->window.as<float>());
-    PHC_HIP(hipGetLastError());
+    // changes the current level: launched once nothing but launches can fail
+    auto begin = [&]() -> phc_status {
+        hipLaunchKernelGGL(sem_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
+                           h->lev[i2].as<float>(), sem_off(h, h->src_node), h->inj_coef, h->rhs.as<float>(), it0, nsteps,
+                           h->window.as<float>());
+        PHC_HIP(hipGetLastError());
+        return PHC_OK;
+    };
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = sem_enqueue_run(h, nsteps, i1, i2, &ev);
+        phc_status st = begin();
+        if (st == PHC_OK) st = sem_enqueue_run(h, nsteps, i1, i2, &ev);
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -1821,8 +1826,10 @@ phc_status phc_sem_run(phc_sem *h, int it0, int nsteps, int *i1p, int *i2p)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        PHC_TRY(run_captured(h->stream, h->graph[i1], nsteps, 0, h->nrec,
-                             [&] { return sem_enqueue_run(h, nsteps, i1, i2, nullptr); }));
+        PHC_TRY(prepare_captured(h->stream, h->graph[i1], nsteps, 0, h->nrec,
+                                 [&] { return sem_enqueue_run(h, nsteps, i1, i2, nullptr); }));
+        PHC_TRY(begin());
+        PHC_HIP(hipGraphLaunch(h->graph[i1].exec, h->stream));
     }
     h->last_n = nsteps;
     h->last_nrec = h->nrec;

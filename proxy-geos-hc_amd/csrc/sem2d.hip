@@ -905,14 +905,19 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
         s2_drop_graph(h);
         PHC_TRY(h->rec.alloc(sizeof(float) * (size_t)nsteps * h->nrec));
     }
-    hipLaunchKernelGGL(sem2d_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
-                       h->lev[i2].as<float>(), s2_off(h, h->src_node), h->inj_coef, h->rhs.as<float>(), it0, nsteps,
-                       h->window.as<float>());
-    PHC_HIP(hipGetLastError());
+    // changes the current level: launched once nothing but launches can fail
+    auto begin = [&]() -> phc_status {
+        hipLaunchKernelGGL(sem2d_begin_run_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, h->stream,
+                           h->lev[i2].as<float>(), s2_off(h, h->src_node), h->inj_coef, h->rhs.as<float>(), it0, nsteps,
+                           h->window.as<float>());
+        PHC_HIP(hipGetLastError());
+        return PHC_OK;
+    };
     if (h->timing) {
         std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
-        phc_status st = s2_enqueue_run(h, nsteps, i1, i2, &ev);
+        phc_status st = begin();
+        if (st == PHC_OK) st = s2_enqueue_run(h, nsteps, i1, i2, &ev);
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
@@ -926,8 +931,11 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        PHC_TRY(run_captured(h->stream, h->graph[i1 + 2 * h->flipped], nsteps, 0, h->nrec,
-                             [&] { return s2_enqueue_run(h, nsteps, i1, i2, nullptr); }));
+        RunGraph &graph = h->graph[i1 + 2 * h->flipped];
+        PHC_TRY(prepare_captured(h->stream, graph, nsteps, 0, h->nrec,
+                                 [&] { return s2_enqueue_run(h, nsteps, i1, i2, nullptr); }));
+        PHC_TRY(begin());
+        PHC_HIP(hipGraphLaunch(graph.exec, h->stream));
         if (h->multi_t && h->nrec <= 2 * 64 * S2_MW && (nsteps / h->multi_t) % 2) {
             for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
             h->flipped ^= 1;
