@@ -680,6 +680,7 @@ phc_status phc_fd_create(const phc_fd_params *p, phc_fd **out)
         (st = fill_field(h->stream, h->vp.as<float>(), h->L.total, 0.f)) ||
         (st = write_field(h->stream, h->readback, h->vp.as<float>(), h->L, 0, 0, 0, p->vp)))
         return bail(st);
+    h->readback.release();  // not held by a handle whose fields are never read
     fd_axis_damping(h->nx, h->sw, h->alpha, h->hfx);
     fd_axis_damping(h->ny, h->sw, h->alpha, h->hfy);
     fd_axis_damping(h->nz, h->sw, h->alpha, h->hfz);

@@ -90,13 +90,14 @@ __host__ __device__ inline float face_damping(int sw, const float *fx, const flo
     return s;
 }
 
-// Four rows per block, 64 lanes along a row.
+// `rows` rows of the field from row r0 on (rows along k, planes after each
+// other); four rows per block, 64 lanes along a row.
 static __global__ void __launch_bounds__(256)
-pack_rows_kernel(const float *p, FdLayout L, int i0, int rows, int ly, int lz, FieldDamping d, float *out)
+pack_rows_kernel(const float *p, FdLayout L, int r0, int rows, int lx, int ly, int lz, FieldDamping d, float *out)
 {
     const int row = blockIdx.x * 4 + threadIdx.y, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz;
     if (row >= rows) return;
-    const int i = i0 + row / NY, j = row % NY - ly;
+    const int i = (r0 + row) / NY - lx, j = (r0 + row) % NY - ly;
     const float *src = p + fd_off(L, i, j, -lz);
     float *dst = out + (int64_t)row * NZ;
     const bool damp = d.sw > 0 && i >= 0 && i < L.nx && j >= 0 && j < L.ny;
@@ -109,11 +110,11 @@ pack_rows_kernel(const float *p, FdLayout L, int i0, int rows, int ly, int lz, F
 }
 
 static __global__ void __launch_bounds__(256)
-unpack_rows_kernel(float *p, FdLayout L, int i0, int rows, int ly, int lz, const float *in)
+unpack_rows_kernel(float *p, FdLayout L, int r0, int rows, int lx, int ly, int lz, const float *in)
 {
     const int row = blockIdx.x * 4 + threadIdx.y, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz;
     if (row >= rows) return;
-    float *dst = p + fd_off(L, i0 + row / NY, row % NY - ly, -lz);
+    float *dst = p + fd_off(L, (r0 + row) / NY - lx, (r0 + row) % NY - ly, -lz);
     const float *src = in + (int64_t)row * NZ;
     for (int c = threadIdx.x; c < NZ; c += 64) dst[c] = src[c];
 }
@@ -143,41 +144,38 @@ static bool ensure_scratch(DevBuf &b, size_t bytes)
     return false;
 }
 
+// Rows of NZ floats that a piece of at most READ_PIECE bytes holds.
+static int piece_rows(int rows, int NZ)
+{
+    return (int)std::min<size_t>(rows, std::max<size_t>(1, READ_PIECE / (sizeof(float) * (size_t)NZ)));
+}
+
 phc_status read_field(hipStream_t stream, DevBuf &scratch, const float *field, const FdLayout &L, int lx, int ly,
                       int lz, const FieldDamping &damping, const float *const host_factors[3], float *host)
 {
-    const int NX = L.nx + 2 * lx, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz;
-    const size_t plane = sizeof(float) * (size_t)NY * NZ;
-    // floats from a plane's first value to its last
-    const int64_t span = (int64_t)(NY - 1) * L.pitch_k + NZ;
-    const int per = (int)std::min<size_t>(NX, std::max<size_t>(1, READ_PIECE / plane));
-    if (!ensure_scratch(scratch, plane * per)) {
+    const int NX = L.nx + 2 * lx, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz, rows = NX * NY;
+    const size_t row = sizeof(float) * (size_t)NZ;
+    const int per = piece_rows(rows, NZ);
+    if (!ensure_scratch(scratch, row * per)) {
         PHC_HIP(hipStreamSynchronize(stream));
-        std::vector<float> buf((size_t)((per - 1) * L.pitch_j + span));
-        for (int i0 = 0; i0 < NX; i0 += per) {
-            const int n = std::min(per, NX - i0);
-            PHC_HIP(hipMemcpy(buf.data(), field + fd_off(L, i0 - lx, -ly, -lz),
-                              sizeof(float) * (size_t)((n - 1) * L.pitch_j + span), hipMemcpyDeviceToHost));
-            for (int i = i0; i < i0 + n; ++i)
-                for (int j = 0; j < NY; ++j) {
-                    float *dst = host + ((int64_t)i * NY + j) * NZ;
-                    const float *src = buf.data() + (i - i0) * L.pitch_j + j * L.pitch_k;
-                    std::copy(src, src + NZ, dst);
-                    if (damping.sw > 0 && i >= lx && i < lx + L.nx && j >= ly && j < ly + L.ny)
-                        for (int k = 0; k < L.nz; ++k)
-                            dst[k + lz] *= face_damping(damping.sw, host_factors[0], host_factors[1],
-                                                        host_factors[2], L, i - lx, j - ly, k);
-                }
+        for (int i = 0; i < NX; ++i) {
+            float *plane = host + (int64_t)i * NY * NZ;
+            PHC_HIP(hipMemcpy2D(plane, row, field + fd_off(L, i - lx, -ly, -lz), sizeof(float) * L.pitch_k, row, NY,
+                                hipMemcpyDeviceToHost));
+            if (damping.sw <= 0 || i < lx || i >= lx + L.nx) continue;
+            for (int j = 0; j < L.ny; ++j)
+                for (int k = 0; k < L.nz; ++k)
+                    plane[(int64_t)(j + ly) * NZ + k + lz] *= face_damping(
+                        damping.sw, host_factors[0], host_factors[1], host_factors[2], L, i - lx, j, k);
         }
         return PHC_OK;
     }
-    for (int i = 0; i < NX; i += per) {
-        const int rows = std::min(per, NX - i) * NY;
-        hipLaunchKernelGGL(pack_rows_kernel, dim3((rows + 3) / 4), dim3(64, 4), 0, stream, field, L, i - lx, rows, ly,
-                           lz, damping, scratch.as<float>());
+    for (int r0 = 0; r0 < rows; r0 += per) {
+        const int n = std::min(per, rows - r0);
+        hipLaunchKernelGGL(pack_rows_kernel, dim3((n + 3) / 4), dim3(64, 4), 0, stream, field, L, r0, n, lx, ly, lz,
+                           damping, scratch.as<float>());
         PHC_HIP(hipGetLastError());
-        PHC_HIP(hipMemcpyAsync(host + (int64_t)i * NY * NZ, scratch.ptr, sizeof(float) * (size_t)rows * NZ,
-                               hipMemcpyDeviceToHost, stream));
+        PHC_HIP(hipMemcpyAsync(host + (int64_t)r0 * NZ, scratch.ptr, row * n, hipMemcpyDeviceToHost, stream));
     }
     PHC_HIP(hipStreamSynchronize(stream));
     return PHC_OK;
@@ -186,33 +184,24 @@ phc_status read_field(hipStream_t stream, DevBuf &scratch, const float *field, c
 phc_status write_field(hipStream_t stream, DevBuf &scratch, float *field, const FdLayout &L, int lx, int ly, int lz,
                        const float *host)
 {
-    const int NX = L.nx + 2 * lx, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz;
-    const size_t plane = sizeof(float) * (size_t)NY * NZ;
-    const int64_t span = (int64_t)(NY - 1) * L.pitch_k + NZ;
-    const int per = (int)std::min<size_t>(NX, std::max<size_t>(1, READ_PIECE / plane));
-    PHC_HIP(hipStreamSynchronize(stream));
-    const bool packed = ensure_scratch(scratch, plane * per);
-    std::vector<float> buf(packed ? 0 : (size_t)((per - 1) * L.pitch_j + span));
-    for (int i0 = 0; i0 < NX; i0 += per) {
-        const int n = std::min(per, NX - i0);
-        const float *src = host + (int64_t)i0 * NY * NZ;
-        if (packed) {
-            PHC_HIP(hipMemcpy(scratch.ptr, src, plane * n, hipMemcpyHostToDevice));
-            hipLaunchKernelGGL(unpack_rows_kernel, dim3((n * NY + 3) / 4), dim3(64, 4), 0, stream, field, L, i0 - lx,
-                               n * NY, ly, lz, scratch.as<float>());
-            PHC_HIP(hipGetLastError());
-            PHC_HIP(hipStreamSynchronize(stream));  // the next piece overwrites the scratch
-            continue;
-        }
-        float *dev = field + fd_off(L, i0 - lx, -ly, -lz);
-        const size_t bytes = sizeof(float) * (size_t)((n - 1) * L.pitch_j + span);
-        PHC_HIP(hipMemcpy(buf.data(), dev, bytes, hipMemcpyDeviceToHost));
-        for (int i = 0; i < n; ++i)
-            for (int j = 0; j < NY; ++j)
-                std::copy(src + ((int64_t)i * NY + j) * NZ, src + ((int64_t)i * NY + j + 1) * NZ,
-                          buf.data() + i * L.pitch_j + j * L.pitch_k);
-        PHC_HIP(hipMemcpy(dev, buf.data(), bytes, hipMemcpyHostToDevice));
+    const int NX = L.nx + 2 * lx, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz, rows = NX * NY;
+    const size_t row = sizeof(float) * (size_t)NZ;
+    const int per = piece_rows(rows, NZ);
+    if (!ensure_scratch(scratch, row * per)) {
+        PHC_HIP(hipStreamSynchronize(stream));
+        for (int i = 0; i < NX; ++i)
+            PHC_HIP(hipMemcpy2D(field + fd_off(L, i - lx, -ly, -lz), sizeof(float) * L.pitch_k,
+                                host + (int64_t)i * NY * NZ, row, row, NY, hipMemcpyHostToDevice));
+        return PHC_OK;
     }
+    for (int r0 = 0; r0 < rows; r0 += per) {
+        const int n = std::min(per, rows - r0);
+        PHC_HIP(hipMemcpyAsync(scratch.ptr, host + (int64_t)r0 * NZ, row * n, hipMemcpyHostToDevice, stream));
+        hipLaunchKernelGGL(unpack_rows_kernel, dim3((n + 3) / 4), dim3(64, 4), 0, stream, field, L, r0, n, lx, ly, lz,
+                           scratch.as<float>());
+        PHC_HIP(hipGetLastError());
+    }
+    PHC_HIP(hipStreamSynchronize(stream));
     return PHC_OK;
 }
 
@@ -230,16 +219,16 @@ phc_status read_slice_xz(hipStream_t stream, DevBuf &scratch, const float *field
     const size_t bytes = sizeof(float) * (size_t)L.nx * L.nz;
     if (!ensure_scratch(scratch, bytes)) {
         PHC_HIP(hipStreamSynchronize(stream));
-        std::vector<float> row((size_t)L.nz);
-        for (int i = 0; i < L.nx; ++i) {
-            PHC_HIP(hipMemcpy(row.data(), field + fd_off(L, i, j, 0), sizeof(float) * L.nz, hipMemcpyDeviceToHost));
+        std::vector<float> buf((size_t)L.nx * L.nz);
+        PHC_HIP(hipMemcpy2D(buf.data(), sizeof(float) * L.nz, field + fd_off(L, 0, j, 0), sizeof(float) * L.pitch_j,
+                            sizeof(float) * L.nz, L.nx, hipMemcpyDeviceToHost));
+        for (int i = 0; i < L.nx; ++i)
             for (int k = 0; k < L.nz; ++k) {
-                float v = row[k];
+                float v = buf[(size_t)i * L.nz + k];
                 if (damping.sw > 0)
                     v *= face_damping(damping.sw, host_factors[0], host_factors[1], host_factors[2], L, i, j, k);
                 host[(int64_t)k * L.nx + i] = v;
             }
-        }
         return PHC_OK;
     }
     hipLaunchKernelGGL(slice_xz_kernel, dim3((L.nz + 63) / 64, (L.nx + 3) / 4), dim3(64, 4), 0, stream, field, L, j,

@@ -1597,6 +1597,7 @@ phc_status phc_sem_create(const phc_sem_params *p, phc_sem **out)
                     Qn[n] = (float)(dt2 * ax.Wg[ix] * az.Wg[iz] * ay.Wg[iy] / M[n]);
                 }
         if ((st = sem_put(h, h->qf, Qn.data()))) return bail(st);
+        h->readback.release();  // not held by a handle whose fields are never read
         // stencil rows by index mod p (identical on every row of an axis with
         // the same residue: the mesh is uniform along each axis)
         std::memset(h->cx, 0, sizeof(h->cx));

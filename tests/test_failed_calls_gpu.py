@@ -1,8 +1,11 @@
-"""Runs whose graph cannot be instantiated: the call returns an error and the
-state is as before it, so the same call succeeds afterwards with the values of
-a run that never failed.  The failures are refusals by a shim between
-libphc.so and the HIP runtime (tests/cpp/hip_faults.c), which has to be loaded
-first: each test runs in a process of its own."""
+"""What calls do when the HIP runtime refuses them something, and how much
+device memory they ask for.  Runs whose graph cannot be instantiated: the call
+returns an error and the state is as before it, so the same call succeeds
+afterwards with the values of a run that never failed.  Fields read and written
+without device memory for the packing: the same values.  The scratch memory of
+the packing: bounded, and none held before a field is read.  A shim between
+libphc.so and the HIP runtime (tests/cpp/hip_faults.c) refuses and counts; it
+has to be loaded first, so each test runs in a process of its own."""
 import ctypes
 import os
 import subprocess
@@ -64,7 +67,68 @@ def check_failed_run(phc, faults, make):
     assert np.abs(state(a)[0]).max() > 0
 
 
+def fd_fields(phc, faults, dims, lh, refuse):
+    """Set, step (the previous level then owes its sponge product), read."""
+    nx, ny, nz = dims
+    sol = phc.FdSolver(phc.FdSetup(nx, ny, nz, L=lh[0], ly=lh[1], lz=lh[2], sponge_width=2, f0=25.0, nsamples=10))
+    rng = np.random.default_rng(nx)
+    faults.hip_faults_set(0 if refuse else NEVER, 0)
+    shape = [n + 2 * l for n, l in zip(dims, lh)]
+    for level in (0, 1):
+        sol.set_field(level, rng.normal(0, 1, shape).astype(np.float32))
+    out = [sol.field(0), sol.field(1)]
+    refused = faults.hip_faults_refused()
+    faults.hip_faults_set(NEVER, 0)  # the first step uploads its schedule
+    sol.step(0)
+    faults.hip_faults_set(0 if refuse else NEVER, 0)
+    out += [sol.field(0), sol.field(1)] + [sol.slice_xz(lv, j) for lv in (0, 1) for j in (0, ny - 1)]
+    refused += faults.hip_faults_refused()
+    faults.hip_faults_set(NEVER, 0)
+    sol.close()
+    return out, refused
+
+
+def check_no_scratch(phc, faults):
+    for dims, lh in (((5, 7, 3), (4, 4, 4)), ((60, 50, 66), (4, 3, 2)), ((6, 11, 130), (1, 4, 2)), ((3, 5, 65), (6, 6, 6))):
+        (want, _), (got, refused) = (fd_fields(phc, faults, dims, lh, r) for r in (False, True))
+        assert refused >= 10  # every read and write went without scratch
+        for a, b in zip(want, got):
+            assert np.array_equal(a, b), (dims, lh)
+    rng = np.random.default_rng(3)
+    for make in (sem, sem2d):
+        sol = make(phc)
+        f = [rng.normal(0, 1, sol.nn).astype(np.float32) for _ in range(2)]
+        faults.hip_faults_set(0, 0)
+        for level in (0, 1):
+            sol.set_field(level, f[level])
+        for level in (0, 1):
+            assert np.array_equal(sol.field(level), f[level])
+        assert faults.hip_faults_refused() >= 2
+        faults.hip_faults_set(NEVER, 0)
+        sol.close()
+
+
+def check_scratch_size(phc, faults):
+    """Fields of 84 and 71 MB (a 2D field is one plane)."""
+    piece = 32 << 20
+    big = (phc.FdSolver(phc.FdSetup(268, 268, 268, sponge_width=0, nsamples=2)),
+           phc.Sem2dSolver(ex=2100, ez=2100, lx=42e3, lz=42e3, order=2, nsamples=2, src_element=50))
+    for sol in big:
+        shape = sol.nn if hasattr(sol, "nn") else (276, 276, 276)
+        f = np.random.default_rng(2).normal(0, 1, shape).astype(np.float32)
+        assert f.nbytes > 64 << 20
+        held = faults.hip_faults_live()
+        faults.hip_faults_set(NEVER, 0)
+        sol.set_field(1, f)
+        assert np.array_equal(sol.field(1), f)
+        assert 0 < faults.hip_faults_peak() <= piece
+        assert 0 < faults.hip_faults_live() - held <= piece
+        sol.close()
+
+
 CASES = {
+    "no_scratch": check_no_scratch,
+    "scratch_size": check_scratch_size,
     "failed_run_fd": lambda phc, f: check_failed_run(phc, f, fd),
     "failed_run_sem": lambda phc, f: check_failed_run(phc, f, sem),
     "failed_run_sem2d": lambda phc, f: check_failed_run(phc, f, sem2d),

@@ -1,6 +1,6 @@
 """Fields read back through the device-packed path: rows shorter, equal and
 longer than a wavefront, unequal half widths, a level that owes its sponge
-product, fields of several 64 MiB pieces, and the x-z slice, against the same
+product, fields of several 32 MiB pieces, and the x-z slice, against the same
 values through single-point reads and the field itself."""
 import numpy as np
 import pytest
@@ -34,7 +34,7 @@ def test_set_get_round_trip_and_points(gpu, dims, lh):
 
 
 def test_field_of_several_pieces(gpu):
-    """276^3 values with the halo: 84 MB, two pieces."""
+    """276^3 values with the halo: 84 MB, three pieces."""
     print("\n[readback] pieces", flush=True)
     s = gpu.FdSetup(268, 268, 268, sponge_width=0, nsamples=2)
     sol = gpu.FdSolver(s)
