@@ -125,15 +125,16 @@ static __global__ void __launch_bounds__(256) fill_field_kernel(float *p, int64_
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += stride) p[t] = v;
 }
 
-// 64 points along k by 4 along i per block: reads run along k.
+// Rows k0 .. k0 + n - 1 of the slice; 64 points along k by 4 along i per block:
+// reads run along k.
 static __global__ void __launch_bounds__(256)
-slice_xz_kernel(const float *p, FdLayout L, int j, FieldDamping d, float *out)
+slice_xz_kernel(const float *p, FdLayout L, int j, int k0, int n, FieldDamping d, float *out)
 {
-    const int k = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y;
-    if (k >= L.nz || i >= L.nx) return;
+    const int r = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y, k = k0 + r;
+    if (r >= n || i >= L.nx) return;
     float v = p[fd_off(L, i, j, k)];
     if (d.sw > 0) v *= face_damping(d.sw, d.fx, d.fy, d.fz, L, i, j, k);
-    out[(int64_t)k * L.nx + i] = v;
+    out[(int64_t)r * L.nx + i] = v;
 }
 
 static bool ensure_scratch(DevBuf &b, size_t bytes)
@@ -216,8 +217,9 @@ phc_status fill_field(hipStream_t stream, float *field, int64_t n, float value)
 phc_status read_slice_xz(hipStream_t stream, DevBuf &scratch, const float *field, const FdLayout &L, int j,
                          const FieldDamping &damping, const float *const host_factors[3], float *host)
 {
-    const size_t bytes = sizeof(float) * (size_t)L.nx * L.nz;
-    if (!ensure_scratch(scratch, bytes)) {
+    const size_t row = sizeof(float) * (size_t)L.nx;
+    const int per = piece_rows(L.nz, L.nx);
+    if (!ensure_scratch(scratch, row * per)) {
         PHC_HIP(hipStreamSynchronize(stream));
         std::vector<float> buf((size_t)L.nx * L.nz);
         PHC_HIP(hipMemcpy2D(buf.data(), sizeof(float) * L.nz, field + fd_off(L, 0, j, 0), sizeof(float) * L.pitch_j,
@@ -231,10 +233,13 @@ phc_status read_slice_xz(hipStream_t stream, DevBuf &scratch, const float *field
             }
         return PHC_OK;
     }
-    hipLaunchKernelGGL(slice_xz_kernel, dim3((L.nz + 63) / 64, (L.nx + 3) / 4), dim3(64, 4), 0, stream, field, L, j,
-                       damping, scratch.as<float>());
-    PHC_HIP(hipGetLastError());
-    PHC_HIP(hipMemcpyAsync(host, scratch.ptr, bytes, hipMemcpyDeviceToHost, stream));
+    for (int k0 = 0; k0 < L.nz; k0 += per) {
+        const int n = std::min(per, L.nz - k0);
+        hipLaunchKernelGGL(slice_xz_kernel, dim3((n + 63) / 64, (L.nx + 3) / 4), dim3(64, 4), 0, stream, field, L, j,
+                           k0, n, damping, scratch.as<float>());
+        PHC_HIP(hipGetLastError());
+        PHC_HIP(hipMemcpyAsync(host + (int64_t)k0 * L.nx, scratch.ptr, row * n, hipMemcpyDeviceToHost, stream));
+    }
     PHC_HIP(hipStreamSynchronize(stream));
     return PHC_OK;
 }

@@ -35,7 +35,8 @@ phc_status write_field(hipStream_t stream, DevBuf &scratch, float *field, const 
 phc_status fill_field(hipStream_t stream, float *field, int64_t n, float value);
 
 // The slice host[k * nx + i] = field(i, j, k) (interior, damping applied),
-// gathered on the device: 0.05 ms at 150^3, 2.0 ms through the whole field.
+// gathered on the device in pieces of at most READ_PIECE bytes: 0.05 ms at
+// 150^3, 2.0 ms through the whole field.
 phc_status read_slice_xz(hipStream_t stream, DevBuf &scratch, const float *field, const FdLayout &L, int j,
                          const FieldDamping &damping, const float *const host_factors[3], float *host);
 

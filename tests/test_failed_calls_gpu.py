@@ -109,7 +109,7 @@ def check_no_scratch(phc, faults):
 
 
 def check_scratch_size(phc, faults):
-    """Fields of 84 and 71 MB (a 2D field is one plane)."""
+    """Fields of 84 and 71 MB (a 2D field is one plane), a slice of 35 MB."""
     piece = 32 << 20
     big = (phc.FdSolver(phc.FdSetup(268, 268, 268, sponge_width=0, nsamples=2)),
            phc.Sem2dSolver(ex=2100, ez=2100, lx=42e3, lz=42e3, order=2, nsamples=2, src_element=50))
@@ -124,6 +124,11 @@ def check_scratch_size(phc, faults):
         assert 0 < faults.hip_faults_peak() <= piece
         assert 0 < faults.hip_faults_live() - held <= piece
         sol.close()
+    sol = phc.FdSolver(phc.FdSetup(2600, 1, 3400, L=1, sponge_width=0, nsamples=2, model="homogeneous"))
+    faults.hip_faults_set(NEVER, 0)
+    sol.slice_xz(0, 0)
+    assert 0 < faults.hip_faults_peak() <= piece
+    sol.close()
 
 
 CASES = {

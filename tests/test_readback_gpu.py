@@ -55,3 +55,16 @@ def test_sem_fields(gpu):
             sol.set_field(level, f)
             assert np.array_equal(sol.field(level), f)
         sol.close()
+
+
+def test_slice_of_a_long_axis(gpu):
+    """More points along x than 4 x 65536, and a slice of two pieces."""
+    print("\n[readback] long slices", flush=True)
+    rng = np.random.default_rng(4)
+    for nx, nz in ((262500, 2), (2600, 3400)):
+        s = gpu.FdSetup(nx, 1, nz, L=1, sponge_width=0, nsamples=2, model="homogeneous")
+        sol = gpu.FdSolver(s)
+        f = rng.normal(0, 1, (nx + 2, 3, nz + 2)).astype(np.float32)
+        sol.set_field(0, f)
+        assert np.array_equal(sol.slice_xz(0, 0), f[1:-1, 1, 1:-1].T)
+        sol.close()
