@@ -161,7 +161,8 @@ phc_status phc_fd_synchronize(phc_fd *h);
  * shapes, FDTDmacros.hpp:57-61): times each block shape and chunk length on
  * scratch copies of the levels (the state is not advanced), keeps the fastest
  * and reports it.  cache_path (may be NULL) is a text cache keyed by grid,
- * radius and arithmetic; a cached entry is used without timing. */
+ * radius, arithmetic, PML, k_remainder and whether a learned boundary is
+ * attached; a cached entry is used without timing. */
 phc_status phc_fd_autotune(phc_fd *h, int steps_per_trial, const char *cache_path, int *tile_j,
                            int *block_waves, int *chunk_i);
 

@@ -1125,10 +1125,14 @@ phc_status phc_fd_synchronize(phc_fd *h)
 // handle's grid (on scratch copies of the two levels, so the simulation state
 // is untouched) and keeps the fastest; with k_remainder 0 it also times the
 // last partial k tile as a tile (-1) and keeps the faster of the two.  Results
-// are cached in a text file, one line per (grid, radius, arithmetic, step
-// variant, requested k mode):
-// "fd nx ny nz R arith pml kmode waves tile_j chunk_i kmode_used ms".
+// are cached in a text file, one line per (learned layer attached or not, grid,
+// radius, arithmetic, PML or not, requested k mode):
+// "fd nx ny nz R arith pml kmode waves tile_j chunk_i kmode_used ms", with the
+// tag "fdlb" for a handle with a learned layer: its trials time other work, and
+// another shape wins (264^3: the figures in the trial loop below).
 namespace phc {
+
+static const char *fd_tune_tag(const phc_fd *h) { return h->lb_on ? "fdlb" : "fd"; }
 
 static bool fd_tune_lookup(const char *path, const phc_fd *h, int *ty, int *tj, int *ci, int *km_used)
 {
@@ -1144,7 +1148,7 @@ static bool fd_tune_lookup(const char *path, const phc_fd *h, int *ty, int *tj, 
         if (std::sscanf(line, "%7s %d %d %d %d %d %d %d %d %d %d %d %lf", tag, &nx, &ny, &nz, &R, &ar, &pml, &km, &a,
                         &b, &c, &ku, &ms) != 13)
             continue;
-        if (!std::strcmp(tag, "fd") && nx == h->nx && ny == h->ny && nz == h->nz && R == h->R && ar == h->arith &&
+        if (!std::strcmp(tag, fd_tune_tag(h)) && nx == h->nx && ny == h->ny && nz == h->nz && R == h->R && ar == h->arith &&
             pml == h->pml_on && km == h->krem_mode && a > 0 && b % a == 0 && c >= -4 && c != 0 && ku >= -1 &&
             ku <= 1 &&
             (ku == km || km == 0) && fd_pick_kernel(h->R, a, b / a, h->arith, true, false)) {
@@ -1238,8 +1242,8 @@ extern "C" phc_status phc_fd_autotune(phc_fd *h, int steps_per_trial, const char
         if (cache_path) {
             FILE *f = std::fopen(cache_path, "a");
             if (f) {
-                std::fprintf(f, "fd %d %d %d %d %d %d %d %d %d %d %d %.5f\n", h->nx, h->ny, h->nz, h->R,
-                             h->arith, h->pml_on, h->krem_mode, bty, bty * bnj, bci, bku, best / steps_per_trial);
+                std::fprintf(f, "%s %d %d %d %d %d %d %d %d %d %d %d %.5f\n", fd_tune_tag(h), h->nx, h->ny, h->nz,
+                             h->R, h->arith, h->pml_on, h->krem_mode, bty, bty * bnj, bci, bku, best / steps_per_trial);
                 std::fclose(f);
             }
         }

@@ -209,6 +209,34 @@ def test_autotune_with_the_layer_leaves_the_run_unchanged(gpu):
         assert np.array_equal(a, b)
 
 
+def test_tuning_cache_keeps_learned_and_plain_shapes_apart(gpu, tmp_path):
+    """A handle with a learned layer times other work than one without: neither
+    takes the other's cached shape, both take their own, and a cached shape
+    follows the layer as it is attached and detached."""
+    banner("tuning cache with and without a learned layer")
+    cache = tmp_path / "tune.txt"
+    plain, learned = "fd 60 60 60 4 1 0 0 8 16 7 0 0.01\n", "fdlb 60 60 60 4 1 0 0 4 16 5 -1 0.02\n"
+    s = thin_solver(gpu, 60, 10)
+    lb = gpu.LearnedBoundary(seed=2)
+    for text, tuned in ((plain, True), (learned, False)):
+        cache.write_text(text)
+        sol = gpu.FdSolver(s, arith=gpu.ARITH_FP32, init_value=0.0)
+        if tuned:
+            sol.set_learned_boundary(lb, halo=0.0)
+        sol.autotune(steps_per_trial=2, cache_path=str(cache))
+        lines = cache.read_text().splitlines()
+        assert len(lines) == 2 and {l.split()[0] for l in lines} == {"fd", "fdlb"}  # the other's line was no hit
+        sol.close()
+    cache.write_text(plain + learned)
+    sol = gpu.FdSolver(s, arith=gpu.ARITH_FP32, init_value=0.0)
+    assert sol.autotune(steps_per_trial=2, cache_path=str(cache)) == (16, 8, 7)
+    sol.set_learned_boundary(lb, halo=0.0)
+    assert sol.autotune(steps_per_trial=2, cache_path=str(cache)) == (16, 4, 5)
+    sol.set_learned_boundary(None)
+    assert sol.autotune(steps_per_trial=2, cache_path=str(cache)) == (16, 8, 7)
+    sol.close()
+
+
 def test_learned_steps_full_size_264(gpu, oracle):
     """The learned grid of the bench (256^3 region + 4-point layer = 264^3):
     from a smooth field that fills the layers, 3 learned steps (reference
