@@ -343,6 +343,8 @@ phc_status phc_sem2d_set_field(phc_sem2d *h, int level, const float *host);
 phc_status phc_sem2d_get_mass(phc_sem2d *h, float *mass, float *boundary);
 phc_status phc_sem2d_check_finite(phc_sem2d *h, int level);
 phc_status phc_sem2d_set_timing(phc_sem2d *h, int enable);
+/* mean duration of the last timed run's step launches, per step (a launch may
+ * hold several steps) */
 phc_status phc_sem2d_last_run_kernel_ms(phc_sem2d *h, double *ms_per_step);
 phc_status phc_sem2d_synchronize(phc_sem2d *h);
 /* Autotuner (no reference counterpart): rows per wavefront, timed on scratch

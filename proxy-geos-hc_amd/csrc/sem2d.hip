@@ -825,6 +825,13 @@ phc_status phc_sem2d_set_source(phc_sem2d *h, int src_element, int nsamples, con
     return PHC_OK;
 }
 
+// Launches of several steps at the start of a run (more receivers than such a
+// launch samples: none).
+static int s2_multi_launches(const phc_sem2d *h, int nsteps)
+{
+    return h->multi_t && h->nrec <= 2 * 64 * S2_MW ? nsteps / h->multi_t : 0;
+}
+
 // A run's steps on h->stream (sem2d_begin_run_kernel has filled the window and
 // injected its first sample), each step's launch sampling the receivers of
 // the one before.  Names no time sample, so that a captured run serves every
@@ -832,10 +839,11 @@ phc_status phc_sem2d_set_source(phc_sem2d *h, int src_element, int nsamples, con
 // Where a mesh takes several steps per launch, whole launches come first
 // (reading lev and writing alt, or the reverse), single steps after them; the
 // levels end in lev, or in alt after an odd number of launches.
-static phc_status s2_enqueue_run(phc_sem2d *h, int nsteps, int i1, int i2, std::vector<hipEvent_t> *ev)
+// With `ev`, events 2n and 2n + 1 bracket the n-th step launch (timing mode).
+static phc_status s2_enqueue_run(phc_sem2d *h, int nsteps, int i1, int i2, hipEvent_t *ev)
 {
     const float *win = h->window.as<float>();
-    const int t = ev || h->nrec > 2 * 64 * S2_MW ? 0 : h->multi_t, launches = t ? nsteps / t : 0;
+    const int t = h->multi_t, launches = s2_multi_launches(h, nsteps);
     for (int l = 0; l < launches; ++l) {
         Sem2dMultiArgs m;
         s2_fill_args(h, m.s, i1, i2);
@@ -856,21 +864,25 @@ static phc_status s2_enqueue_run(phc_sem2d *h, int nsteps, int i1, int i2, std::
         m.s.rec_stride = nsteps;
         const int tx = 64 - 2 * h->p * t, tz = S2_MW * h->multi_rz - 2 * h->p * t;
         m.tiles_x = (h->nx + tx - 1) / tx;
+        if (ev) PHC_HIP(hipEventRecord(ev[2 * l], h->stream));
         hipLaunchKernelGGL(sem2d_pick_multi(h->p, t, h->multi_rz), dim3(m.tiles_x * ((h->nz + tz - 1) / tz)),
                            dim3(64 * S2_MW), 0, h->stream, m);
         PHC_HIP(hipGetLastError());
+        if (ev) PHC_HIP(hipEventRecord(ev[2 * l + 1], h->stream));
     }
+    if (ev) ev += 2 * launches;
     if (launches & 1)
         for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
     phc_status st = PHC_OK;
-    for (int s = launches * t; s < nsteps && st == PHC_OK; ++s) {
+    const int single = launches * t;  // first step of a launch of its own
+    for (int s = single; s < nsteps && st == PHC_OK; ++s) {
         // the launches above have sampled their own steps
-        const int rs = h->nrec > 0 && s > launches * t ? s - 1 : -1;
+        const int rs = h->nrec > 0 && s > single ? s - 1 : -1;
         st = s2_launch(h, i1, i2, s + 1 < nsteps ? win + s + 1 : nullptr, h->trace.as<float>() + s,
-                       ev ? (*ev)[2 * s] : nullptr, ev ? (*ev)[2 * s + 1] : nullptr, rs, nsteps);
+                       ev ? ev[2 * (s - single)] : nullptr, ev ? ev[2 * (s - single) + 1] : nullptr, rs, nsteps);
         std::swap(i1, i2);
     }
-    if (st == PHC_OK && h->nrec > 0 && launches * t < nsteps) {
+    if (st == PHC_OK && h->nrec > 0 && single < nsteps) {
         hipLaunchKernelGGL(sem2d_sample_kernel, dim3((h->nrec + 255) / 256), dim3(256), 0, h->stream,
                            h->lev[i2].as<float>(), h->recoff.as<int64_t>(), h->nrec, h->rec.as<float>(), nsteps,
                            nsteps - 1, s2_off(h, h->src_node), h->trace.as<float>());
@@ -913,17 +925,19 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
         PHC_HIP(hipGetLastError());
         return PHC_OK;
     };
+    const int multi = s2_multi_launches(h, nsteps);
     if (h->timing) {
-        std::vector<hipEvent_t> ev(2 * (size_t)nsteps);
+        const int launches = multi ? multi + nsteps % h->multi_t : nsteps;
+        std::vector<hipEvent_t> ev(2 * (size_t)launches);
         for (auto &e : ev) PHC_HIP(hipEventCreate(&e));
         phc_status st = begin();
-        if (st == PHC_OK) st = s2_enqueue_run(h, nsteps, i1, i2, &ev);
+        if (st == PHC_OK) st = s2_enqueue_run(h, nsteps, i1, i2, ev.data());
         if (st == PHC_OK) {
             PHC_HIP(hipStreamSynchronize(h->stream));
             double tot = 0.0;
-            for (int s = 0; s < nsteps; ++s) {
+            for (int l = 0; l < launches; ++l) {
                 float ms = 0.f;
-                PHC_HIP(hipEventElapsedTime(&ms, ev[2 * s], ev[2 * s + 1]));
+                PHC_HIP(hipEventElapsedTime(&ms, ev[2 * l], ev[2 * l + 1]));
                 tot += ms;
             }
             h->last_ms = tot / nsteps;
@@ -936,10 +950,10 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
                                  [&] { return s2_enqueue_run(h, nsteps, i1, i2, nullptr); }));
         PHC_TRY(begin());
         PHC_HIP(hipGraphLaunch(graph.exec, h->stream));
-        if (h->multi_t && h->nrec <= 2 * 64 * S2_MW && (nsteps / h->multi_t) % 2) {
-            for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
-            h->flipped ^= 1;
-        }
+    }
+    if (multi % 2) {
+        for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);
+        h->flipped ^= 1;
     }
     h->last_n = nsteps;
     h->last_nrec = h->nrec;

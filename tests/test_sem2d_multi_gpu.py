@@ -51,8 +51,27 @@ def test_receiver_counts_and_steps_between_runs(gpu):
         a.step()
         b.step()
         assert np.array_equal(a.current(), b.current()) and np.array_equal(a.previous(), b.previous())
-    a.set_timing(True)  # event-bracketed single steps
-    (sa, _), (sb, _) = a.run(11), b.run(11)
-    assert np.array_equal(sa, sb) and np.array_equal(a.current(), b.current())
+    a.set_timing(True)  # event-bracketed launches
+    for n in (11, 8):
+        (sa, ra), (sb, rb) = a.run(n), b.run(n)
+        assert np.array_equal(sa, sb) and np.array_equal(ra, rb)
+        assert np.array_equal(a.current(), b.current()) and np.array_equal(a.previous(), b.previous())
     a.close()
     b.close()
+
+
+def test_timed_runs_time_the_launches_that_runs_make(gpu):
+    """A timed run takes the same launches as an untimed one: on a mesh that
+    takes several steps per launch its time per step is well under a single
+    step's (2.5 of 6 us)."""
+    print("\n[sem2d-multi] timing", flush=True)
+    ms = {}
+    for chunk in (0, 4):
+        s = gpu.Sem2dSolver(ex=65, nsamples=400, chunk=chunk)
+        s.run(80)
+        s.set_timing(True)
+        s.run(200)
+        ms[chunk] = s.last_kernel_ms()
+        s.close()
+    print("[sem2d-multi] ms per step", ms, flush=True)
+    assert ms[0] < 0.8 * ms[4]
