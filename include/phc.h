@@ -347,6 +347,13 @@ phc_status phc_sem2d_set_timing(phc_sem2d *h, int enable);
  * hold several steps) */
 phc_status phc_sem2d_last_run_kernel_ms(phc_sem2d *h, double *ms_per_step);
 phc_status phc_sem2d_synchronize(phc_sem2d *h);
+/* No counterpart in the reference.  Steps per launch of a run's whole launches
+ * (4 or 8, what is left in single steps) with 2 to 4 rows per wavefront; 0, 0:
+ * single steps.  Same values either way.  create chooses from the mesh (single
+ * steps with an explicit chunk_i or index64); a combination without a kernel
+ * for the order is PHC_ERR_INVALID. */
+phc_status phc_sem2d_set_steps_per_launch(phc_sem2d *h, int steps, int rows_per_wave);
+phc_status phc_sem2d_steps_per_launch(phc_sem2d *h, int *steps, int *rows_per_wave);
 /* Autotuner (no reference counterpart): rows per wavefront, timed on scratch
  * copies of the levels. */
 phc_status phc_sem2d_autotune(phc_sem2d *h, int steps_per_trial, int *chunk);

@@ -407,6 +407,7 @@ static Sem2dMultiFn s2_multi_rows(int rz)
 // leaves less than 16 columns or 8 rows.
 static Sem2dMultiFn sem2d_pick_multi(int p, int t, int rz)
 {
+    if (t != 4 && t != 8) return nullptr;
     switch (p * 10 + t) {
     case 14: return s2_multi_rows<1, 4>(rz);
     case 18: return s2_multi_rows<1, 8>(rz);
@@ -538,6 +539,23 @@ static void s2_plan_multi(phc_sem2d *h)
                 h->multi_rz = rz;
             }
         }
+}
+
+// The second pair of levels: both or none, halos zero as the first pair's.
+static phc_status s2_alloc_alt(phc_sem2d *h)
+{
+    const size_t bytes = sizeof(float) * (size_t)h->L.total;
+    if (h->alt[1].ptr) return PHC_OK;
+    phc_status st = PHC_OK;
+    for (DevBuf &b : h->alt)
+        if (st == PHC_OK) st = b.alloc(bytes);
+    if (st != PHC_OK) {
+        for (DevBuf &b : h->alt) b.release();
+        (void)hipGetLastError();
+        return st;
+    }
+    for (DevBuf &b : h->alt) PHC_TRY(fill_field(h->stream, b.as<float>(), h->L.total, 0.f));
+    return PHC_OK;
 }
 
 static void s2_fill_args(const phc_sem2d *h, Sem2dArgs &a, int i1, int i2)
@@ -747,15 +765,39 @@ phc_status phc_sem2d_create(const phc_sem_params *p, phc_sem2d **out)
     }
     h->index64 = p->index64 ? 1 : 0;
     if (!h->chunk && !h->index64) s2_plan_multi(h);
-    if (h->multi_t && (h->alt[0].alloc(bytes) || h->alt[1].alloc(bytes))) {
-        for (DevBuf &b : h->alt) b.release();
-        (void)hipGetLastError();
-        h->multi_t = 0;  // no room for the second pair of levels: single steps
+    if (h->multi_t && (st = s2_alloc_alt(h)) != PHC_OK) {
+        if (h->alt[1].ptr) return bail(st);
+        h->multi_t = h->multi_rz = 0;  // no room for the second pair of levels: single steps
     }
-    if (h->multi_t)
-        for (DevBuf &b : h->alt)
-            if ((st = fill_field(h->stream, b.as<float>(), h->L.total, 0.f))) return bail(st);
     *out = h;
+    return PHC_OK;
+}
+
+phc_status phc_sem2d_set_steps_per_launch(phc_sem2d *h, int steps, int rows)
+{
+    if (!h) return fail(PHC_ERR_INVALID, "handle is NULL");
+    if (steps == 0 && rows == 0) {
+        PHC_HIP(hipStreamSynchronize(h->stream));
+        s2_drop_graph(h);
+        h->multi_t = h->multi_rz = 0;
+        return PHC_OK;
+    }
+    if (!sem2d_pick_multi(h->p, steps, rows))
+        return fail(PHC_ERR_INVALID, "no kernel of %d steps per launch with %d rows per wavefront for order %d", steps,
+                    rows, h->p);
+    PHC_HIP(hipStreamSynchronize(h->stream));
+    PHC_TRY(s2_alloc_alt(h));
+    s2_drop_graph(h);
+    h->multi_t = steps;
+    h->multi_rz = rows;
+    return PHC_OK;
+}
+
+phc_status phc_sem2d_steps_per_launch(phc_sem2d *h, int *steps, int *rows)
+{
+    if (!h) return fail(PHC_ERR_INVALID, "handle is NULL");
+    if (steps) *steps = h->multi_t;
+    if (rows) *rows = h->multi_rz;
     return PHC_OK;
 }
 

@@ -743,6 +743,8 @@ SIGNATURES.update({
     "phc_sem2d_set_timing": (c_int, [c_void_p, c_int]),
     "phc_sem2d_last_run_kernel_ms": (c_int, [c_void_p, ctypes.POINTER(c_double)]),
     "phc_sem2d_synchronize": (c_int, [c_void_p]),
+    "phc_sem2d_set_steps_per_launch": (c_int, [c_void_p, c_int, c_int]),
+    "phc_sem2d_steps_per_launch": (c_int, [c_void_p, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "phc_sem2d_autotune": (c_int, [c_void_p, c_int, ctypes.POINTER(c_int)]),
 })
 
@@ -862,6 +864,15 @@ class Sem2dSolver:
 
     def check_finite(self, level):
         return lib().phc_sem2d_check_finite(self.h, level)
+
+    def set_steps_per_launch(self, steps, rows_per_wave):
+        check(lib().phc_sem2d_set_steps_per_launch(self.h, steps, rows_per_wave))
+
+    def steps_per_launch(self):
+        """(steps, rows per wavefront) of a run's whole launches; (0, 0): single steps."""
+        t, r = c_int(), c_int()
+        check(lib().phc_sem2d_steps_per_launch(self.h, ctypes.byref(t), ctypes.byref(r)))
+        return t.value, r.value
 
     def autotune(self, steps_per_trial=10):
         c = c_int()

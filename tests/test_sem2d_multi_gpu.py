@@ -1,26 +1,35 @@
-"""SEM2D meshes that take several steps per launch, against the one-step kernel
-(an explicit number of rows per wavefront), bit for bit: every order, meshes
-of one and of several tiles with ragged last ones, runs shorter than, equal to
-and past whole launches (odd and even numbers of them), sources on edges,
-corners and in the interior, receivers on the source and past the number the
-multi-step launch samples."""
+"""SEM2D runs of several steps per launch, against the one-step kernel (an
+explicit number of rows per wavefront), bit for bit: every kernel (order, steps
+per launch, rows per wavefront) on a mesh of several tiles with ragged last
+ones and on one of 2 x 2 elements, and the shapes that create chooses on its own;
+runs shorter than, equal to and past whole launches (odd and even numbers of
+them), sources on edges, corners and in the interior, receivers on the source
+and past the number the multi-step launch samples."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-MESHES = [(2, 2, 1), (60, 33, 1), (9, 40, 2), (30, 31, 2), (65, 20, 3), (13, 14, 3), (20, 11, 4), (3, 30, 5), (14, 9, 5)]
+# (order, steps per launch, rows per wavefront): the tile, 64 columns by 16
+# wavefronts' rows less order x steps on each side, is at least 16 x 8 nodes
+SHAPES = [(p, t, r) for p in range(1, 6) for t in (4, 8) for r in (2, 3, 4)
+          if 2 * p * t + 16 <= 64 and 2 * p * t + 8 <= 16 * r]
+# meshes, and whether create chooses several steps per launch for them (256 CUs)
+PLANNED = [(2, 2, 1, True), (60, 33, 1, True), (9, 40, 2, True), (30, 31, 2, True), (65, 20, 3, True),
+           (13, 14, 3, True), (20, 11, 4, True), (26, 26, 5, True), (3, 30, 5, False), (14, 9, 5, False)]
 
 
-@pytest.mark.parametrize("ex,ez,order", MESHES)
-def test_multi_step_launches_equal_single_steps(gpu, ex, ez, order):
-    print("\n[sem2d-multi] %d x %d order %d" % (ex, ez, order), flush=True)
+def check_equal(gpu, ex, ez, order, shape=None, multi=True):
     rng = np.random.default_rng(ex * 100 + ez)
     model = rng.uniform(1500, 3000, ex * ez).astype(np.float32)
     for se in (0, (ez // 2) * ex + ex // 2, ex * ez - 1):
         kw = dict(ex=ex, ez=ez, lx=20.0 * ex, lz=20.0 * ez, order=order, dt=4e-4, f0=60.0, nsamples=80, model=model,
                   src_element=se)
         a, b = gpu.Sem2dSolver(**kw), gpu.Sem2dSolver(chunk=3, **kw)
+        if shape:
+            a.set_steps_per_launch(*shape)
+            assert a.steps_per_launch() == shape
+        assert (a.steps_per_launch()[0] > 0) == multi and b.steps_per_launch() == (0, 0)
         cur, prev = (rng.normal(0, 1, a.nn).astype(np.float32) for _ in range(2))
         nodes = rng.integers(0, a.nn, 150)
         nodes[3] = a.src_node
@@ -35,6 +44,39 @@ def test_multi_step_launches_equal_single_steps(gpu, ex, ez, order):
         assert np.isfinite(a.current()).all() and np.abs(a.current()).max() > 0
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("order,steps,rows", SHAPES)
+def test_every_kernel_equals_single_steps(gpu, order, steps, rows):
+    print("\n[sem2d-multi] order %d, %d steps, %d rows" % (order, steps, rows), flush=True)
+    tx, tz = 64 - 2 * order * steps, 16 * rows - 2 * order * steps
+    check_equal(gpu, (2 * tx + 7) // order + 1, (3 * tz + 5) // order + 1, order, (steps, rows))
+    check_equal(gpu, 2, 2, order, (steps, rows))
+
+
+@pytest.mark.parametrize("ex,ez,order,multi", PLANNED)
+def test_planned_launches_equal_single_steps(gpu, ex, ez, order, multi):
+    print("\n[sem2d-multi] %d x %d order %d" % (ex, ez, order), flush=True)
+    check_equal(gpu, ex, ez, order, multi=multi)
+
+
+def test_choosing_steps_between_runs(gpu):
+    """The choice changes between runs (levels in either pair of buffers); what
+    has no kernel is refused and leaves the choice."""
+    print("\n[sem2d-multi] choosing", flush=True)
+    kw = dict(ex=30, ez=31, lx=600.0, lz=620.0, order=2, dt=4e-4, f0=60.0, nsamples=80, src_element=400)
+    a, b = gpu.Sem2dSolver(chunk=4, **kw), gpu.Sem2dSolver(chunk=4, **kw)
+    for shape, n in (((8, 3), 9), ((4, 2), 5), ((0, 0), 3), ((4, 4), 13), ((8, 4), 8)):
+        a.set_steps_per_launch(*shape)
+        for bad in ((8, 2), (3, 2), (14, 2), (-6, 2), (4, 5), (4, 0), (0, 2)):
+            with pytest.raises(gpu.PhcError):
+                a.set_steps_per_launch(*bad)
+        assert a.steps_per_launch() == shape
+        (sa, _), (sb, _) = a.run(n), b.run(n)
+        assert np.array_equal(sa, sb)
+        assert np.array_equal(a.current(), b.current()) and np.array_equal(a.previous(), b.previous()), shape
+    a.close()
+    b.close()
 
 
 def test_receiver_counts_and_steps_between_runs(gpu):
