@@ -354,8 +354,9 @@ phc_status phc_sem2d_synchronize(phc_sem2d *h);
  * for the order is PHC_ERR_INVALID. */
 phc_status phc_sem2d_set_steps_per_launch(phc_sem2d *h, int steps, int rows_per_wave);
 phc_status phc_sem2d_steps_per_launch(phc_sem2d *h, int *steps, int *rows_per_wave);
-/* Autotuner (no reference counterpart): rows per wavefront, timed on scratch
- * copies of the levels. */
+/* Autotuner (no reference counterpart), timed on scratch copies of the levels:
+ * *chunk = rows per wavefront of a single step; a handle that takes several
+ * steps per launch goes on with them only if they are faster than that. */
 phc_status phc_sem2d_autotune(phc_sem2d *h, int steps_per_trial, int *chunk);
 
 /* SEMmesh::getElementNumberFromPoints (SEMmesh.cpp:266-285). */

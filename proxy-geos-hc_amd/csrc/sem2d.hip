@@ -867,6 +867,36 @@ phc_status phc_sem2d_set_source(phc_sem2d *h, int src_element, int nsamples, con
     return PHC_OK;
 }
 
+// multi_t steps from the levels in `from` to those in `to`, the first one step0
+// of a run of nsteps (0: nothing injected).
+static phc_status s2_launch_multi(phc_sem2d *h, int i1, int i2, const DevBuf *from, const DevBuf *to, int step0,
+                                  int nsteps, float *trace, int nrec)
+{
+    const int t = h->multi_t;
+    Sem2dMultiArgs m;
+    s2_fill_args(h, m.s, i1, i2);
+    m.s.pn = from[i2].as<float>();
+    m.s.pnm1 = from[i1].as<float>();
+    m.out_n = to[i2].as<float>();
+    m.out_nm1 = to[i1].as<float>();
+    m.src_x = h->src_node % h->nx;
+    m.src_z = h->src_node / h->nx;
+    m.window = h->window.as<float>();
+    m.step0 = step0;
+    m.nsteps = nsteps;
+    m.trace = trace;
+    m.rec_node = h->recnode.as<int>();
+    m.s.rec_out = h->rec.as<float>();
+    m.s.rec_n = nrec;
+    m.s.rec_stride = nsteps;
+    const int tx = 64 - 2 * h->p * t, tz = S2_MW * h->multi_rz - 2 * h->p * t;
+    m.tiles_x = (h->nx + tx - 1) / tx;
+    hipLaunchKernelGGL(sem2d_pick_multi(h->p, t, h->multi_rz), dim3(m.tiles_x * ((h->nz + tz - 1) / tz)),
+                       dim3(64 * S2_MW), 0, h->stream, m);
+    PHC_HIP(hipGetLastError());
+    return PHC_OK;
+}
+
 // Launches of several steps at the start of a run (more receivers than such a
 // launch samples: none).
 static int s2_multi_launches(const phc_sem2d *h, int nsteps)
@@ -887,29 +917,9 @@ static phc_status s2_enqueue_run(phc_sem2d *h, int nsteps, int i1, int i2, hipEv
     const float *win = h->window.as<float>();
     const int t = h->multi_t, launches = s2_multi_launches(h, nsteps);
     for (int l = 0; l < launches; ++l) {
-        Sem2dMultiArgs m;
-        s2_fill_args(h, m.s, i1, i2);
         DevBuf *from = (l & 1) ? h->alt : h->lev, *to = (l & 1) ? h->lev : h->alt;
-        m.s.pn = from[i2].as<float>();
-        m.s.pnm1 = from[i1].as<float>();
-        m.out_n = to[i2].as<float>();
-        m.out_nm1 = to[i1].as<float>();
-        m.src_x = h->src_node % h->nx;
-        m.src_z = h->src_node / h->nx;
-        m.window = win;
-        m.step0 = l * t;
-        m.nsteps = nsteps;
-        m.trace = h->trace.as<float>();
-        m.rec_node = h->recnode.as<int>();
-        m.s.rec_out = h->rec.as<float>();
-        m.s.rec_n = h->nrec;
-        m.s.rec_stride = nsteps;
-        const int tx = 64 - 2 * h->p * t, tz = S2_MW * h->multi_rz - 2 * h->p * t;
-        m.tiles_x = (h->nx + tx - 1) / tx;
         if (ev) PHC_HIP(hipEventRecord(ev[2 * l], h->stream));
-        hipLaunchKernelGGL(sem2d_pick_multi(h->p, t, h->multi_rz), dim3(m.tiles_x * ((h->nz + tz - 1) / tz)),
-                           dim3(64 * S2_MW), 0, h->stream, m);
-        PHC_HIP(hipGetLastError());
+        PHC_TRY(s2_launch_multi(h, i1, i2, from, to, l * t, nsteps, h->trace.as<float>(), h->nrec));
         if (ev) PHC_HIP(hipEventRecord(ev[2 * l + 1], h->stream));
     }
     if (ev) ev += 2 * launches;
@@ -1091,17 +1101,19 @@ phc_status phc_sem2d_synchronize(phc_sem2d *h)
     return PHC_OK;
 }
 
-// Autotuner (no reference counterpart): rows per wave, timed on scratch
-// copies of the levels (state untouched).
+// Autotuner (no reference counterpart): rows per wave of a single step, and
+// whether a run's several steps per launch stay, timed on scratch copies of the
+// levels (state untouched; the second pair of levels holds none between runs).
 phc_status phc_sem2d_autotune(phc_sem2d *h, int steps_per_trial, int *chunk)
 {
     if (!h) return fail(PHC_ERR_INVALID, "handle is NULL");
     if (steps_per_trial < 1) return fail(PHC_ERR_INVALID, "steps_per_trial must be >= 1");
     const size_t bytes = sizeof(float) * (size_t)h->L.total;
-    DevBuf s0, s1;
+    DevBuf s0, s1, trace;
     PHC_TRY(s0.alloc(bytes));
     phc_status st = s1.alloc(bytes);
-    if (st != PHC_OK) { s0.release(); return st; }
+    if (st == PHC_OK && h->multi_t) st = trace.alloc(sizeof(float) * h->multi_t);
+    if (st != PHC_OK) return st;
     if (hipMemcpyAsync(s0.ptr, h->lev[0].ptr, bytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess ||
         hipMemcpyAsync(s1.ptr, h->lev[1].ptr, bytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess)
         st = fail(PHC_ERR_HIP, "scratch copy failed");
@@ -1114,33 +1126,47 @@ phc_status phc_sem2d_autotune(phc_sem2d *h, int steps_per_trial, int *chunk)
     double best = 1e30;
     int bc = h->chunk;
     int last = -1;
+    // ms of n launches, the second of two passes
+    auto trial = [&](int n, auto launch) {
+        float ms = 0.f;
+        for (int rep = 0; rep < 2 && st == PHC_OK; ++rep) {
+            if (hipEventRecord(e0, h->stream) != hipSuccess) st = fail(PHC_ERR_HIP, "event record failed");
+            for (int s = 0; s < n && st == PHC_OK; ++s) st = launch(s);
+            if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+                                 hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+                st = fail(PHC_ERR_HIP, "trial timing failed");
+        }
+        return (double)ms;
+    };
     for (int c0 : chunks) {
         if (st != PHC_OK) break;
         const int c = std::min(c0, h->nz);
         if (c == last) continue;
         last = c;
         h->chunk = c;
-        float ms = 0.f;
-        for (int rep = 0; rep < 2 && st == PHC_OK; ++rep) {
-            if (hipEventRecord(e0, h->stream) != hipSuccess) st = fail(PHC_ERR_HIP, "event record failed");
-            for (int s = 0; s < steps_per_trial && st == PHC_OK; ++s)
-                st = s2_launch(h, s & 1, 1 - (s & 1), nullptr, nullptr, nullptr, nullptr);
-            if (st == PHC_OK && (hipEventRecord(e1, h->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                                 hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
-                st = fail(PHC_ERR_HIP, "trial timing failed");
-        }
+        const double ms = trial(steps_per_trial, [&](int s) {
+            return s2_launch(h, s & 1, 1 - (s & 1), nullptr, nullptr, nullptr, nullptr);
+        });
         if (st == PHC_OK && ms < best) { best = ms; bc = c; }
+    }
+    bool keep_multi = h->multi_t > 0;
+    if (st == PHC_OK && h->multi_t) {
+        const int n = (steps_per_trial + h->multi_t - 1) / h->multi_t;
+        const double ms = trial(n, [&](int s) {
+            return s2_launch_multi(h, 0, 1, (s & 1) ? h->alt : h->lev, (s & 1) ? h->lev : h->alt, 0, 0,
+                                   trace.as<float>(), 0);
+        });
+        keep_multi = ms / (n * h->multi_t) < best / steps_per_trial;
     }
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     (void)hipStreamSynchronize(h->stream);
     std::swap(h->lev[0], s0);
     std::swap(h->lev[1], s1);
-    s0.release();
-    s1.release();
     h->chunk = bc;
     s2_drop_graph(h);
     PHC_TRY(st);
+    if (!keep_multi) h->multi_t = h->multi_rz = 0;
     if (chunk) *chunk = h->chunk;
     return PHC_OK;
 }

@@ -117,3 +117,24 @@ def test_timed_runs_time_the_launches_that_runs_make(gpu):
         s.close()
     print("[sem2d-multi] ms per step", ms, flush=True)
     assert ms[0] < 0.8 * ms[4]
+
+
+def test_autotune_drops_a_slower_choice_and_keeps_a_faster_one(gpu):
+    """2001^2 nodes of order 5 with 4 steps per launch: some 100 us per step
+    against 20 in single steps; 196^2 nodes of order 3: 1.6 against 2.9."""
+    print("\n[sem2d-multi] autotune", flush=True)
+    for kw, shape, want in ((dict(ex=400, ez=400, order=5, lx=8000.0, src_element=80200), (4, 3), (0, 0)),
+                            (dict(ex=65, ez=65, order=3, lx=2600.0, src_element=2000), (4, 2), (4, 2))):
+        a, b = (gpu.Sem2dSolver(dt=4e-4, f0=60.0, nsamples=40, **kw) for _ in range(2))
+        a.set_steps_per_launch(*shape)
+        b.set_steps_per_launch(0, 0)
+        for s in (a, b):
+            s.run(12)
+        state = a.current(), a.previous()
+        assert a.autotune(steps_per_trial=20) >= 1
+        assert a.steps_per_launch() == want
+        assert np.array_equal(a.current(), state[0]) and np.array_equal(a.previous(), state[1])
+        assert np.array_equal(a.run(13)[0], b.run(13)[0])
+        assert np.array_equal(a.current(), b.current()) and np.array_equal(a.previous(), b.previous())
+        a.close()
+        b.close()
