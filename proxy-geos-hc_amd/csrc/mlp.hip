@@ -1071,7 +1071,8 @@ using namespace phc;
 
 struct phc_lb {
     int device = 0;  // the device current at create (the stream's device)
-    DevBuf theta, grad, m, v, loss, wbf;
+    DevBuf theta, m, v, wbf;
+    DevBuf grad, loss;  // results of phc_lb_eval
     DevBuf data[LB_FACES];
     DevBuf count;  // unsigned long long per face
     int64_t cap = 0;
@@ -1192,8 +1193,7 @@ phc_status phc_lb_create(uint64_t seed, phc_lb **out)
     if (hipMemcpy(h->theta.ptr, th.data(), 4 * n, hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(PHC_ERR_HIP, "upload failed"));
     std::vector<float> z(n, 0.f);
-    if (hipMemcpy(h->grad.ptr, z.data(), 4 * n, hipMemcpyHostToDevice) ||
-        hipMemcpy(h->m.ptr, z.data(), 4 * n, hipMemcpyHostToDevice) ||
+    if (hipMemcpy(h->m.ptr, z.data(), 4 * n, hipMemcpyHostToDevice) ||
         hipMemcpy(h->v.ptr, z.data(), 4 * n, hipMemcpyHostToDevice) ||
         hipMemset(h->count.ptr, 0, 8 * LB_FACES) != hipSuccess)
         return bail(fail(PHC_ERR_HIP, "upload failed"));
@@ -1234,7 +1234,6 @@ phc_status phc_lb_set_params(phc_lb *h, const float *host)
     std::vector<float> z(LB_FACES * LB_NP, 0.f);
     PHC_HIP(hipMemcpy(h->m.ptr, z.data(), 4 * z.size(), hipMemcpyHostToDevice));
     PHC_HIP(hipMemcpy(h->v.ptr, z.data(), 4 * z.size(), hipMemcpyHostToDevice));
-    PHC_HIP(hipMemcpy(h->grad.ptr, z.data(), 4 * z.size(), hipMemcpyHostToDevice));
     PHC_HIP(hipStreamSynchronize(h->stream));
     return PHC_OK;
 }
@@ -1423,16 +1422,12 @@ phc_status phc_lb_eval(phc_lb *h, float *loss, float *grad)
     }
     B.inv_total = 1.f / (float)tot;
     const int np = LB_FACES * LB_NP;
-    DevBuf saved;
-    PHC_TRY(saved.alloc(4 * (size_t)np));  // keep the gradient a training run may be accumulating
-    PHC_HIP(hipMemcpyAsync(saved.ptr, h->grad.ptr, 4 * np, hipMemcpyDeviceToDevice, h->stream));
     lb_fill(h, h->grad.as<float>(), np, 0.f);
     lb_fill(h, h->loss.as<float>(), 1, 0.f);
     PHC_TRY(lb_launch_train(h, B));
     PHC_HIP(hipStreamSynchronize(h->stream));
     PHC_HIP(hipMemcpy(loss, h->loss.ptr, 4, hipMemcpyDeviceToHost));
     if (grad) PHC_HIP(hipMemcpy(grad, h->grad.ptr, 4 * np, hipMemcpyDeviceToHost));
-    PHC_HIP(hipMemcpy(h->grad.ptr, saved.ptr, 4 * np, hipMemcpyDeviceToDevice));
     return PHC_OK;
 }
 
@@ -1473,7 +1468,7 @@ static phc_status lb_train_core(phc_lb *h, const int64_t *c, int steps, int batc
         B.noise = h->noise;
         B.nseed = seed * 7919ull + (uint64_t)s;
         hipLaunchKernelGGL(lb_train_kernel, dim3(B.block_start[LB_FACES]), dim3(LB_TT), 0, h->stream,
-                           h->theta.as<float>(), h->grad.as<float>(), lh + s, B);
+                           h->theta.as<float>(), (float *)nullptr, lh + s, B);
         ++h->adam_t;
         const float c1 = 1.f / (1.f - std::pow(b1, (float)h->adam_t));
         const float c2 = 1.f / (1.f - std::pow(b2, (float)h->adam_t));

@@ -3,7 +3,8 @@ device memory they ask for.  Runs whose graph cannot be instantiated: the call
 returns an error and the state is as before it, so the same call succeeds
 afterwards with the values of a run that never failed.  Fields read and written
 without device memory for the packing: the same values.  The scratch memory of
-the packing: bounded, and none held before a field is read.  A shim between
+the packing: bounded, and none held before a field is read.  A learned layer's
+loss and gradient: no device memory asked for.  A shim between
 libphc.so and the HIP runtime (tests/cpp/hip_faults.c) refuses and counts; it
 has to be loaded first, so each test runs in a process of its own."""
 import ctypes
@@ -131,7 +132,23 @@ def check_scratch_size(phc, faults):
     sol.close()
 
 
+def check_eval_allocates_nothing(phc, faults):
+    rng = np.random.default_rng(5)
+    lb = phc.LearnedBoundary(seed=3)
+    lb.set_capacity(300)
+    for f in range(phc.LB_FACES):
+        lb.add_samples(f, rng.uniform(0, 1, (300, phc.LB_SAMPLE)).astype(np.float32))
+    want = lb.eval()
+    faults.hip_faults_set(0, 0)
+    got = lb.eval()
+    faults.hip_faults_set(NEVER, 0)
+    # float atomics: sums of 1800 terms in any order
+    assert abs(got[0] - want[0]) <= 1e-5 * want[0]
+    assert np.allclose(got[1], want[1], rtol=1e-4, atol=1e-5 * np.abs(want[1]).max())
+
+
 CASES = {
+    "eval_allocates_nothing": check_eval_allocates_nothing,
     "no_scratch": check_no_scratch,
     "scratch_size": check_scratch_size,
     "failed_run_fd": lambda phc, f: check_failed_run(phc, f, fd),
