@@ -549,6 +549,19 @@ static phc_status fd_plan_launch(phc_fd *h, FdStepArgs &a, int *nb)
 // 480 x 380 x 480, 512^3: 9.1, 17.1, 38.1, 62.9, 90.3, 204, 274, 358 us
 // against 7.5, 14.3, 29.2, 58.9, 88.7, 198, 258, 347).  A partial last k tile
 // stays a tile there (point by point it cost 10-30% more at 96^3 to 264^3).
+// The other radii have one shape, 4 waves x 8 rows, and the schedules were
+// faster than chunks of 256 planes at every size in the cache (radius 1 to 6,
+// 64^3 to 304^3 and two slabs: 1.4 to 11 times) and at most beyond it (512^3 of
+// radius 5 and 6 464 and 477 us against 510 and 525; 640^3 of radius 1 to 6 792
+// to 836 against 898 to 1094).  Radii 1 and 2 beyond the cache take chunks where
+// those load the busiest CU hardly more: with few planes to prime, a schedule
+// has little to win, and its ranges keep more rows open in memory (radius 1: 512^3 381
+// against 424, 504 x 249 x 751 259 against 303, 900 x 400 x 300 371 against 383;
+// radius 2: 504 x 249 x 751 267 against 312; at costs of 1.16 and 1.14, 442 x 767
+// x 584 698 against 661 and 900 x 400 x 300 391 against 375).  Radii 1 to 3
+// count the tiles without the remainder slabs (480^3 of radius 3 361 us, with
+// them 398), 5 and 6 with them (480 x 380 x 480 297 us, without 326).  Of 48
+// grids of radius 1 to 3, three are still 2-5% faster with chunks.
 static void fd_default_shape(phc_fd *h)
 {
     static const int quad[][2] = {{8, 4}, {4, 4}}, other[][2] = {{4, 2}};
@@ -559,18 +572,32 @@ static void fd_default_shape(phc_fd *h)
         const int ty = shapes[s][0], nj = shapes[s][1], TJ = ty * nj;
         FdKernelFn fn = fd_pick_kernel(h->R, ty, nj, h->arith, !h->index64 && h->L.total * 4 < ((int64_t)1 << 32),
                                        false, fd_streams_past_cache(h->L));
-        const int ncol = ((h->nz + FD_TK - 1) / FD_TK) * ((h->ny + TJ - 1) / TJ);
+        int ncol = ((h->nz + FD_TK - 1) / FD_TK) * ((h->ny + TJ - 1) / TJ);
+        if (h->R <= 3) {
+            FdStepArgs a;
+            h->ty = ty;
+            h->nj = nj;
+            fd_fill_args(h, a, 0, 1);
+            (void)fd_plan_blocks(a, h->krem_eff, FD_TK * ty, TJ);
+            ncol = a.tiles_k * a.tiles_j;
+        }
         const int cux = std::max(h->cus / 8, 1), slots = cux * fd_resident(fn, ty, nj);
         std::vector<int4> tab;
+        auto cost = [&] { return xcd_schedule_cost(tab, cux, TJ, 0.35 * 2 * h->R, 2 * h->R); };
         for (int m = 1; m <= 4; ++m) {
             build_xcd_schedule(h->nx, 0, ncol, slots, m, 1, tab);
-            const double c = xcd_schedule_cost(tab, cux, TJ, 0.35 * 2 * h->R, 2 * h->R);
+            const double c = cost();
             if (best < 0.0 || c < best) {
                 best = c;
                 h->ty = ty;
                 h->nj = nj;
                 h->chunk_i = -m;
             }
+        }
+        if (h->R <= 2 && fd_streams_past_cache(h->L)) {
+            const int chunk = std::min(h->nx, 256);
+            build_chunk_table(h->nx, ncol, chunk, tab);
+            if (cost() < (h->R == 1 ? 1.15 : 1.06) * best) h->chunk_i = chunk;
         }
     }
 }

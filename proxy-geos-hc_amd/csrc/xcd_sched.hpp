@@ -53,6 +53,18 @@ inline void build_xcd_schedule(int planes, int plane0, int ncol, int slots_per_x
         for (size_t l = 0; l < lists[x].size(); ++l) tab[8 * l + x] = lists[x][l];
 }
 
+// The table of plain chunks of `chunk` planes, one block per (chunk, tile
+// column) in XCD block order (xcd_block, march.hpp).
+inline void build_chunk_table(int planes, int ncol, int chunk, std::vector<int4> &tab)
+{
+    const int nb = ncol * ((planes + chunk - 1) / chunk), q = nb / 8, r = nb % 8;
+    tab.assign((size_t)(nb + 7) / 8 * 8, make_int4(0, 0, 0, 0));
+    for (int b = 0; b < nb; ++b) {
+        const int x = b % 8, t = x * q + std::min(x, r) + b / 8, i0 = t / ncol * chunk;
+        tab[b] = make_int4(t % ncol, i0, std::min(i0 + chunk, planes), 0);
+    }
+}
+
 // Work of the busiest CU under a schedule table, in rows x planes: an XCD's
 // entries go in order to its least loaded CU; an entry of n planes costs
 // (n + lead) x (rows + halo).  lead: planes' worth of a march's first loads
