@@ -1216,13 +1216,19 @@ static int sem_resident(const phc_sem *h)
 // 4: 9.7 / 10.3; 101^3, at once above the line: order 1 10.2 / 8.7, order 2
 // 11.9 / 9.5, order 5 15.3 / 14.3).  Above, 4 waves x 16 rows, split 1, the
 // best or within 5% of the best table entry from 101^3 to 321^3 (order 1
-// alone prefers chunks of 12-24 planes by up to 14%).  From 500 MB of arrays
-// the shape and split with the least work on the busiest CU, as in the FD
-// step: us per step of 8 x 1 / 4 x 16 split 1 / chosen: 341^3 order 2 122 /
-// 117 / 111, 331 x 346 x 331 order 3 127 / 112 / 104, 353 x 361 x 345 order 4
-// 148 / 141 / 122, 351 x 361 x 351 order 5 186 / 138 / 126, 481^3-sized orders
-// 3, 4, 5 373, 346, 377 / - / 295, 281, 279; below the line that choice loses
-// (321^3 order 4 95.6 against 90.0, 261^3 order 2 71 against 55).
+// alone prefers chunks of 12-24 planes by up to 14%).  For large arrays the
+// shape and split with the least work on the busiest CU, as in the FD step: us
+// per step of 8 x 1 / 4 x 16 split 1 / chosen: 331 x 346 x 331 order 3 127 / 112
+// / 104, 353 x 361 x 345 order 4 148 / 141 / 122, 351 x 361 x 351 order 5 186 /
+// 138 / 126, 481^3-sized orders 3, 4, 5 373, 346, 377 / - / 295, 281, 279.  The
+// lines lie where 4 x 16 split 1 stops winning (it / the choice, MB of arrays):
+//   order 1  331^3  511  99.9 / 102.2   341^3  542 110.2 / 115.6 | 356^3  640 136.5 / 132.5
+//   order 2  327^3  505 101.6 / 109.3   333^3  523 102.2 / 102.0 | 341^3  548 115.8 / 108.2
+//   order 3  292^3  375  75.6 /  76.2   313^3  430  83.5 /  91.9 | 325^3  505 105.7 /  95.0
+//   order 4  313^3  435  83.8 /  94.2   321^3  499  87.9 /  92.6 | 325^3  511 109.6 /  98.9
+//   order 5  291^3  383  82.1 /  79.9   311^3  435  98.9 /  94.2 | 321^3  505 102.9 /  95.4
+// 321 nodes are 5 whole tiles along x; the sixth and the next row of tiles
+// cost split 1 its balance.
 static void sem_default_shape(phc_sem *h)
 {
     h->ty = 8;
@@ -1232,7 +1238,7 @@ static void sem_default_shape(phc_sem *h)
     h->ty = 4;
     h->nj = 4;
     h->chunk_i = -1;
-    if (12 * h->L.total < (int64_t)500e6) return;
+    if (12 * h->L.total < (h->p <= 2 ? (int64_t)545e6 : (int64_t)500e6)) return;
     double best = -1.0;
     int ty = 4, m = 1;
     for (int t : {8, 4}) {
