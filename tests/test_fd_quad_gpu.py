@@ -45,3 +45,33 @@ def test_quad_shapes_equal_the_one_point_tile(gpu, grid, boundary):
                    dict()):
             for w, g in zip(want, run(arith=arith, **kw)):
                 assert np.array_equal(w, g), (arith, kw)
+
+
+@pytest.mark.parametrize("boundary", ["sponge", "pml"])
+def test_streaming_quad_shapes_equal_the_one_point_tile(gpu, boundary):
+    """Arrays past the memory-side cache (three of them above 300 MB) take
+    non-temporal accesses, with 32-bit offsets."""
+    nx, ny, nz = 40, 803, 790
+    pitch = (32 + nz + 4 + 31) // 32 * 32
+    assert 12 * pitch * (ny + 8) * (nx + 8) > 300e6
+    print("\n[fd-quad] streaming %s" % boundary, flush=True)
+    rng = np.random.default_rng(11)
+    s = gpu.FdSetup(nx, ny, nz, L=4, f0=25.0, sponge_width=5 if boundary == "sponge" else 0,
+                    model=rng.uniform(0.5, 2.0, nx * ny * nz).astype(np.float32), nsamples=6, zs=nz - 1)
+    fields = rng.normal(0, 1, (2, nx + 8, ny + 8, nz + 8)).astype(np.float32)
+
+    def run(**kw):
+        sol = gpu.FdSolver(s, **kw)
+        if boundary == "pml":
+            sol.set_pml(ndamp=6)
+        for level in (0, 1):
+            sol.set_field(level, fields[level])
+        out = [sol.run(0, 3)[0], sol.current(), sol.previous()]
+        sol.close()
+        return out
+    for arith in (gpu.ARITH_REF, gpu.ARITH_FP32):
+        want = run(arith=arith, tile_j=8, block_waves=8, chunk_i=20)
+        assert all(np.isfinite(w).all() for w in want)
+        for kw in (dict(tile_j=16, block_waves=4, chunk_i=13), dict(tile_j=32, block_waves=8, chunk_i=-2)):
+            for w, g in zip(want, run(arith=arith, **kw)):
+                assert np.array_equal(w, g), (arith, kw)

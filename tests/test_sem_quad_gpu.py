@@ -39,3 +39,32 @@ def test_quad_shapes_equal_the_one_node_tile(gpu, mesh, order):
                    dict(block_waves=4, tile_j=16, chunk_i=-2, k_remainder=-1), dict()):
             for w, g in zip(want, run(pt, **sh)):
                 assert np.array_equal(w, g), sh
+
+
+@pytest.mark.parametrize("order", [1, 2, 3, 4, 5])
+def test_streaming_quad_shapes_equal_the_one_node_tile(gpu, order):
+    """Arrays past the memory-side cache (three of them above 300 MB) take
+    non-temporal accesses, with 32-bit offsets."""
+    ex, ez, ey = 790 // order, 803 // order, 40 // order
+    nx, ny, nz = (e * order + 1 for e in (ex, ey, ez))
+    pitch = (32 + nx + order + 31) // 32 * 32
+    assert 12 * pitch * (nz + 2 * order) * (ny + 2 * order) > 300e6
+    print("\n[sem-quad] streaming order %d" % order, flush=True)
+    rng = np.random.default_rng(order)
+    f = rng.normal(0, 1, (2, nx * ny * nz)).astype(np.float32)
+    kw = dict(ex=ex, ey=ey, ez=ez, lx=20.0 * ex, ly=20.0 * ey, lz=20.0 * ez, order=order, dt=0.001 / order ** 2,
+              model=rng.uniform(1000, 2000, ex * ey * ez), rhs=rng.normal(0, 1e3, 6).astype(np.float32),
+              src_point=(20.0 * (ex - 1) + 1, 20.0 * (ey // 2) + 1, 20.0 * (ez // 2) + 1))
+
+    def run(**sh):
+        s = gpu.SemSolver(**kw, **sh)
+        for level in (0, 1):
+            s.set_field(level, f[level])
+        out = [s.run(3)[0], s.field(0), s.field(1)]
+        s.close()
+        return out
+    want = run(block_waves=8, tile_j=8, chunk_i=20)
+    assert all(np.isfinite(w).all() for w in want)
+    for sh in (dict(block_waves=4, tile_j=16, chunk_i=8), dict(block_waves=8, tile_j=32, chunk_i=-2)):
+        for w, g in zip(want, run(**sh)):
+            assert np.array_equal(w, g), sh
