@@ -188,8 +188,8 @@ phc_status write_field(hipStream_t stream, DevBuf &scratch, float *field, const 
     const int NX = L.nx + 2 * lx, NY = L.ny + 2 * ly, NZ = L.nz + 2 * lz, rows = NX * NY;
     const size_t row = sizeof(float) * (size_t)NZ;
     const int per = piece_rows(rows, NZ);
+    PHC_HIP(hipStreamSynchronize(stream));
     if (!ensure_scratch(scratch, row * per)) {
-        PHC_HIP(hipStreamSynchronize(stream));
         for (int i = 0; i < NX; ++i)
             PHC_HIP(hipMemcpy2D(field + fd_off(L, i - lx, -ly, -lz), sizeof(float) * L.pitch_k,
                                 host + (int64_t)i * NY * NZ, row, row, NY, hipMemcpyHostToDevice));
@@ -197,12 +197,14 @@ phc_status write_field(hipStream_t stream, DevBuf &scratch, float *field, const 
     }
     for (int r0 = 0; r0 < rows; r0 += per) {
         const int n = std::min(per, rows - r0);
-        PHC_HIP(hipMemcpyAsync(scratch.ptr, host + (int64_t)r0 * NZ, row * n, hipMemcpyHostToDevice, stream));
+        // a plain copy: the first large asynchronous copy on a stream sets up
+        // staging memory, which would add 4 ms to every create
+        PHC_HIP(hipMemcpy(scratch.ptr, host + (int64_t)r0 * NZ, row * n, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(unpack_rows_kernel, dim3((n + 3) / 4), dim3(64, 4), 0, stream, field, L, r0, n, lx, ly, lz,
                            scratch.as<float>());
         PHC_HIP(hipGetLastError());
+        PHC_HIP(hipStreamSynchronize(stream));  // the next piece overwrites the scratch
     }
-    PHC_HIP(hipStreamSynchronize(stream));
     return PHC_OK;
 }
 
