@@ -223,7 +223,8 @@ def bench_sem2d(phc, steps=1000, big_ex=2000, big_order=4, big_steps=200):
     (big_ex^2 elements of order big_order) for the HBM roofline."""
     out = {}
     G = phc.Sem2dSolver(ex=65, order=3, lx=2000.0, dt=1e-3, f0=10.0, nsamples=steps + 1)
-    chunk = G.autotune(steps_per_trial=20)
+    chunk = G.autotune(steps_per_trial=20)  # rows per wavefront of the steps outside whole launches
+    per_launch = G.steps_per_launch()[0]
     G.run(steps)  # capture + warm
     G.synchronize()
     G.it = 0
@@ -242,6 +243,7 @@ def bench_sem2d(phc, steps=1000, big_ex=2000, big_order=4, big_steps=200):
         "workload": "SEM2D 65 x 65 elements of order 3 (38,416 nodes), %d steps" % steps,
         "wall_s": round(wall, 5), "value": round(v, 1), "unit": "Mnode-updates/s",
         "us_per_step": round(wall / steps * 1e6, 2), "kernel_us": round(kms * 1e3, 2), "chunk": chunk,
+        "steps_per_launch": per_launch,
         "published_best": PUBLISHED_SEM2D,
         "vs_published_best": round(v / max(PUBLISHED_SEM2D.values()), 1)}
     n = big_ex * big_order + 1

@@ -91,7 +91,7 @@ __device__ __forceinline__ void batch_sample(const BatchSample &r, const ShotDes
 // that claimed their items from a queue one after the other left that
 // latency and the claim's open: 12 shots of U[96,224]^3, best one-point shape
 // of each, 200 us per step against 240 (47.7 M points: 3.8 against 3.2 TB/s;
-// 182 with four points per lane, 4.2 TB/s).
+// 189 with four points per lane, 4.0 TB/s).
 //
 // fd_batch_item fills the grid of the block's item; false: nothing to march
 // (a sampling block, padding, or slab points, which it has updated).
@@ -449,9 +449,9 @@ phc_status phc_batch_create(const phc_batch_params *p, phc_batch **out)
         return fail(PHC_ERR_INVALID, "k_remainder must be -1, 0 or 1 (got %d)", p->k_remainder);
     // default: 4 waves x 16 rows, four points per lane, the fastest shape on
     // every survey measured (12 shots of U[96,224]^3 / 8 of U[106,190]^3 / 14
-    // of U[60,100]^3 / 24 of U[128,256]^3, best chunk of each: 182 / 89 / 29 /
-    // 609 us per step; 8 waves x 32 rows 202 / 102 / 33 / 633; 8 waves x 1 row
-    // 199 / 103 / 40 / 642; 4 waves x 2 rows 216 / 113 / 43 / 690)
+    // of U[60,100]^3 / 24 of U[128,256]^3, best chunk of each: 188 / 88 / 31 /
+    // 649 us per step; 8 waves x 32 rows 202 / 102 / 34 / 672; 8 waves x 1 row
+    // 200 / 102 / 45 / 685; 4 waves x 2 rows 217 / 112 / 53 / 728)
     const bool shape = p->block_waves || p->tile_j;
     const int ty = p->block_waves ? p->block_waves : shape ? 16 : 4;
     const int tj = p->tile_j ? p->tile_j : shape ? ty : 16;

@@ -547,7 +547,9 @@ static phc_status fd_plan_launch(phc_fd *h, FdStepArgs &a, int *nb)
 // the one-point shapes were slower at every size (best of all shapes and
 // chunks at 96^3, 150^3, 203 x 178 x 261, 264^3, 336 x 300 x 290, 401^3,
 // 480 x 380 x 480, 512^3: 9.1, 17.1, 38.1, 62.9, 90.3, 204, 274, 358 us
-// against 7.5, 14.3, 29.2, 58.9, 88.7, 198, 258, 347).  A partial last k tile
+// against 7.5, 14.3, 29.2, 58.9, 88.7, 198, 258, 347 for the best pair of the
+// quad shapes; the pair chosen here is that or within 6% of it, but for 264^3,
+// where it is split 4 of 8 waves x 32 rows, 67).  A partial last k tile
 // stays a tile there (point by point it cost 10-30% more at 96^3 to 264^3).
 // The other radii have one shape, 4 waves x 8 rows, and the schedules were
 // faster than chunks of 256 planes at every size in the cache (radius 1 to 6,
