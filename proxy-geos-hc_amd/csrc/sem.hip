@@ -1229,15 +1229,26 @@ static int sem_resident(const phc_sem *h)
 //   order 5  291^3  383  82.1 /  79.9   311^3  435  98.9 /  94.2 | 321^3  505 102.9 /  95.4
 // 321 nodes are 5 whole tiles along x; the sixth and the next row of tiles
 // cost split 1 its balance.
+// Flat meshes have few planes to cut: 8 ranges of whole groups leave XCDs idle
+// below 32 planes and prime the ring over and over.  Up to 25 planes the XCDs
+// take bands of columns over the whole axis (split 4), up to 63 halves of it
+// (split 3).  Us per step of 4 x 16 split 1 (8 x 1 split 2 below 600,000 nodes) /
+// 16 x 1 whole axis / this, orders 1 and 5: 801 x 5 x 801 47 / 15 / 14, 84 / 27 / 24;
+// 401 x 21 x 401 19 / 18 / 14, 31 / 22 / 20; 17 x 21 x 3001 13 / 17 / 11, 27 / 22 / 18;
+// 801 x 49 x 801 109 / 88 / 88, 141 / 106 / 100; 1767 x 51 x 341 98 / 90 / 83, 140 /
+// 117 / 99; 361 x 61 x 541 39 / 46 / 41, 50 / 52 / 40.  At 65 planes split 1 is level
+// or ahead at orders 1, 2 and 4.  Planes under 25,000 nodes keep 8 x 1 (145 x 33 x
+// 145 order 4 10.0 against 10.7).
 static void sem_default_shape(phc_sem *h)
 {
     h->ty = 8;
     h->nj = 1;
     h->chunk_i = -2;
-    if (h->nn < 600000) return;
+    const bool flat = h->ny < 64 && (int64_t)h->nx * h->nz >= 25000;
+    if (h->nn < 600000 && !flat) return;
     h->ty = 4;
     h->nj = 4;
-    h->chunk_i = -1;
+    h->chunk_i = !flat ? -1 : h->ny <= 25 ? -4 : -3;
     if (12 * h->L.total < (h->p <= 2 ? (int64_t)545e6 : (int64_t)500e6)) return;
     double best = -1.0;
     int ty = 4, m = 1;

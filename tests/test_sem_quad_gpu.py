@@ -68,3 +68,31 @@ def test_streaming_quad_shapes_equal_the_one_node_tile(gpu, order):
     for sh in (dict(block_waves=4, tile_j=16, chunk_i=8), dict(block_waves=8, tile_j=32, chunk_i=-2)):
         for w, g in zip(want, run(**sh)):
             assert np.array_equal(w, g), sh
+
+
+@pytest.mark.parametrize("order", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("planes", [6, 25, 30, 60, 66])
+def test_default_shapes_of_flat_meshes_equal_the_one_node_tile(gpu, order, planes):
+    """Few planes along the march axis under a plane of at least 25,000 nodes
+    (fewer than 26, than 64, more): the shapes that create chooses."""
+    print("\n[sem-quad] flat order %d, %d planes" % (order, planes), flush=True)
+    ex, ey, ez = 190 // order, planes // order, 150 // order
+    assert (ex * order + 1) * (ez * order + 1) >= 25000
+    rng = np.random.default_rng(planes)
+    kw = dict(ex=ex, ey=ey, ez=ez, lx=100.0 * ex, ly=100.0 * ey, lz=100.0 * ez, order=order, dt=0.001 / order ** 2,
+              model=rng.uniform(1000, 2000, ex * ey * ez), rhs=rng.normal(0, 1e3, 6).astype(np.float32),
+              src_point=(100.0 * (ex - 1) + 1, 100.0 * (ey // 2) + 1, 100.0 * (ez // 2) + 1))
+    nn = (ex * order + 1) * (ey * order + 1) * (ez * order + 1)
+    f = rng.normal(0, 1, (2, nn)).astype(np.float32)
+
+    def run(**sh):
+        s = gpu.SemSolver(**kw, **sh)
+        for level in (0, 1):
+            s.set_field(level, f[level])
+        out = [s.run(4)[0], s.field(0), s.field(1)]
+        s.close()
+        return out
+    want = run(block_waves=8, tile_j=8, chunk_i=1 << 20)
+    assert all(np.isfinite(w).all() for w in want)
+    for w, g in zip(want, run()):
+        assert np.array_equal(w, g)
