@@ -242,12 +242,12 @@ struct phc_batch {
     int timing = 0;
     double last_ms = 0.0;
     int last_n = 0, last_nrec = 0;
-    RunGraph graph[2];  // of phc_batch_run, by the level it starts from
+    RunGraphs graph[2];  // of phc_batch_run, by the level it starts from
 };
 
 static void batch_drop_graph(phc_batch *h)
 {
-    for (RunGraph &g : h->graph) g.drop();
+    for (RunGraphs &g : h->graph) g.drop();
 }
 
 // Planes per work item when the caller gives none: 24, fewer where a resident
@@ -628,7 +628,7 @@ phc_status phc_batch_run(phc_batch *h, int it0, int nsteps)
         PHC_TRY(prepare_captured(h->stream, h->graph[h->cur], nsteps, h->pending, h->nrec,
                                  [&] { return batch_enqueue(h, nsteps, nullptr); }));
         PHC_TRY(begin());
-        PHC_HIP(hipGraphLaunch(h->graph[h->cur].exec, h->stream));
+        PHC_HIP(hipGraphLaunch(h->graph[h->cur].exec(), h->stream));
     }
     if (nsteps % 2) h->cur = 1 - h->cur;
     h->pending = h->sw > 0 ? 1 : 0;

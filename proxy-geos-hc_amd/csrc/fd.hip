@@ -322,7 +322,7 @@ struct phc_fd {
     int lb_on = 0;
     LbInfer lbi;
     DevBuf lb_w, lb_corr, lb_kvcs, lb_kslab;
-    RunGraph graph[2];  // of phc_fd_run, by the level it starts from
+    RunGraphs graph[2];  // of phc_fd_run, by the level it starts from
 };
 
 static phc_status fd_validate(const phc_fd_params *p)
@@ -474,7 +474,7 @@ static phc_status fd_materialize(phc_fd *h, int level)
 
 static void fd_drop_graph(phc_fd *h)
 {
-    for (RunGraph &g : h->graph) g.drop();
+    for (RunGraphs &g : h->graph) g.drop();
 }
 
 // Whether a step's three arrays exceed what the 256 MB memory-side cache
@@ -930,7 +930,7 @@ phc_status phc_fd_run(phc_fd *h, int it0, int nsteps, int *cur)
         PHC_TRY(prepare_captured(h->stream, h->graph[c0], nsteps, damp0 ? 1 : 0, h->nrec,
                                  [&] { return fd_enqueue_run(h, nsteps, c0, damp0, nullptr); }));
         PHC_TRY(begin());
-        PHC_HIP(hipGraphLaunch(h->graph[c0].exec, h->stream));
+        PHC_HIP(hipGraphLaunch(h->graph[c0].exec(), h->stream));
     }
     const int cend = (nsteps % 2 == 0) ? c0 : 1 - c0;
     h->pending[cend] = 0;

@@ -70,9 +70,8 @@ struct DevBuf {
 // A captured chunk of a time loop.  Its nodes name no time sample (the chunk's
 // samples sit in a device window that a launch before the graph fills), so
 // one graph serves every chunk of the same length that starts from the same
-// levels; a handle keeps two, one per level parity.  Captured anew, a chunk
-// of 100 steps of the 196^2-node 2D mesh took 0.42 ms longer (1.19 against
-// 0.77 ms).
+// levels.  Captured anew, a chunk of 100 steps of the 196^2-node 2D mesh took
+// 0.42 ms longer (1.19 against 0.77 ms).
 struct RunGraph {
     hipGraphExec_t exec = nullptr;
     int n = -1, key = -1, nrec = -1;
@@ -84,14 +83,31 @@ struct RunGraph {
     }
 };
 
-// Has the slot hold the graph of an n-step chunk, capturing `enqueue` when it
-// holds another one (key: whatever else the nodes depend on).  Launches
-// nothing: a run changes its levels only after this has succeeded, so that one
-// that could not be captured can be called again.
+// The last two chunk lengths that started from the same levels: a program that
+// alternates between two (snapshots, a shorter last chunk per shot) captures
+// each once.  With one, runs of 10 and 7 steps in turn took 500 us each for the
+// capture on the 1201^2-node 2D mesh of order 4, 140 and 106 without.
+struct RunGraphs {
+    RunGraph slot[2];
+    int used = 0;  // the slot of the last run
+    hipGraphExec_t exec() const { return slot[used].exec; }
+    void drop()
+    {
+        for (RunGraph &g : slot) g.drop();
+    }
+};
+
+// Has gs.exec() be the graph of an n-step chunk, capturing `enqueue` in place
+// of the one not used last where neither slot holds it (key: whatever else the
+// nodes depend on).  Launches nothing: a run changes its levels only after this
+// has succeeded, so that one that could not be captured can be called again.
 template <class F>
-phc_status prepare_captured(hipStream_t stream, RunGraph &g, int n, int key, int nrec, F enqueue)
+phc_status prepare_captured(hipStream_t stream, RunGraphs &gs, int n, int key, int nrec, F enqueue)
 {
-    if (!(g.exec && g.n == n && g.key == key && g.nrec == nrec)) {
+    auto holds = [&](const RunGraph &g) { return g.exec && g.n == n && g.key == key && g.nrec == nrec; };
+    if (!holds(gs.slot[gs.used])) gs.used = 1 - gs.used;
+    RunGraph &g = gs.slot[gs.used];
+    if (!holds(g)) {
         if (g.exec) PHC_HIP(hipStreamSynchronize(stream));  // the old graph may still run
         g.drop();
         hipGraph_t graph = nullptr;

@@ -1132,7 +1132,7 @@ struct phc_sem {
     int nrec = 0, last_n = 0, last_nrec = 0;
     int timing = 0;
     double last_ms = 0.0;
-    RunGraph graph[2];  // of phc_sem_run, by i1
+    RunGraphs graph[2];  // of phc_sem_run, by i1
 };
 
 static int64_t sem_off(const phc_sem *h, int64_t node)
@@ -1145,7 +1145,7 @@ static int64_t sem_off(const phc_sem *h, int64_t node)
 
 static void sem_drop_graph(phc_sem *h)
 {
-    for (RunGraph &g : h->graph) g.drop();
+    for (RunGraphs &g : h->graph) g.drop();
 }
 
 // A node-order host field into a level (layout conversion for the
@@ -1847,7 +1847,7 @@ phc_status phc_sem_run(phc_sem *h, int it0, int nsteps, int *i1p, int *i2p)
         PHC_TRY(prepare_captured(h->stream, h->graph[i1], nsteps, 0, h->nrec,
                                  [&] { return sem_enqueue_run(h, nsteps, i1, i2, nullptr); }));
         PHC_TRY(begin());
-        PHC_HIP(hipGraphLaunch(h->graph[i1].exec, h->stream));
+        PHC_HIP(hipGraphLaunch(h->graph[i1].exec(), h->stream));
     }
     h->last_n = nsteps;
     h->last_nrec = h->nrec;

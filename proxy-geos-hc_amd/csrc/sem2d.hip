@@ -470,7 +470,7 @@ struct phc_sem2d {
     int multi_t = 0, multi_rz = 0;
     DevBuf alt[2], recnode;
     int flipped = 0;    // lev and alt have changed places an odd number of times
-    RunGraph graph[4];  // of phc_sem2d_run, by i1 and flipped
+    RunGraphs graph[4];  // of phc_sem2d_run, by i1 and flipped
 };
 
 static int64_t s2_off(const phc_sem2d *h, int64_t node)
@@ -481,7 +481,7 @@ static int64_t s2_off(const phc_sem2d *h, int64_t node)
 
 static void s2_drop_graph(phc_sem2d *h)
 {
-    for (RunGraph &g : h->graph) g.drop();
+    for (RunGraphs &g : h->graph) g.drop();
 }
 
 static phc_status s2_put(phc_sem2d *h, DevBuf &dst, const float *host)
@@ -997,11 +997,11 @@ phc_status phc_sem2d_run(phc_sem2d *h, int it0, int nsteps, int *i1p, int *i2p)
         for (auto &e : ev) (void)hipEventDestroy(e);
         PHC_TRY(st);
     } else {
-        RunGraph &graph = h->graph[i1 + 2 * h->flipped];
+        RunGraphs &graph = h->graph[i1 + 2 * h->flipped];
         PHC_TRY(prepare_captured(h->stream, graph, nsteps, 0, h->nrec,
                                  [&] { return s2_enqueue_run(h, nsteps, i1, i2, nullptr); }));
         PHC_TRY(begin());
-        PHC_HIP(hipGraphLaunch(graph.exec, h->stream));
+        PHC_HIP(hipGraphLaunch(graph.exec(), h->stream));
     }
     if (multi % 2) {
         for (int k = 0; k < 2; ++k) std::swap(h->lev[k], h->alt[k]);

@@ -1,6 +1,7 @@
 /* Test shim between libphc.so and the HIP runtime: device allocations and
  * graph instantiations that fail on request (the call is refused here and
- * never reaches the runtime), and a record of the live device allocations.
+ * never reaches the runtime), and a record of the live device allocations and
+ * of the graphs instantiated.
  * Loaded with RTLD_GLOBAL before libphc.so, so that its calls bind to it. */
 #define _GNU_SOURCE
 #include <dlfcn.h>
@@ -14,7 +15,7 @@ static size_t fail_from = (size_t)-1; /* allocations of at least this many bytes
 static int fail_graphs;
 static struct { void *p; size_t n; } live[4096];
 static size_t peak_call, live_bytes; /* largest request since the last reset, bytes held */
-static int refused;
+static int refused, instantiated;
 
 static void *real(const char *name)
 {
@@ -69,16 +70,19 @@ int hipGraphInstantiate(void **exec, void *graph, void **node, char *log, size_t
         ++refused;
         return OUT_OF_MEMORY;
     }
+    ++instantiated;
     return f(exec, graph, node, log, size);
 }
 
-void hip_faults_set(size_t alloc_from, int graphs)
+void hip_faults_set(size_t alloc_from, int refuse_graphs)
 {
     fail_from = alloc_from;
-    fail_graphs = graphs;
+    fail_graphs = refuse_graphs;
     refused = 0;
+    instantiated = 0;
     peak_call = 0;
 }
+int hip_faults_graphs(void) { return instantiated; } /* since the last set */
 int hip_faults_refused(void) { return refused; }
 size_t hip_faults_peak(void) { return peak_call; }
 size_t hip_faults_live(void) { return live_bytes; }

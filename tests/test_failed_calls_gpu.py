@@ -4,7 +4,8 @@ returns an error and the state is as before it, so the same call succeeds
 afterwards with the values of a run that never failed.  Fields read and written
 without device memory for the packing: the same values.  The scratch memory of
 the packing: bounded, and none held before a field is read.  A learned layer's
-loss and gradient: no device memory asked for.  A shim between
+loss and gradient: no device memory asked for.  Runs that alternate between two
+lengths: no graph instantiated twice.  A shim between
 libphc.so and the HIP runtime (tests/cpp/hip_faults.c) refuses and counts; it
 has to be loaded first, so each test runs in a process of its own."""
 import ctypes
@@ -66,6 +67,23 @@ def check_failed_run(phc, faults, make):
         for x, y in zip(state(a), state(b)):
             assert np.array_equal(x, y), (it, n)
     assert np.abs(state(a)[0]).max() > 0
+
+
+def check_graphs_kept(phc, faults):
+    """Runs of two lengths in turn from one sample instantiate each graph once."""
+    for make in (fd, sem, sem2d, batch):
+        a = make(phc)
+        for k in range(24):
+            if k == 8:
+                faults.hip_faults_set(NEVER, 0)
+            if hasattr(a, "it"):
+                a.it = 0
+            run(a, 0, (10, 7)[k % 2])
+        assert faults.hip_faults_graphs() == 0, make.__name__
+        if hasattr(a, "it"):
+            a.it = 0
+        run(a, 0, 5)
+        assert faults.hip_faults_graphs() == 1, make.__name__
 
 
 def fd_fields(phc, faults, dims, lh, refuse):
@@ -148,6 +166,7 @@ def check_eval_allocates_nothing(phc, faults):
 
 
 CASES = {
+    "graphs_kept": check_graphs_kept,
     "eval_allocates_nothing": check_eval_allocates_nothing,
     "no_scratch": check_no_scratch,
     "scratch_size": check_scratch_size,
